@@ -1,0 +1,49 @@
+/*
+ * Schedule entries of libmpx_attn.so beside mpx_attn.h: variants of its calls
+ * whose caller sizes the workspace for one schedule. Conventions (return
+ * codes, strides, streams) are those of mpx_attn.h.
+ */
+#ifndef MPX_ATTN_SCHED_H
+#define MPX_ATTN_SCHED_H
+
+#include "mpx_attn.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/*
+ * mpx_attn_bwd_dropout (dropout_p = 0: mpx_attn_bwd) on the recomputing
+ * schedule, for grouped K/V heads: with a workspace of at least
+ * mpx_attn_bwd_grouped_workspace_bytes(...) bytes the query heads of a K/V
+ * head are cut into parts that run as separate workgroups and leave float32
+ * sums in the workspace, added up and rounded once by a last kernel; with less
+ * (mpx_attn_bwd_workspace_bytes at least) each group is one part. No
+ * counterpart in the reference, whose flash_attention takes equal head counts
+ * (mlx_primitives/attention/flash.py:151-154).
+ */
+size_t mpx_attn_bwd_grouped_workspace_bytes(int B, int H, int H_kv, int Sq, int Sk, int D,
+                                            int dtype, int window_left);
+
+int mpx_attn_bwd_grouped(const void* q, const void* k, const void* v, const void* o,
+                         const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                         const int64_t* q_strides, const int64_t* k_strides,
+                         const int64_t* v_strides, const int64_t* o_strides,
+                         const int64_t* do_strides, const int64_t* dq_strides,
+                         const int64_t* dk_strides, const int64_t* dv_strides,
+                         int B, int H, int H_kv, int Sq, int Sk, int D, float scale, int causal,
+                         int window_left, int window_right, int dtype, float dropout_p,
+                         uint64_t seed, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * 1 when mpx_attn_bwd_dropout runs faster with the stored-dS workspace
+ * (mpx_attn_bwd_ds_workspace_bytes) than without it, else 0.
+ */
+int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk, int D, int dtype,
+                              int window_left);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* MPX_ATTN_SCHED_H */

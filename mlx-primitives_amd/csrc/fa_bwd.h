@@ -26,6 +26,11 @@ struct BwdParams {
   // words of the keep-mask hash, and the 1 / (1 - p) of the kept weights.
   uint32_t drop_thresh, seed0, seed1;
   float drop_scale;
+  // Key-parallel work of a K/V head cut into kv_parts parts of its query heads
+  // (1: none): each part's dK and dV go to dkv_part as float32 sums, (B, H_kv,
+  // part, Sk, D) dK first, which fa_bwd_dkv_sum_kernel adds up.
+  float* dkv_part;
+  int kv_parts;
   // Stored dS^T (the stored-dS schedule only): ds_tot blocks per query head.
   void* ds;
   int64_t ds_tot;

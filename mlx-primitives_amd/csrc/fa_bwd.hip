@@ -25,6 +25,7 @@
 // packed, they are directly the B operand of the next product over those rows.
 // Transposed operands come from the row-major tiles through ds_read_b64_tr_b16.
 #include "fa_bwd.h"
+#include "mpx_attn_sched.h"
 
 #include <algorithm>
 #include <cmath>
@@ -143,6 +144,50 @@ __device__ __forceinline__ void store_row(uint16_t* row, int g, const f32x16 (&a
                          pack2<BF16>(acc[db][4 * e4 + 2] * mul, acc[db][4 * e4 + 3] * mul)};
       *(u32x2*)(row + d) = val;
     }
+}
+
+// One key's dK (times scale) and dV (times mul_v) as float32 sums of a part of
+// the K/V head's query heads (BwdParams::dkv_part).
+template <int NDB>
+__device__ __forceinline__ void store_part(const BwdParams& p, int bhk, int part, int key, int g,
+                                           const f32x16 (&dk)[NDB], const f32x16 (&dv)[NDB],
+                                           float mul_v) {
+  constexpr int D = 32 * NDB;
+  const int64_t plane = (int64_t)p.B * p.H_kv * p.kv_parts * p.Sk * D;
+  float* row = p.dkv_part + (((int64_t)bhk * p.kv_parts + part) * p.Sk + key) * D + 4 * g;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4) {
+      f32x4 a, c;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a[i] = dk[db][4 * e4 + i] * p.scale;
+        c[i] = dv[db][4 * e4 + i] * mul_v;
+      }
+      *(f32x4*)(row + db * 32 + 8 * e4) = a;
+      *(f32x4*)(row + plane + db * 32 + 8 * e4) = c;
+    }
+}
+
+// dK (blockIdx.y == 0) or dV = the parts' float32 sums added up, rounded once:
+// four dims of one key per thread.
+template <int D, bool BF16>
+__global__ __launch_bounds__(256) void fa_bwd_dkv_sum_kernel(BwdParams p) {
+  const int64_t n = (int64_t)p.B * p.H_kv * p.Sk * (D / 4);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int d = (int)(i % (D / 4)) * 4;
+  const int64_t row = i / (D / 4), bhk = row / p.Sk;
+  const int key = (int)(row - bhk * p.Sk), b = (int)(bhk / p.H_kv), hk = (int)(bhk % p.H_kv);
+  const float* src = p.dkv_part + ((bhk * p.kv_parts + (int64_t)p.B * p.H_kv * p.kv_parts *
+                                    blockIdx.y) * p.Sk + key) * D + d;
+  f32x4 sum = *(const f32x4*)src;
+  for (int k = 1; k < p.kv_parts; ++k) sum += *(const f32x4*)(src + (int64_t)k * p.Sk * D);
+  uint16_t* dst = blockIdx.y == 0
+                      ? (uint16_t*)p.dk + b * p.dk_sb + hk * p.dk_sh + (int64_t)key * p.dk_ss
+                      : (uint16_t*)p.dv + b * p.dv_sb + hk * p.dv_sh + (int64_t)key * p.dv_ss;
+  *(u32x2*)(dst + d) = (u32x2){pack2<BF16>(sum[0], sum[1]), pack2<BF16>(sum[2], sum[3])};
 }
 
 // The same for the wave's 32 rows (row0 + j) at once, through the wave's own
@@ -267,20 +312,14 @@ __device__ __forceinline__ void grid_tile(int n_heads, int n_tiles, int& tile, i
 // fragments it holds and the O row) and writes it for the dK/dV kernel that
 // runs after it.
 // ---------------------------------------------------------------------------
-template <int D, bool BF16, bool DROP = false>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2, D > 128 ? 1 : 2)))
-void fa_bwd_dq_kernel(BwdParams p) {
-  constexpr int NKS = D / 16, NDB = D / 32, TILE = kBwdTile * D;
-  // Stage s: K tile at [2s], V tile at [2s + 1].
-  __shared__ __align__(1024) uint16_t lds[4 * TILE];
+template <int D>
+constexpr int kDqLds = 4 * kBwdTile * D;  // LDS elements: stage s: K tile at [2s], V tile at [2s + 1]
 
-  const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn;
-  // A workgroup runs query tiles n_qt - 1 - pt and pt, the longer (under a
-  // causal mask, the last) first: their key-tile counts add up to the same
-  // total for every pair, so all workgroups carry equal work.
-  int pt, bh, single;
-  grid_pair(p.B * p.H, n_qt, MPX_BWD_TAIL_DQ, pt, bh, single);
+// Query tiles qt_a, then qt_b (none when < 0), of (batch, head) bh.
+template <int D, bool BF16, bool DROP>
+__device__ __forceinline__ void bwd_dq_tiles(const BwdParams& p, uint16_t* lds, int bh, int qt_a,
+                                             int qt_b, bool write_dvec) {
+  constexpr int NKS = D / 16, NDB = D / 32, TILE = kBwdTile * D;
   const int b = bh / p.H, h = bh % p.H;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 31, g = lane >> 5;
@@ -298,9 +337,8 @@ void fa_bwd_dq_kernel(BwdParams p) {
   const u32 lbase = lds_addr(lds);
 
   for (int pass = 0; pass < 2; ++pass) {
-    const int qt = single >= 0 ? n_qt - 1 - single : (pass == 0 ? n_qt - 1 - pt : pt);
-    // odd n_qt: the middle tile runs alone
-    if (pass == 1 && (single >= 0 || qt == n_qt - 1 - pt)) break;
+    const int qt = pass == 0 ? qt_a : qt_b;
+    if (qt < 0) break;
     const int q0 = qt * kBwdOwn, wq0 = q0 + wave * 32, myq = wq0 + j;
     const int qrow = min(myq, p.Sq - 1);
     u32x4 qf[NKS], df[NKS];
@@ -326,7 +364,7 @@ void fa_bwd_dq_kernel(BwdParams p) {
           part += h2f<BF16>((uint16_t)(of[ks][w] >> 16)) * h2f<BF16>((uint16_t)(df[ks][w] >> 16));
         }
       dvc = pair_sum32(part);
-      if (g == 0 && myq < p.Sq) p.dvec[rix] = dvc;
+      if (write_dvec && g == 0 && myq < p.Sq) p.dvec[rix] = dvc;
     }
     // Keys this row sees: [kv_first, kv_last] (rows past Sq have lse = +inf, so
     // their probabilities vanish without a mask).
@@ -439,6 +477,22 @@ void fa_bwd_dq_kernel(BwdParams p) {
   }
 }
 
+// Query tiles of a paired launch: n_qt - 1 - pt and pt, the longer (under a
+// causal mask, the last) first: their key-tile counts add up to the same total
+// for every pair, so all workgroups carry equal work.
+template <int D, bool BF16, bool DROP = false>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2, D > 128 ? 1 : 2)))
+void fa_bwd_dq_kernel(BwdParams p) {
+  __shared__ __align__(1024) uint16_t lds[kDqLds<D>];
+  const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn;
+  int pt, bh, single;
+  grid_pair(p.B * p.H, n_qt, MPX_BWD_TAIL_DQ, pt, bh, single);
+  // odd n_qt: the middle tile runs alone
+  const int qt_a = n_qt - 1 - (single >= 0 ? single : pt);
+  bwd_dq_tiles<D, BF16, DROP>(p, lds, bh, qt_a, single >= 0 || qt_a == pt ? -1 : pt, true);
+}
+
 // ---------------------------------------------------------------------------
 // dK, dV: a workgroup owns keys [128 * kt, +128) of one (batch, K/V head);
 // wave w keys +32w. Per Q tile (of every query head in the K/V head's group):
@@ -452,23 +506,25 @@ void fa_bwd_dq_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------
 constexpr int kBoth = 0, kOnlyK = 1, kOnlyV = 2;
 
-template <int D, bool BF16, int MODE, bool DROP = false>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2, D > 128 ? 1 : 2)))
-void fa_bwd_dkdv_kernel(BwdParams p) {
+template <int D>
+constexpr int kDkdvRows = D > 128 ? 32 : kBwdTile;  // streamed Q / dO rows per step
+// LDS elements: two stages of (Q tile, dO tile), then lse and Dvec rows of each.
+template <int D>
+constexpr int kDkdvLds = 4 * kDkdvRows<D> * D + 8 * kDkdvRows<D>;
+
+// Key tile kt of (batch, K/V head) bhk, for part `part` of the head's query heads.
+template <int D, bool BF16, int MODE, bool DROP, bool SPLIT>
+__device__ __forceinline__ void bwd_dkdv_tile(const BwdParams& p, uint16_t* lds, int bhk, int part,
+                                              int kt) {
   constexpr bool WANT_K = MODE != kOnlyV, WANT_V = MODE != kOnlyK;
   // Streamed Q / dO rows per step: 64, or 32 at D = 256 (four 64-row tiles of
   // 512-byte rows would fill 128 KB of LDS). NBLK 32-row blocks per step.
-  constexpr int ROWS = D > 128 ? 32 : kBwdTile, NBLK = ROWS / 32;
+  constexpr int ROWS = kDkdvRows<D>, NBLK = ROWS / 32;
   constexpr int NKS = D / 16, NDB = D / 32, TILE = ROWS * D;
   // Stage s: Q tile at [2s], dO tile at [2s + 1].
-  __shared__ __align__(1024) uint16_t lds[4 * TILE];
-  __shared__ __align__(16) float lse_lds[2][ROWS];
-  __shared__ __align__(16) float dvc_lds[2][ROWS];
+  float(*lse_lds)[ROWS] = (float(*)[ROWS])(lds + 4 * TILE);
+  float(*dvc_lds)[ROWS] = lse_lds + 2;
 
-  const int n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn;
-  int kt, bhk;  // key tile (first, under a causal mask the longest, first), (batch, K/V head)
-  grid_tile(p.B * p.H_kv, n_kt, kt, bhk);
   const int b = bhk / p.H_kv, hk = bhk % p.H_kv;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 31, g = lane >> 5;
@@ -497,7 +553,9 @@ void fa_bwd_dkdv_kernel(BwdParams p) {
   const int q_hi = p.win_left >= 0 ? min(p.Sq, k_last + p.win_left + 1) : p.Sq;
   const int t0 = q_lo / ROWS;
   const int n_t = q_hi > q_lo ? (q_hi - 1) / ROWS - t0 + 1 : 0;
-  const int n_steps = n_t * p.kv_group;
+  const int heads = SPLIT ? p.kv_group / p.kv_parts : p.kv_group;
+  const int h0 = hk * p.kv_group + (SPLIT ? part * heads : 0);
+  const int n_steps = n_t * heads;
 
   Addr<D> ad;
   ad.init(lane);
@@ -515,7 +573,7 @@ void fa_bwd_dkdv_kernel(BwdParams p) {
   float lse_r = 0.f, dvc_r = 0.f;  // row threadIdx.x of the tile in flight (first 64 threads)
   // Step u's Q and dO tiles into stage S by DMA, its lse and Dvec rows into registers.
   auto load = [&](int u, int S) __attribute__((always_inline)) {
-    const int h = hk * p.kv_group + u / n_t;
+    const int h = h0 + u / n_t;
     const int row0 = (t0 + u % n_t) * ROWS;
     qd.load((const uint16_t*)p.q + b * p.q_sb + h * p.q_sh, lbase + (2 * S) * TILE * 2, row0,
             p.Sq);
@@ -549,9 +607,7 @@ void fa_bwd_dkdv_kernel(BwdParams p) {
     const int qr0 = (t0 + u % n_t) * ROWS;
     // (dropout: row key of query qr0 + 8 g of this step's head)
     const u32 drop_rk =
-        DROP ? drop_row_key((u32)(((int64_t)b * p.H + hk * p.kv_group + u / n_t) * p.Sq + qr0 +
-                                  8 * g),
-                            p.seed0)
+        DROP ? drop_row_key((u32)(((int64_t)b * p.H + h0 + u / n_t) * p.Sq + qr0 + 8 * g), p.seed0)
              : 0u;
     const bool skip = wk0 >= p.Sk ||
                       (p.win_right >= 0 && wk0 > qr0 + ROWS - 1 + p.win_right) ||
@@ -641,7 +697,9 @@ void fa_bwd_dkdv_kernel(BwdParams p) {
     if (u + 1 < n_steps) store_vec(S ^ 1);
     stage_barrier();
   }
-  if (mykey < p.Sk) {
+  if (SPLIT && mykey < p.Sk) {
+    store_part<NDB>(p, bhk, part, mykey, g, dk, dv, DROP ? p.drop_scale : 1.f);
+  } else if (mykey < p.Sk) {
     if constexpr (WANT_K)
       store_row<NDB, BF16>(
           (uint16_t*)p.dk + b * p.dk_sb + hk * p.dk_sh + (int64_t)mykey * p.dk_ss, g, dk,
@@ -651,6 +709,18 @@ void fa_bwd_dkdv_kernel(BwdParams p) {
           (uint16_t*)p.dv + b * p.dv_sb + hk * p.dv_sh + (int64_t)mykey * p.dv_ss, g, dv,
           DROP ? p.drop_scale : 1.f);
   }
+}
+
+template <int D, bool BF16, int MODE, bool DROP = false, bool SPLIT = false>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2, D > 128 ? 1 : 2)))
+void fa_bwd_dkdv_kernel(BwdParams p) {
+  __shared__ __align__(1024) uint16_t lds[kDkdvLds<D>];
+  int kt, bhk;  // key tile (first, under a causal mask the longest, first), (batch, K/V head)
+  const int heads = p.B * p.H_kv;
+  grid_tile(SPLIT ? heads * p.kv_parts : heads, (p.Sk + kBwdOwn - 1) / kBwdOwn, kt, bhk);
+  const int part = SPLIT ? bhk / heads : 0;
+  bwd_dkdv_tile<D, BF16, MODE, DROP, SPLIT>(p, lds, bhk - part * heads, part, kt);
 }
 
 // ---------------------------------------------------------------------------
@@ -670,26 +740,23 @@ void fa_bwd_dkdv_kernel(BwdParams p) {
 // reads of the block are conflict-free.
 constexpr int kFusedTile = 32;
 
-template <bool BF16, bool DROP = false, bool DS = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void fa_bwd_dkdv_fused_kernel(BwdParams p) {
+// LDS elements: the K tile, two stages of (Q tile, dO tile), the lse / Dvec rows.
+constexpr int kFusedLds = kBwdOwn * 128 + 4 * kFusedTile * 128 + 2 * 2 * 64 * 2;
+static_assert(kFusedLds * 2 <= 80 * 1024, "two workgroups per CU");
+
+// Key tiles kt_a, then kt_b (none when < 0), of (batch, K/V head) bhk, for part
+// `part` of the head's query heads.
+template <bool BF16, bool DROP, bool DS, bool SPLIT>
+__device__ __forceinline__ void bwd_dkdv_fused_tiles(const BwdParams& p, uint16_t* smem, int bhk,
+                                                     int part, int kt_a, int kt_b) {
   constexpr int D = 128, NKS = D / 16, NDB = D / 32, TILE = kFusedTile * D;
-  __shared__ __align__(1024) uint16_t ktile[kBwdOwn * D];
+  uint16_t* const ktile = smem;
   // Stage s: Q tile at [2s], dO tile at [2s + 1].
-  __shared__ __align__(1024) uint16_t lds[4 * TILE];
+  uint16_t* const lds = smem + kBwdOwn * D;
   // Stage s: lse of the tile's rows at [s][0], Dvec at [s][1], one 64-lane DMA
   // each (the second half holds the 32 rows after the tile, unused).
-  __shared__ __align__(16) float vec_lds[2][2][64];
-  static_assert(sizeof(ktile) + sizeof(lds) + sizeof(vec_lds) <= 80 * 1024,
-                "two workgroups per CU");
+  float(*vec_lds)[2][64] = (float(*)[2][64])(lds + 4 * TILE);
 
-  const int n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn;
-  // A workgroup runs key tiles pt and n_kt - 1 - pt, the longer (under a
-  // causal mask, the first) first: their step counts add up to the same total
-  // for every pair, so all workgroups carry equal work and the launch ends
-  // without a tail of long tiles that started late.
-  int pt, bhk, single;  // tile pair, (batch, K/V head), single tile rank
-  grid_pair(p.B * p.H_kv, n_kt, DS || MPX_BWD_TAIL_DKDV, pt, bhk, single);
   // (scalar: the lse / Dvec DMA descriptors are built from them)
   const int b = __builtin_amdgcn_readfirstlane(bhk / p.H_kv);
   const int hk = __builtin_amdgcn_readfirstlane(bhk % p.H_kv);
@@ -727,9 +794,8 @@ void fa_bwd_dkdv_fused_kernel(BwdParams p) {
   const u32 lbase = lds_addr(lds);
 
   for (int pass = 0; pass < 2; ++pass) {
-    const int kt = single >= 0 ? single : (pass == 0 ? pt : n_kt - 1 - pt);
-    // odd n_kt: the middle tile runs alone
-    if (pass == 1 && (single >= 0 || kt == pt)) break;
+    const int kt = pass == 0 ? kt_a : kt_b;
+    if (kt < 0) break;
     const int k0 = kt * kBwdOwn, wk0 = k0 + wave * 32, mykey = wk0 + j;
     const int krow = min(mykey, p.Sk - 1);
     // Visible query rows of this key, cut at Sq (rows past it are clamped
@@ -754,7 +820,9 @@ void fa_bwd_dkdv_fused_kernel(BwdParams p) {
     const int q_hi = p.win_left >= 0 ? min(p.Sq, k_last + p.win_left + 1) : p.Sq;
     const int t0 = q_lo / kFusedTile;
     const int n_t = q_hi > q_lo ? (q_hi - 1) / kFusedTile - t0 + 1 : 0;
-    const int n_steps = n_t * p.kv_group;
+    const int heads = SPLIT ? p.kv_group / p.kv_parts : p.kv_group;
+    const int h0 = hk * p.kv_group + (SPLIT ? part * heads : 0);
+    const int n_steps = n_t * heads;
 
     f32x16 dk[NDB], dv[NDB];
 #pragma unroll
@@ -778,11 +846,11 @@ void fa_bwd_dkdv_fused_kernel(BwdParams p) {
                (((int64_t)(b * p.H + hk * p.kv_group) * p.ds_tot + off + wave) * kDsBlockBytes);
     }
 
-    // Step u covers query tile t0 + u % n_t of head hk * kv_group + u / n_t; the
+    // Step u covers query tile t0 + u % n_t of head h0 + u / n_t; the
     // pair is stepped, not divided, for the tile being loaded (lt, lh) and the
     // tile being computed (ct). Waves 0 and 1 also bring the tile's lse and
     // Dvec rows (clamped at Sq) into LDS.
-    int lt = 0, lh = hk * p.kv_group, ct = 0, ch = hk * p.kv_group;
+    int lt = 0, lh = h0, ct = 0, ch = h0;
     auto load = [&](int S) __attribute__((always_inline)) {
       const int row0 = (t0 + lt) * kFusedTile;
       if (wave < 2) {
@@ -914,13 +982,33 @@ void fa_bwd_dkdv_fused_kernel(BwdParams p) {
               dsp[hh], (u32x4*)(ds_blk + hh * 1024 + (32 * g + (j ^ (4 * (2 * hh + g)))) * 16));
       }
     }
-    if (mykey < p.Sk) {
+    if (SPLIT && mykey < p.Sk) {
+      store_part<NDB>(p, bhk, part, mykey, g, dk, dv, DROP ? p.drop_scale : 1.f);
+    } else if (mykey < p.Sk) {
       store_row<NDB, BF16>((uint16_t*)p.dk + b * p.dk_sb + hk * p.dk_sh + (int64_t)mykey * p.dk_ss,
                            g, dk, p.scale);
       store_row<NDB, BF16>((uint16_t*)p.dv + b * p.dv_sb + hk * p.dv_sh + (int64_t)mykey * p.dv_ss,
                            g, dv, DROP ? p.drop_scale : 1.f);
     }
   }
+}
+
+// Key tiles of a paired launch: pt and n_kt - 1 - pt, the longer (under a
+// causal mask, the first) first: their step counts add up to the same total
+// for every pair, so all workgroups carry equal work and the launch ends
+// without a tail of long tiles that started late.
+template <bool BF16, bool DROP = false, bool DS = false, bool SPLIT = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void fa_bwd_dkdv_fused_kernel(BwdParams p) {
+  __shared__ __align__(1024) uint16_t smem[kFusedLds];
+  const int n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn, heads = p.B * p.H_kv;
+  int pt, bhk, single;  // tile pair, (batch, K/V head), single tile rank
+  grid_pair(SPLIT ? heads * p.kv_parts : heads, n_kt, DS || MPX_BWD_TAIL_DKDV, pt, bhk, single);
+  const int part = SPLIT ? bhk / heads : 0;
+  // odd n_kt: the middle tile runs alone
+  const int kt_a = single >= 0 ? single : pt, kt_b = n_kt - 1 - pt;
+  bwd_dkdv_fused_tiles<BF16, DROP, DS, SPLIT>(p, smem, bhk - part * heads, part, kt_a,
+                                              single >= 0 || kt_b == kt_a ? -1 : kt_b);
 }
 
 // ---------------------------------------------------------------------------
@@ -1137,12 +1225,160 @@ void fa_bwd_dq_ds_kernel(BwdParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// dQ and dK/dV of one backward in one launch, one tile per workgroup, the
+// longest tiles first (Dvec comes from fa_bwd_dvec_kernel before it). For
+// problems whose dQ or dK/dV launch alone leaves slots of the chip empty (two
+// workgroups per CU: 512): a wave that has its SIMD to itself takes nearly as
+// long per step as two that share it (2.4 against 2.8 us per 64-key dQ step),
+// so filling the second slot is close to free, and tiles handed out longest
+// first need no pairing. Backward of a causal bf16 (batch, S, heads, D), two
+// launches against one: (2, 2048, 16, 128) 167 -> 147 us, (1, 1024, 16, 128)
+// 98 -> 64, (4, 1000, 12, 64) 67 -> 44, (1, 300, 8, 128) 46 -> 26.
+// ---------------------------------------------------------------------------
+// The heads go in chunks of chunk_heads (batch, K/V head)s, chunk_wgs
+// workgroups each. Within a chunk, entry i of the order covers the workgroups
+// first[i] .. first[i + 1] - 1: dK/dV of key tile code >> 1 (code & 1; one per
+// K/V head and part) or dQ of query tile code >> 1 (one per query head).
+constexpr int kMaxOrder = 128;
+struct BwdOrder {
+  int n, chunk_heads, chunk_wgs;
+  int first[kMaxOrder + 1];
+  uint16_t code[kMaxOrder];
+};
+
+template <int D, bool BF16, bool DROP, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void fa_bwd_joint_kernel(BwdParams p, BwdOrder order) {
+  constexpr int kLds = D == 128 ? kFusedLds : kDkdvLds<D>;
+  static_assert(kLds >= kDqLds<D>, "dQ stages");
+  __shared__ __align__(1024) uint16_t lds[kLds];
+  const int chunk = blockIdx.x / order.chunk_wgs, wg = blockIdx.x - chunk * order.chunk_wgs;
+  int lo = 0, hi = order.n;  // first[lo] <= wg < first[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (order.first[mid] <= wg)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  const int code = order.code[lo], tile = code >> 1;
+  // K/V heads fastest: with a multiple of 8 heads in a chunk every entry starts
+  // on XCD 0, and a K/V head and its query heads stay on XCD head % 8 through
+  // all their tiles.
+  const int i = wg - order.first[lo];
+  const int sub = i / order.chunk_heads;  // part, or query head of the group
+  const int bhk = chunk * order.chunk_heads + (i - sub * order.chunk_heads);
+  if (code & 1) {
+    if constexpr (D == 128)
+      bwd_dkdv_fused_tiles<BF16, DROP, false, SPLIT>(p, lds, bhk, sub, tile, -1);
+    else
+      bwd_dkdv_tile<D, BF16, kBoth, DROP, SPLIT>(p, lds, bhk, sub, tile);
+  } else {
+    bwd_dq_tiles<D, BF16, DROP>(p, lds, bhk * p.kv_group + sub, tile, -1, false);
+  }
+}
+
+// Rows (or keys) the masks of tile `t` of n_own reach among n_other: keys per
+// query tile (left = win_left, right = win_right) or, with the two swapped,
+// queries per key tile.
+int tile_reach(int t, int n_own, int n_other, int left, int right) {
+  const int o0 = t * kBwdOwn, o1 = std::min(o0 + kBwdOwn, n_own) - 1;
+  const int lo = left >= 0 ? std::max(0, o0 - left) : 0;
+  const int hi = right >= 0 ? std::min(n_other, o1 + right + 1) : n_other;
+  return std::max(0, hi - lo);
+}
+
+// Workgroups per XCD that a chunk of heads has at least: fewer heads at a time
+// keep their streamed tiles in the XCD's L2, more give the longest-first order
+// more to choose from. Causal bf16 backward with 32 / 64 / 128 / no chunks:
+// (2, 2048, 16, 128) 187 / 160 / 148 / 151 us, (4, 2048, 32, 64) 318 / 306 /
+// 298 / 319 us.
+constexpr int kChunkWgs = 128;
+
+// The order of a joint launch: tiles by cost, products per row of the streamed
+// side (dK/dV: 4 for every query head of the part, dQ: 3), largest first.
+// (bwd_joint: the tiles of a head fit an order.)
+void make_order(const BwdParams& p, BwdOrder& order) {
+  const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn, n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn;
+  struct Item {
+    int64_t cost;
+    int code;
+  } items[kMaxOrder];
+  int n = 0;
+  for (int t = 0; t < n_kt; ++t)
+    items[n++] = {4LL * (p.kv_group / p.kv_parts) *
+                      tile_reach(t, p.Sk, p.Sq, p.win_right, p.win_left),
+                  2 * t + 1};
+  for (int t = 0; t < n_qt; ++t)
+    items[n++] = {3LL * tile_reach(t, p.Sq, p.Sk, p.win_left, p.win_right), 2 * t};
+  std::stable_sort(items, items + n,
+                   [](const Item& a, const Item& b) { return a.cost > b.cost; });
+  const int heads = p.B * p.H_kv, per_head = n_kt * p.kv_parts + n_qt * p.kv_group;
+  order.chunk_heads = heads;
+  if (heads % 8 == 0)
+    for (int m = 1; m < heads / 8; ++m)
+      if (heads / 8 % m == 0 && m * per_head >= kChunkWgs) {
+        order.chunk_heads = 8 * m;
+        break;
+      }
+  order.n = n;
+  int at = 0;
+  for (int i = 0; i < n; ++i) {
+    order.first[i] = at;
+    order.code[i] = (uint16_t)items[i].code;
+    at += order.chunk_heads * ((items[i].code & 1) ? p.kv_parts : p.kv_group);
+  }
+  order.first[n] = order.chunk_wgs = at;
+}
+
 constexpr int kDqDsQB = 2;  // query blocks per wave of fa_bwd_dq_ds_kernel
 
-template <int D, bool BF16, bool DROP>
+// One joint launch (fa_bwd_joint_kernel) instead of a dQ and a dK/dV launch:
+// while the pairs of one side do not fill the 512 slots, that is below 2048
+// tiles of 128 rows over both sides. Past that the paired launches win at
+// D = 128, whose workgroups stream one head at a time: causal bf16
+// (4, 2048, 16, 128), 2048 tiles, 257 us paired, 278 joint; (2, 3000, 16, 128),
+// 1536 tiles, 300 paired, 289 joint. At D = 64 (dK/dV unpaired) and under a
+// window (nothing to pair) the line is at twice that: (2, 4096, 16, 64), 2048
+// tiles, 298 two launches, 272 joint, level at 8192 tiles; (2, 3000, 24, 128)
+// window 512, 2304 tiles, 247 and 198; (8, 2048, 32, 128) window 256, 8192
+// tiles, 495 and 516.
+bool bwd_joint(int B, int H, int Sq, int Sk, int D, int win_left) {
+  const int n_qt = (Sq + kBwdOwn - 1) / kBwdOwn, n_kt = (Sk + kBwdOwn - 1) / kBwdOwn;
+  const long limit = D == 64 || win_left >= 0 ? 4096 : 2047;
+  return D <= 128 && n_qt < kMaxOrder && n_kt < kMaxOrder && n_qt + n_kt <= kMaxOrder &&
+         (long)B * H * (n_qt + n_kt) <= limit;
+}
+
+// Parts that a K/V head's query heads are cut into (1: none) for the grouped
+// 16-bit backward at D <= 128: the fewest (a divisor of the group) that give
+// the dK/dV side a workgroup for each of the chip's 512 slots. Causal bf16
+// (1, 2048, 32 heads over 8, 128): 409 -> 158 us with 4 parts in the joint
+// launch; (8, 1024, 32 over 4, 128): 488 -> 325 us with 4 parts of paired
+// tiles. The parts' sums are at most 512 + 511 tiles of 128 keys (256 MB).
+int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, int dtype) {
+  const int group = H / H_kv;
+  if (group == 1 || dtype == MPX_F32 || D > 128) return 1;
+  const int n_kt = (Sk + kBwdOwn - 1) / kBwdOwn;
+  const bool pairs = D == 128 && !bwd_joint(B, H, Sq, Sk, D, win_left);
+  const long wgs = (long)B * H_kv * (pairs ? (n_kt + 1) / 2 : n_kt);
+  for (int parts = 1; parts < group; ++parts)
+    if (group % parts == 0 && wgs * parts >= 512) return parts;
+  return group;
+}
+
+template <int D, bool BF16>
+void launch_kv_sum(const BwdParams& p, hipStream_t st) {
+  const long n = (long)p.B * p.H_kv * p.Sk * (D / 4);
+  hipLaunchKernelGGL((fa_bwd_dkv_sum_kernel<D, BF16>), dim3((unsigned)((n + 255) / 256), 2),
+                     dim3(256), 0, st, p);
+}
+
+template <int D, bool BF16, bool DROP, bool SPLIT = false>
 hipError_t launch_bwd(const BwdParams& p, hipStream_t st) {
   const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn, n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn;
-  if constexpr (D == 128) {
+  if constexpr (D == 128 && !SPLIT) {
     if (p.ds != nullptr) {
       // Stored dS: Dvec, then dK / dV (which stores dS), then dQ = scale dS K.
       const long rows = (long)p.B * p.H * p.Sq;
@@ -1156,21 +1392,40 @@ hipError_t launch_bwd(const BwdParams& p, hipStream_t st) {
       return hipGetLastError();
     }
   }
+  if constexpr (D <= 128) {
+    BwdOrder order;
+    if (bwd_joint(p.B, p.H, p.Sq, p.Sk, D, p.win_left)) {
+      make_order(p, order);
+      const long rows = (long)p.B * p.H * p.Sq, rpb = 256 / (D / 8);
+      const long tiles = (long)p.B * p.H * n_qt + (long)p.B * p.H_kv * p.kv_parts * n_kt;
+      hipLaunchKernelGGL((fa_bwd_dvec_kernel<D, BF16>), dim3((rows + rpb - 1) / rpb), dim3(256), 0,
+                         st, p);
+      hipLaunchKernelGGL((fa_bwd_joint_kernel<D, BF16, DROP, SPLIT>), dim3((unsigned)tiles), dim3(256), 0,
+                         st, p, order);
+      if constexpr (SPLIT) launch_kv_sum<D, BF16>(p, st);
+      return hipGetLastError();
+    }
+  }
   // dQ (which also writes Dvec) before dK / dV, which reads it.
   hipLaunchKernelGGL((fa_bwd_dq_kernel<D, BF16, DROP>),
                      dim3(bwd_pair_grid(p.B * p.H, n_qt, MPX_BWD_TAIL_DQ)), dim3(256), 0, st, p);
-  const dim3 grid_kv(p.B * p.H_kv * n_kt);
+  const int kv_heads = p.B * p.H_kv * p.kv_parts;
   if constexpr (D == 128) {
-    const dim3 grid_pairs(bwd_pair_grid(p.B * p.H_kv, n_kt, MPX_BWD_TAIL_DKDV));
-    hipLaunchKernelGGL((fa_bwd_dkdv_fused_kernel<BF16, DROP>), grid_pairs, dim3(256), 0, st, p);
+    const dim3 grid_pairs(bwd_pair_grid(kv_heads, n_kt, MPX_BWD_TAIL_DKDV));
+    hipLaunchKernelGGL((fa_bwd_dkdv_fused_kernel<BF16, DROP, false, SPLIT>), grid_pairs, dim3(256), 0, st, p);
   } else {  // D = 64, and D = 256 (one wave per SIMD)
-    hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, BF16, kBoth, DROP>), grid_kv, dim3(256), 0, st, p);
+    hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, BF16, kBoth, DROP, SPLIT>), dim3(kv_heads * n_kt),
+                       dim3(256), 0, st, p);
   }
+  if constexpr (SPLIT) launch_kv_sum<D, BF16>(p, st);
   return hipGetLastError();
 }
 
 template <bool BF16, bool DROP>
 hipError_t launch_bwd_d(const BwdParams& p, int D, hipStream_t st) {
+  if (p.kv_parts > 1)
+    return D == 64 ? launch_bwd<64, BF16, DROP, true>(p, st)
+                   : launch_bwd<128, BF16, DROP, true>(p, st);
   if (D == 64) return launch_bwd<64, BF16, DROP>(p, st);
   if (D == 256) return launch_bwd<256, BF16, DROP>(p, st);
   return launch_bwd<128, BF16, DROP>(p, st);
@@ -1215,6 +1470,21 @@ extern "C" size_t mpx_attn_bwd_ds_workspace_bytes(int B, int H, int Sq, int Sk, 
   return dvec_region_bytes(B, H, Sq) + (size_t)std::max<int64_t>(blocks, 2) * kDsBlockBytes;
 }
 
+extern "C" size_t mpx_attn_bwd_grouped_workspace_bytes(int B, int H, int H_kv, int Sq, int Sk,
+                                                       int D, int dtype, int window_left) {
+  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || Sq <= 0 || Sk <= 0 || D <= 0) return 0;
+  const int parts = bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype);
+  if (parts == 1) return mpx_attn_bwd_workspace_bytes(B, H, Sq);
+  return dvec_region_bytes(B, H, Sq) + (size_t)2 * B * H_kv * parts * Sk * D * sizeof(float);
+}
+
+extern "C" int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk, int D, int dtype,
+                                         int window_left) {
+  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || Sq <= 0 || Sk <= 0) return 0;
+  return D == 128 && dtype != MPX_F32 && !bwd_joint(B, H, Sq, Sk, D, window_left) &&
+         bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype) == 1;
+}
+
 static int attn_bwd_entry(const void* q, const void* k, const void* v, const void* o,
                           const void* dout, const float* lse, void* dq, void* dk, void* dv,
                           const int64_t* q_strides, const int64_t* k_strides,
@@ -1223,7 +1493,8 @@ static int attn_bwd_entry(const void* q, const void* k, const void* v, const voi
                           const int64_t* dk_strides, const int64_t* dv_strides, int B, int H,
                           int H_kv, int Sq, int Sk, int D, float scale, int causal,
                           int window_left, int window_right, int dtype, float dropout_p,
-                          uint64_t seed, void* workspace, size_t workspace_bytes, void* stream) {
+                          uint64_t seed, bool grouped, void* workspace, size_t workspace_bytes,
+                          void* stream) {
   MPX_CHECK_ARG(dropout_p >= 0.f && dropout_p < 1.f,
                 "mpx_attn_bwd_dropout: dropout_p must be in [0, 1), got %g", (double)dropout_p);
   MPX_CHECK_ARG(dtype == MPX_F32 || dtype == MPX_F16 || dtype == MPX_BF16,
@@ -1280,7 +1551,7 @@ static int attn_bwd_entry(const void* q, const void* k, const void* v, const voi
   p.dq_sb = dq_strides[0]; p.dq_sh = dq_strides[1]; p.dq_ss = dq_strides[2];
   p.dk_sb = dk_strides[0]; p.dk_sh = dk_strides[1]; p.dk_ss = dk_strides[2];
   p.dv_sb = dv_strides[0]; p.dv_sh = dv_strides[1]; p.dv_ss = dv_strides[2];
-  p.B = B; p.H = H; p.H_kv = H_kv; p.kv_group = H / H_kv; p.Sq = Sq; p.Sk = Sk;
+  p.B = B; p.H = H; p.H_kv = H_kv; p.kv_group = H / H_kv; p.kv_parts = 1; p.Sq = Sq; p.Sk = Sk;
   p.win_left = window_left < 0 ? -1 : window_left;
   p.win_right = causal ? 0 : (window_right < 0 ? -1 : window_right);
   p.scale = scale;
@@ -1295,7 +1566,13 @@ static int attn_bwd_entry(const void* q, const void* k, const void* v, const voi
   // The stored-dS schedule when the workspace holds it.
   const size_t ds_need = mpx_attn_bwd_ds_workspace_bytes(B, H, Sq, Sk, D, dtype, causal,
                                                          window_left, window_right);
-  if (ds_need > 0 && workspace_bytes >= ds_need) {
+  if (grouped) {
+    if (workspace_bytes >= mpx_attn_bwd_grouped_workspace_bytes(B, H, H_kv, Sq, Sk, D, dtype,
+                                                                window_left)) {
+      p.kv_parts = bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype);
+      p.dkv_part = (float*)((char*)workspace + dvec_region_bytes(B, H, Sq));
+    }
+  } else if (ds_need > 0 && workspace_bytes >= ds_need) {
     p.ds = (char*)workspace + dvec_region_bytes(B, H, Sq);
     p.ds_tot = ds_blocks_per_head(Sq, Sk, p.win_left, p.win_right);
   }
@@ -1323,8 +1600,8 @@ extern "C" int mpx_attn_bwd(const void* q, const void* k, const void* v, const v
   clear_error();
   return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
                         o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
-                        Sk, D, scale, causal, window_left, window_right, dtype, 0.f, 0, workspace,
-                        workspace_bytes, stream);
+                        Sk, D, scale, causal, window_left, window_right, dtype, 0.f, 0, false,
+                        workspace, workspace_bytes, stream);
 }
 
 extern "C" int mpx_attn_bwd_dropout(const void* q, const void* k, const void* v, const void* o,
@@ -1341,5 +1618,22 @@ extern "C" int mpx_attn_bwd_dropout(const void* q, const void* k, const void* v,
   return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
                         o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
                         Sk, D, scale, causal, window_left, window_right, dtype, dropout_p, seed,
-                        workspace, workspace_bytes, stream);
+                        false, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mpx_attn_bwd_grouped(const void* q, const void* k, const void* v, const void* o,
+                                    const void* dout, const float* lse, void* dq, void* dk,
+                                    void* dv, const int64_t* q_strides,
+                                    const int64_t* k_strides, const int64_t* v_strides,
+                                    const int64_t* o_strides, const int64_t* do_strides,
+                                    const int64_t* dq_strides, const int64_t* dk_strides,
+                                    const int64_t* dv_strides, int B, int H, int H_kv, int Sq,
+                                    int Sk, int D, float scale, int causal, int window_left,
+                                    int window_right, int dtype, float dropout_p, uint64_t seed,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
+                        o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
+                        Sk, D, scale, causal, window_left, window_right, dtype, dropout_p, seed,
+                        true, workspace, workspace_bytes, stream);
 }

@@ -101,6 +101,12 @@ def load() -> ctypes.CDLL:
         lib.mpx_attn_bwd_dropout.argtypes = [ctypes.c_void_p] * 9 + [_i64p] * 8 + [
             ctypes.c_int] * 6 + [ctypes.c_float] + [ctypes.c_int] * 4 + [
             ctypes.c_float, ctypes.c_uint64, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        lib.mpx_attn_bwd_grouped.restype = ctypes.c_int
+        lib.mpx_attn_bwd_grouped.argtypes = lib.mpx_attn_bwd_dropout.argtypes
+        lib.mpx_attn_bwd_ds_preferred.restype = ctypes.c_int
+        lib.mpx_attn_bwd_ds_preferred.argtypes = [ctypes.c_int] * 8
+        lib.mpx_attn_bwd_grouped_workspace_bytes.restype = ctypes.c_size_t
+        lib.mpx_attn_bwd_grouped_workspace_bytes.argtypes = [ctypes.c_int] * 8
         lib.mpx_attn_bwd_workspace_bytes.restype = ctypes.c_size_t
         lib.mpx_attn_bwd_workspace_bytes.argtypes = [ctypes.c_int] * 3
         lib.mpx_attn_bwd_ds_workspace_bytes.restype = ctypes.c_size_t
@@ -325,9 +331,10 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     stored_ds: the stored-dS schedule (mpx_attn_bwd_ds_workspace_bytes) or the
     recomputing one. None takes the stored one for the dropout backward (whose
     dQ kernel would otherwise regenerate the keep mask as well: 6% faster over
-    forward and backward at the headline shape), where the problem has it and
-    its workspace is at most an eighth of the device's memory and can be
-    allocated; without dropout the two schedules run level and the recomputing
+    forward and backward at the headline shape), where the library prefers it
+    (mpx_attn_bwd_ds_preferred: launches that fill the chip) and its workspace
+    is at most an eighth of the device's memory and can be allocated; without
+    dropout the two schedules run level and the recomputing
     one needs no workspace. False keeps the recomputing schedule; True requires
     the stored one."""
     lib = load()
@@ -335,7 +342,9 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     code = dtype_code(q.dtype)
     ws_bytes = int(lib.mpx_attn_bwd_workspace_bytes(B, H, Sq))
     ws = None
-    if stored_ds or (stored_ds is None and dropout is not None):
+    if stored_ds or (stored_ds is None and dropout is not None
+                     and lib.mpx_attn_bwd_ds_preferred(B, H, H_kv, Sq, Sk, D, code,
+                                                       int(window_left))):
         ds_bytes = int(lib.mpx_attn_bwd_ds_workspace_bytes(
             B, H, Sq, Sk, D, code, int(causal), int(window_left), int(window_right)))
         if stored_ds and not ds_bytes:
@@ -347,6 +356,18 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
             except torch.OutOfMemoryError:
                 if stored_ds:
                     raise
+    grouped = False
+    if ws is None and H_kv != H:
+        # room for the parts that a K/V head's query heads are cut into (at
+        # most about a quarter of a GiB: the parts stop at one workgroup per
+        # slot of the chip); without it each head's group is one part
+        part_bytes = int(lib.mpx_attn_bwd_grouped_workspace_bytes(
+            B, H, H_kv, Sq, Sk, D, code, int(window_left)))
+        try:
+            ws = torch.empty(max(part_bytes, 16), dtype=torch.uint8, device=dev)
+            ws_bytes, grouped = part_bytes, True
+        except torch.OutOfMemoryError:
+            pass
     if ws is None:
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(),
@@ -355,7 +376,10 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
             B, H, H_kv, Sq, Sk, D, float(scale), int(causal), int(window_left),
             int(window_right), code)
     tail = (ws.data_ptr(), ws_bytes, _stream_ptr(dev))
-    if dropout is not None:
+    if grouped:
+        p, seed = dropout if dropout is not None else (0.0, 0)
+        rc = lib.mpx_attn_bwd_grouped(*args, float(p), int(seed) & (2**64 - 1), *tail)
+    elif dropout is not None:
         p, seed = dropout
         rc = lib.mpx_attn_bwd_dropout(*args, float(p), int(seed) & (2**64 - 1), *tail)
     else:

@@ -1,0 +1,167 @@
+"""GPU parity of the joint backward launch (dQ and dK/dV tiles in one grid) and
+of the grouped backward that cuts a K/V head's query heads into parts, at the
+sizes where their launch rules and tile orders change: gradients against a
+float64 evaluation of the closed form, itself pinned to the oracle on the CPU.
+
+Tolerance: normwise ||g - ref|| / ||ref||, 2e-3 (float16) and 1.5e-2 (bfloat16),
+the bars of test_gpu_attention_bwd.py (a few units of the rounding of P, dS and
+the result to dtype).
+"""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from mlx_primitives import _native
+from mlx_primitives.attention import _launch, flash_attention, sliding_window_attention
+from oracle import attention_grad as oag
+
+NREL = {torch.float16: 2e-3, torch.bfloat16: 1.5e-2}
+
+
+def rnd(shape, seed, dtype):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(shape, generator=g).to(dtype)
+
+
+def grads64(q, k, v, dout, scale, left, right):
+    """dq, dk, dv (BSHD, float64) with query i seeing keys i - left .. i + right
+    (None: no limit); every query sees a key."""
+    B, Sq, H, D = q.shape
+    Sk, Hk = k.shape[1], k.shape[2]
+    out = [torch.zeros(x.shape, dtype=torch.float64, device=q.device) for x in (q, k, v)]
+    i = torch.arange(Sq, device=q.device)[:, None]
+    j = torch.arange(Sk, device=q.device)[None, :]
+    for b in range(B):
+        for h in range(H):
+            q1, k1, v1, d1 = (x.double().contiguous() for x in (
+                q[b, :, h], k[b, :, h // (H // Hk)], v[b, :, h // (H // Hk)], dout[b, :, h]))
+            s = (q1 @ k1.t()) * scale
+            if left is not None:
+                s.masked_fill_(j < i - left, -math.inf)
+            if right is not None:
+                s.masked_fill_(j > i + right, -math.inf)
+            p = torch.exp(s - s.amax(1, keepdim=True))
+            p = p / (p.sum(1, keepdim=True) + 1e-6)
+            ds = p * (d1 @ v1.t() - (d1 * (p @ v1)).sum(1, keepdim=True)) * scale
+            out[0][b, :, h] = ds @ k1
+            out[1][b, :, h // (H // Hk)] += ds.t() @ q1
+            out[2][b, :, h // (H // Hk)] += p.t() @ d1
+    return out
+
+
+@pytest.mark.parametrize("left,right", [(None, 0), (None, None), (5, 0), (None, 20)])
+def test_reference_matches_oracle(left, right):
+    q, d = rnd((2, 20, 4, 8), 0, torch.float32), rnd((2, 20, 4, 8), 1, torch.float32)
+    k, v = rnd((2, 40, 2, 8), 2, torch.float32), rnd((2, 40, 2, 8), 3, torch.float32)
+    want = oag.attention_grad(*(x.double().numpy() for x in (q, k, v, d)), 0.3, False,
+                              -1 if left is None else left, -1 if right is None else right)
+    for g, w in zip(grads64(q, k, v, d, 0.3, left, right), want):
+        np.testing.assert_allclose(g.numpy(), w, rtol=1e-9, atol=1e-11)
+
+
+def run(device, q, k, v, d, causal=True, window=None, dropout=0.0):
+    q, k, v = (x.to(device).requires_grad_(True) for x in (q, k, v))
+    if window is None:
+        out = flash_attention(q, k, v, causal=causal, dropout_p=dropout,
+                              enable_gqa=q.shape[2] != k.shape[2])
+    else:
+        out = sliding_window_attention(q, k, v, window, causal=causal)
+    return torch.autograd.grad(out, (q, k, v), d.to(device))
+
+
+CASES = [
+    # B, H, H_kv, Sq, Sk, D, causal, window
+    (1, 1, 1, 1, 1, 128, True, None),
+    (1, 1, 1, 2, 128, 64, False, None),
+    (1, 8, 8, 129, 257, 128, False, None),       # 8 heads: one per XCD
+    (1, 3, 3, 257, 129, 128, True, None),        # queries past the last key tile
+    (1, 8, 1, 130, 70, 128, True, None),         # 8 parts of one head
+    (2, 16, 4, 300, 300, 128, True, None),       # 4 parts
+    (1, 12, 4, 200, 333, 64, False, None),       # group of 3
+    (3, 6, 6, 260, 260, 64, True, 75),           # window, heads not a multiple of 8
+    (1, 8, 8, 400, 400, 128, False, 60),
+    (1, 1, 1, 128, 16256, 128, False, None),     # 1 + 127 tiles: the longest order
+    (1, 1, 1, 128, 16257, 128, False, None),     # 1 + 128: two launches
+    (1, 1, 1, 16129, 100, 64, True, None),       # 127 + 1
+    (4, 8, 8, 4096, 4096, 64, True, None),       # chunks of 16 heads per XCD
+    (2, 16, 16, 4096, 200, 128, False, None),    # 32 x 34 tiles: joint
+    (1, 32, 4, 4096, 4096, 128, True, None),     # 2048 tiles: paired, 4 parts
+    (1, 31, 31, 4100, 4100, 128, True, None),    # 2046 tiles: joint
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES)
+def test_joint_backward(device, dtype, case):
+    B, H, H_kv, Sq, Sk, D, causal, W = case
+    q, d = rnd((B, Sq, H, D), Sq, dtype), rnd((B, Sq, H, D), Sq + 1, dtype)
+    k, v = rnd((B, Sk, H_kv, D), Sk + 2, dtype), rnd((B, Sk, H_kv, D), Sk + 3, dtype)
+    got = run(device, q, k, v, d, causal, W)
+    left = W
+    right = (0 if causal else W) if W is not None else (max(0, Sk - Sq) if causal else None)
+    want = grads64(*(x.to(device) for x in (q, k, v, d)), 1 / math.sqrt(D), left, right)
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        assert torch.isfinite(g).all(), name
+        err = float((g.double() - w).norm())
+        # (one visible key: dq and dk vanish, rounding noise is left)
+        assert err <= NREL[dtype] * float(w.norm()) + 1e-2 * (Sk == 1), (name, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,H_kv,S", [(4, 4, 300), (8, 2, 257), (16, 16, 2000)])
+def test_joint_dropout_agrees_with_stored_schedule(device, monkeypatch, H, H_kv, S):
+    # Same keep mask from the same seed; the schedules differ in summation order
+    # and rounding of the same 16-bit P and dS.
+    q, d = rnd((1, S, H, 128), 1, torch.bfloat16), rnd((1, S, H, 128), 2, torch.bfloat16)
+    k, v = rnd((1, S, H_kv, 128), 3, torch.bfloat16), rnd((1, S, H_kv, 128), 4, torch.bfloat16)
+    got = {}
+    for stored in (True, None):
+        monkeypatch.setattr(_launch, "BWD_STORED_DS", stored)
+        torch.manual_seed(5)
+        got[stored] = run(device, q, k, v, d, dropout=0.2)
+    for name, a, b in zip(("dq", "dk", "dv"), got[True], got[None]):
+        rel = float((a.double() - b.double()).norm() / a.double().norm())
+        assert rel <= 4e-3, (name, rel)
+
+
+@pytest.mark.gpu
+def test_grouped_backward_without_room_for_parts(device):
+    # A workspace for Dvec alone: each group is one part, the same gradients up
+    # to summation order.
+    B, H, H_kv, S, D = 1, 8, 2, 300, 128
+    q, d = rnd((B, S, H, D), 1, torch.float16).to(device), rnd((B, S, H, D), 2, torch.float16).to(device)
+    k, v = (rnd((B, S, H_kv, D), s, torch.float16).to(device) for s in (3, 4))
+    lib = _native.load()
+    want = run(device, q, k, v, d)
+    o, lse = torch.empty_like(q), torch.empty(B, H, S, device=device)
+    bhs = lambda x: (x.stride(0), x.stride(2), x.stride(1))
+    _native.attn_fwd(q, k, v, o, bhs(q), bhs(k), bhs(v), bhs(o), B, H, S, S, D, D ** -0.5, True,
+                     H_kv=H_kv, lse=lse)
+    got = [torch.empty_like(x) for x in (q, k, v)]
+    ws = torch.empty(lib.mpx_attn_bwd_workspace_bytes(B, H, S), dtype=torch.uint8, device=device)
+    rc = lib.mpx_attn_bwd_grouped(
+        *(x.data_ptr() for x in (q, k, v, o, d, lse, *got)),
+        *(_native._strides(bhs(x)) for x in (q, k, v, o, d, *got)), B, H, H_kv, S, S, D,
+        D ** -0.5, 1, -1, -1, _native.dtype_code(q.dtype), 0.0, 0, ws.data_ptr(), ws.numel(),
+        _native._stream_ptr(device))
+    assert rc == _native.MPX_OK
+    for a, b in zip(got, want):
+        assert float((a.double() - b.double()).norm() / b.double().norm()) <= 1e-3
+
+
+def test_grouped_workspace_bytes():
+    lib = _native.load()
+    ws = lib.mpx_attn_bwd_grouped_workspace_bytes
+    plain = lib.mpx_attn_bwd_workspace_bytes(1, 8, 300)
+    assert ws(1, 8, 8, 300, 300, 128, 2, -1) == plain       # no groups
+    assert ws(1, 8, 2, 300, 300, 256, 2, -1) == plain       # no parts at head dim 256
+    assert ws(1, 8, 2, 300, 300, 128, 0, -1) == plain       # nor in float32
+    # 4 parts of 2 K/V heads, dK and dV sums in float32
+    assert ws(1, 8, 2, 300, 300, 128, 2, -1) == -(-plain // 256) * 256 + 2 * 8 * 300 * 128 * 4
+    assert ws(1, 8, 3, 300, 300, 128, 2, -1) == 0
+    # parts stop at one workgroup per slot of the chip
+    assert ws(4, 32, 8, 4096, 4096, 128, 2, -1) == lib.mpx_attn_bwd_workspace_bytes(4, 32, 4096)
