@@ -7,8 +7,9 @@
 // bias slope_h * (t - context_len) (163-178); exact softmax.
 //
 // Design (memory bound, ~1 FLOP/byte):
-//   * split-K: each sequence's tokens are cut into partitions of PART tokens;
-//     a workgroup = 2 or 4 waves = consecutive query heads of one (sequence,
+//   * split-K: each sequence's tokens are cut into partitions of 512 tokens,
+//     down to 64 where the call would not fill the chip (decode_part); a
+//     workgroup = 2 or 4 waves = consecutive query heads of one (sequence,
 //     partition), so its waves stream adjacent head rows of the same pages
 //     (or, with grouped-query heads, share them);
 //   * one pass over the partition: a token row of one head is read by LPT
@@ -41,14 +42,15 @@ struct DecodeParams {
   float* ws_o;   // (B, H, max_parts, D)
   float* ws_ml;  // (B, H, max_parts, 2), m in log2 units
   int B, H, num_blocks, bs, max_blocks, max_parts;
+  int part;  // tokens per partition (at most kPart)
   int H_kv, kv_group;  // K/V heads of the pools; query heads per K/V head
   int dp;   // head dim of q, the pools and o (elements, <= the kernel's D)
   float c;  // scale * log2(e)
   u32 pool_bytes;  // bytes of one pool; 0: 4 GiB - 256 bytes or more (64-bit addressing)
 };
 
-// Tokens per partition and 16-byte loads in flight per lane (overridable at
-// build time for tuning builds).
+// Most tokens per partition and 16-byte loads in flight per lane (overridable
+// at build time for tuning builds).
 #ifndef MPX_PD_PART
 #define MPX_PD_PART 512
 #endif
@@ -113,9 +115,9 @@ __global__ __launch_bounds__(64 * kHeadsPerWG<NT>) void paged_decode_part_kernel
   const int h = blockIdx.x * kHeadsPerWG<NT> + wave;
   const int part = blockIdx.y, b = blockIdx.z;
   const int ctx = max(0, min(p.cl[b], p.max_blocks * p.bs));
-  const int p0 = part * kPart;
+  const int p0 = part * p.part;
   if (p0 >= ctx) return;  // uniform over the workgroup
-  const int p1 = min(p0 + kPart, ctx);
+  const int p1 = min(p0 + p.part, ctx);
   const int pg0 = p0 / p.bs;
   const int npg = (p1 - 1) / p.bs - pg0 + 1;
 
@@ -232,59 +234,79 @@ __global__ __launch_bounds__(64 * kHeadsPerWG<NT>) void paged_decode_part_kernel
 
 // Combine the partitions of one (sequence, head): the online-softmax merge
 // (mlx_primitives/attention/_online_softmax.py:42-106) over all partitions,
-// then the exact normalisation o / l of the reference's softmax. One wave per
-// (sequence, head): lane i takes the (m, l) of partition i and its weight
+// then the exact normalisation o / l of the reference's softmax. W waves per
+// (sequence, head), wave w taking chunks w, w + W, ... of 16 partitions: lane
+// i < 16 of a chunk takes the (m, l) of its partition i and the weight
 // 2^(m_i - M), lane l accumulates dims 2l, 2l+1 over the partitions (16
-// partition rows in flight, each a coalesced 2 D-float read). D is the kernel
-// head dim (the partials' row length); dp <= D columns are written. Head dims
-// above 128 take one workgroup per 128 dims (blockIdx.y).
-template <int DT>
-__global__ __launch_bounds__(64) void paged_decode_merge_kernel(DecodeParams p, int D) {
+// partition rows in flight, each a coalesced 2 D-float read); the waves'
+// (acc, M, L) meet in LDS. D is the kernel head dim (the partials' row
+// length); dp <= D columns are written. Head dims above 128 take one workgroup
+// per 128 dims (blockIdx.y).
+template <int DT, int W>
+__global__ __launch_bounds__(64 * W) void paged_decode_merge_kernel(DecodeParams p, int D) {
   const int bh = blockIdx.x;
   const int b = bh / p.H, h = bh - (bh / p.H) * p.H;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ctx = max(0, min(p.cl[b], p.max_blocks * p.bs));
-  const int nparts = (ctx + kPart - 1) / kPart;
+  const int nparts = (ctx + p.part - 1) / p.part;
   const int64_t base = (int64_t)bh * p.max_parts;
   const int d = 2 * lane + 128 * (int)blockIdx.y;
   const bool dl = d < D;
-  // Online over chunks of 64 partitions (one chunk up to 32768 tokens): a
-  // chunk's (m, l) and its first 16 partition rows are requested together.
+  // A chunk's (m, l) and its partition rows are requested together.
   float M = -INFINITY, L = 0.f, acc0 = 0.f, acc1 = 0.f;
-  for (int i0 = 0; i0 < nparts; i0 += 64) {
-    const int n = min(64, nparts - i0);
+  for (int i0 = 16 * wave; i0 < nparts; i0 += 16 * W) {
+    const int n = min(16, nparts - i0);
     float mi = -INFINITY, li = 0.f;
     if (lane < n) {
       mi = p.ws_ml[2 * (base + i0 + lane)];
       li = p.ws_ml[2 * (base + i0 + lane) + 1];
     }
-    float w = 0.f;
-    for (int k = 0; k < n; k += 16) {
-      float2 ov[16];
+    float2 ov[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u)
-        ov[u] = (k + u < n && dl) ? *(const float2*)(p.ws_o + (base + i0 + k + u) * D + d)
-                                  : make_float2(0.f, 0.f);
-      if (k == 0) {
-        const float mn = fmaxf(M, wave_max(mi));
-        const float keep = M == -INFINITY ? 0.f : fast_exp2(M - mn);
-        acc0 *= keep;
-        acc1 *= keep;
-        L *= keep;
-        M = mn;
-        // 0 for partitions that saw no key (and while no partition has)
-        w = (lane < n && M != -INFINITY) ? fast_exp2(mi - M) : 0.f;
-        L += w * li;
-      }
+    for (int u = 0; u < 16; ++u)
+      ov[u] = (u < n && dl) ? *(const float2*)(p.ws_o + (base + i0 + u) * D + d)
+                            : make_float2(0.f, 0.f);
+    const float mn = fmaxf(M, wave_max(mi));
+    const float keep = M == -INFINITY ? 0.f : fast_exp2(M - mn);
+    acc0 *= keep;
+    acc1 *= keep;
+    L *= keep;
+    M = mn;
+    // 0 for partitions that saw no key (and while no partition has)
+    const float w = (lane < n && M != -INFINITY) ? fast_exp2(mi - M) : 0.f;
+    L += w * li;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const float wk = __shfl(w, k + u, 64);
-        acc0 = fmaf(wk, ov[u].x, acc0);
-        acc1 = fmaf(wk, ov[u].y, acc1);
-      }
+    for (int u = 0; u < 16; ++u) {
+      const float wk = __shfl(w, u, 64);
+      acc0 = fmaf(wk, ov[u].x, acc0);
+      acc1 = fmaf(wk, ov[u].y, acc1);
     }
   }
   L = wave_sum(L);
+  if constexpr (W > 1) {
+    __shared__ float accs[W][2][64];
+    __shared__ float mls[W][2];
+    accs[wave][0][lane] = acc0;
+    accs[wave][1][lane] = acc1;
+    if (lane == 0) {
+      mls[wave][0] = M;
+      mls[wave][1] = L;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float mx = mls[0][0];
+#pragma unroll
+    for (int k = 1; k < W; ++k) mx = fmaxf(mx, mls[k][0]);
+    acc0 = acc1 = L = 0.f;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      const float f = mls[k][0] == -INFINITY ? 0.f : fast_exp2(mls[k][0] - mx);
+      acc0 = fmaf(f, accs[k][0][lane], acc0);
+      acc1 = fmaf(f, accs[k][1][lane], acc1);
+      L = fmaf(f, mls[k][1], L);
+    }
+  }
   if (d >= p.dp) return;
   // no valid token: 0 / 0 = NaN, as the reference
   const float out0 = acc0 / L, out1 = acc1 / L;
@@ -307,7 +329,7 @@ __global__ __launch_bounds__(64) void paged_decode_merge_kernel(DecodeParams p, 
 
 // ---------------------------------------------------------------------------
 // Grouped-query decode on MFMAs (16-bit, head dim 128, 2..16 query heads per
-// K/V head). A wave owns one (sequence, K/V head, partition of kPart tokens)
+// K/V head). A wave owns one (sequence, K/V head, partition)
 // and scores every K row against all query heads of the group at once:
 //   S^T (16 tokens x 16 heads) = K (16 x 128) Q^T (128 x 16): four 16x16x32
 //   MFMAs per 16 tokens (columns past the group are zero heads);
@@ -357,9 +379,9 @@ __global__ __launch_bounds__(64 * kGqaWaves) void paged_decode_gqa_kernel(Decode
   // read all heads of the same token rows (whole rows of the pool's pages).
   const int hk = blockIdx.x, part = blockIdx.y * kGqaWaves + wave, b = blockIdx.z;
   const int ctx = max(0, min(p.cl[b], p.max_blocks * p.bs));
-  const int p0 = part * kPart;
+  const int p0 = part * p.part;
   if (p0 >= ctx) return;  // uniform over the wave
-  const int p1 = min(p0 + kPart, ctx);
+  const int p1 = min(p0 + p.part, ctx);
   const int bsh = POW2 ? __builtin_ctz((unsigned)p.bs) : 0;
   auto page_of = [&](int t) __attribute__((always_inline)) { return POW2 ? t >> bsh : t / p.bs; };
   auto slot_of = [&](int t) __attribute__((always_inline)) {
@@ -554,17 +576,24 @@ __global__ __launch_bounds__(64 * kGqaWaves) void paged_decode_gqa_kernel(Decode
 
 namespace {
 
-int max_parts_for(int block_size, int max_blocks) {
+int max_parts_for(int block_size, int max_blocks, int part) {
   const long tokens = (long)block_size * max_blocks;
-  return (int)((tokens + kPart - 1) / kPart);
+  return (int)std::max(1L, (tokens + part - 1) / part);
 }
 
 // Kernel head dim serving pools of head dim D (<= 256): 32, 64, 128 or 256.
 int kernel_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256; }
 
-// Merge workgroups per (sequence, head): one per 128 dims.
-dim3 merge_grid(const DecodeParams& p, int D) {
-  return dim3(p.B * p.H, D > 128 ? D / 128 : 1);
+// One merge workgroup per (sequence, head) and 128 dims: four waves where
+// there can be more than one chunk of 16 partitions.
+template <int DT>
+hipError_t launch_merge(const DecodeParams& p, int D, hipStream_t st) {
+  const dim3 grid(p.B * p.H, D > 128 ? D / 128 : 1);
+  if (p.max_parts > 16)
+    hipLaunchKernelGGL((paged_decode_merge_kernel<DT, 4>), grid, dim3(256), 0, st, p, D);
+  else
+    hipLaunchKernelGGL((paged_decode_merge_kernel<DT, 1>), grid, dim3(64), 0, st, p, D);
+  return hipGetLastError();
 }
 
 // The grouped-query MFMA kernel serves 16-bit pools of head dim 128 with 2 to
@@ -596,8 +625,7 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t st) {
       }
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(paged_decode_merge_kernel<DT>, merge_grid(p, D), dim3(64), 0, st, p, D);
-      return hipGetLastError();
+      return launch_merge<DT>(p, D, st);
     }
   }
   if (p.kv_group == 1) {
@@ -611,8 +639,7 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t st) {
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(paged_decode_merge_kernel<DT>, merge_grid(p, D), dim3(64), 0, st, p, D);
-  return hipGetLastError();
+  return launch_merge<DT>(p, D, st);
 }
 
 template <int DT>
@@ -626,9 +653,59 @@ hipError_t dispatch_decode_d(const DecodeParams& p, int D, hipStream_t st) {
 }
 
 // Workspace bytes of one call: (o, m, l) per (sequence, head, partition).
-size_t decode_ws_bytes(int B, int H, int D, int block_size, int max_blocks) {
-  const int parts = std::max(1, max_parts_for(block_size, max_blocks));
-  return (size_t)B * H * parts * (kernel_dim(D) + 2) * sizeof(float);
+size_t decode_ws_bytes(int B, int H, int D, int block_size, int max_blocks, int part) {
+  return (size_t)B * H * max_parts_for(block_size, max_blocks, part) * (kernel_dim(D) + 2) *
+         sizeof(float);
+}
+
+// Tokens per partition: kPart, halved (down to `least`) while a call of
+// `heads` waves per sequence and partition has fewer than `target` of them and
+// the partials fit the no-allocation scratch. The host knows the tables'
+// capacity, not the contexts, so the count is an upper bound.
+int halved_part(int B, int H, long heads, int D, int block_size, int max_blocks, long target,
+                int least) {
+  int part = kPart;
+  while (part > least && B * heads * max_parts_for(block_size, max_blocks, part) < target &&
+         decode_ws_bytes(B, H, D, block_size, max_blocks, part / 2) <=
+             (size_t)MPX_NOALLOC_SCRATCH_BYTES)
+    part /= 2;
+  return part;
+}
+
+// A wave walks its partition in dependent steps of about 1 us, so few long
+// partitions leave the call waiting on a handful of waves. The grouped MFMA
+// kernel (four one-wave workgroups per CU) wants its 1024 slots filled, the
+// per-head kernel 2048 waves; below 64 tokens the merge costs what the shorter
+// walk gains. Decode times with partitions of 512 / 256 / 128 / 64 / 32
+// tokens (bf16, contexts up to the number given, 16-token pages):
+//   grouped, 4 x 2100 tokens, 32 heads over 8:  24.4 / 15.9 / 11.7 / 10.0 / 12.5 us
+//            24 x 1795, 16 over 4:              26.2 / 17.3 / 14.9 / 16.2 / 17.9
+//            64 x 8192, 32 over 8:              227 / 230 / 238 / 258 / 319
+//   per head, 4 x 1932, 32 heads of 128:        42.3 / 29.6 / 20.7 / 20.7 / 22.7
+//            32 x 4096, 32 heads of 128:        204 / 202 / 208 / 205 / 249
+//            30 x 6000, 16 heads of 64:         96.9 / 90.1 / 88.2 / 111 / 170
+// Head dims up to 64 in 16 bits take 128 tokens per batch of loads (64 at head
+// dim 128): they stop there, and gain up to a larger grid.
+constexpr long kGroupedWaves = 1024, kHeadWaves = 2048, kSmallHeadWaves = 8192;
+
+int decode_part(int B, int H, int H_kv, int D, int block_size, int max_blocks, int dtype) {
+  const int group = H / H_kv;
+  if (dtype != MPX_F32 && D == 128 && group >= 2 && group <= 16)
+    return halved_part(B, H, H_kv, D, block_size, max_blocks, kGroupedWaves, 64);
+  if (dtype != MPX_F32 && D <= 64)
+    return halved_part(B, H, H, D, block_size, max_blocks, kSmallHeadWaves, 128);
+  return halved_part(B, H, H, D, block_size, max_blocks, kHeadWaves, 64);
+}
+
+// The smallest of the partitions a call may take whatever its K/V head count
+// and dtype, which a workspace query does not name.
+int least_part(int B, int H, int D, int block_size, int max_blocks) {
+  int part = halved_part(B, H, H, D, block_size, max_blocks, kHeadWaves, 64);
+  if (D == 128)
+    part = std::min(part, halved_part(B, H, 1, D, block_size, max_blocks, kGroupedWaves, 64));
+  if (D <= 64)
+    part = std::min(part, halved_part(B, H, H, D, block_size, max_blocks, kSmallHeadWaves, 128));
+  return part;
 }
 
 // Validation, parameters and launches shared by the workspace entry and the
@@ -674,12 +751,15 @@ int paged_decode_run(const void* q, const void* k_pool, const void* v_pool,
   p.B = B; p.H = H; p.num_blocks = num_blocks; p.bs = block_size; p.max_blocks = max_blocks;
   p.H_kv = H_kv; p.kv_group = H / H_kv;
   p.dp = D;
-  p.max_parts = std::max(1, max_parts_for(block_size, max_blocks));
+  // (a workspace for partitions of kPart tokens is enough for any call)
+  p.part = decode_part(B, H, H_kv, D, block_size, max_blocks, dtype);
+  if (workspace_bytes < decode_ws_bytes(B, H, D, block_size, max_blocks, p.part)) p.part = kPart;
+  p.max_parts = max_parts_for(block_size, max_blocks, p.part);
   p.c = scale * kLog2e;
   const uint64_t pool_bytes =
       (uint64_t)num_blocks * block_size * H_kv * D * (dtype == MPX_F32 ? 4 : 2);
   p.pool_bytes = pool_bytes < 0xFFFFFF00ull ? (u32)pool_bytes : 0u;
-  const size_t need = decode_ws_bytes(B, H, D, block_size, max_blocks);
+  const size_t need = decode_ws_bytes(B, H, D, block_size, max_blocks, p.part);
   MPX_CHECK_ARG(workspace != nullptr && workspace_bytes >= need && ((uintptr_t)workspace & 15u) == 0,
                 "%s: 16-byte aligned workspace of %zu bytes required, %zu given", who, need,
                 workspace_bytes);
@@ -755,7 +835,8 @@ using namespace mpx;
 extern "C" size_t mpx_paged_decode_workspace_bytes(int B, int H, int D, int block_size,
                                                    int max_blocks) {
   if (B <= 0 || H <= 0 || D <= 0 || block_size <= 0 || max_blocks <= 0) return 0;
-  return decode_ws_bytes(B, H, D, block_size, max_blocks);
+  return decode_ws_bytes(B, H, D, block_size, max_blocks,
+                         least_part(B, H, D, block_size, max_blocks));
 }
 
 extern "C" int mpx_paged_decode_gqa(const void* q, const void* k_pool, const void* v_pool,
@@ -793,7 +874,7 @@ extern "C" int mpx_paged_decode_noalloc(const void* q, const void* k_pool, const
                                         void* stream) {
   clear_error();
   if (B > 0 && H > 0 && D > 0 && block_size > 0 && max_blocks >= 0) {
-    const size_t need = decode_ws_bytes(B, H, D, block_size, max_blocks);
+    const size_t need = decode_ws_bytes(B, H, D, block_size, max_blocks, kPart);
     MPX_CHECK_ARG(need <= (size_t)MPX_NOALLOC_SCRATCH_BYTES,
                   "mpx_paged_decode_noalloc: the call needs %zu bytes of partials, more than "
                   "the %zu-byte device scratch (B * H * ceil(max_blocks * block_size / 512) * "
