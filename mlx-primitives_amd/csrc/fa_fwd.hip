@@ -10,7 +10,8 @@ namespace mpx {
 // Host side.
 // ---------------------------------------------------------------------------
 // The dropout forward launches (fa_fwd_drop.hip).
-hipError_t dispatch_fwd_drop(const FwdParams& p, int D, int dtype, int grid, hipStream_t st);
+hipError_t dispatch_fwd_drop(const FwdParams& p, int D, int dtype, int kg, int grid,
+                             hipStream_t st);
 
 namespace {
 
@@ -29,6 +30,7 @@ int target_workgroups(int D, int dtype) {
 }
 
 struct Plan {
+  int kg;  // key groups of a workgroup's waves (make_plan)
   int BM, BN, n_qtiles, splits, tiles_per_split, win_left, win_right;
   int n_slots, paired, win_first;
   int tail_bh;  // paired: (batch, head)s per XCD run as single q-tiles at the end
@@ -54,11 +56,12 @@ int tile_n(int D, int dtype, bool paged = false, int bs_log2 = -1, bool alibi = 
   return D < 64 || !MPX_FA_DIRECT ? 64 : MPX_FA_BN16;
 }
 
-Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
-               int window_right, int dtype, int max_tiles_per_split = 1 << 30,
-               bool paged = false, int bs_log2 = -1, bool alibi = false) {
+Plan plan_for(int kg, int B, int H, int Sq, int Sk, int D, int causal, int window_left,
+              int window_right, int dtype, int max_tiles_per_split, bool paged, int bs_log2,
+              bool alibi) {
   Plan pl;
-  pl.BM = 32 * (dtype == MPX_F32 ? kNumWaves32 : (D > 128 ? kNumWavesWide : kNumWaves16));
+  pl.kg = kg;
+  pl.BM = 32 * (dtype == MPX_F32 ? kNumWaves32 : (D > 128 ? kNumWavesWide : kNumWaves16)) / kg;
   pl.BN = tile_n(D, dtype, paged, bs_log2, alibi);
   pl.win_left = window_left < 0 ? -1 : window_left;
   pl.win_right = causal ? 0 : (window_right < 0 ? -1 : window_right);
@@ -132,29 +135,105 @@ Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
   return pl;
 }
 
+// Estimated time of a 16-bit launch at D = 64 or 128, in us: steps of the CU
+// that runs the most of them times a step's time, plus the fixed part of its
+// items (Q, filling the DMA pipeline, the epilogue) and the split merge.
+// A step of 128 keys takes 3.5 / 2.3 / 1.8 us with 1 / 2 / 4 key groups at
+// D = 128 and 2.3 / 1.25 / 0.8 at D = 64 (a workgroup's row count halves each
+// time, but its tile still has to come in), an item about 6 us, splitting and
+// merging about 14.
+double plan_time(const Plan& pl, long bh, int Sq, int Sk, int D) {
+  static const double kStep[2][3] = {{2.3, 1.25, 0.8}, {3.5, 2.3, 1.8}};
+  const double step = kStep[D == 128][pl.kg == 4 ? 2 : pl.kg - 1] * pl.BN / 128;
+  const double item = pl.kg == 1 ? 6.0 : 7.2;
+  const double cus = kNumCUs;
+  if (pl.splits > 1) {
+    const double wgs = (double)bh * (pl.var_split > 0 ? pl.var_split : pl.n_qtiles * pl.splits);
+    return std::ceil(wgs / cus) * (pl.tiles_per_split * step + item) + 14.0;
+  }
+  double longest = 0, total = 0;
+  for (int t = 0; t < pl.n_qtiles; ++t) {
+    const int n = qtile_kv_tiles(t, pl.BM, pl.BN, Sq, Sk, pl.win_left, pl.win_right);
+    total += n;
+    longest = std::max<double>(longest, n);
+  }
+  const double wgs = (double)bh * pl.n_slots, mean = total / pl.n_slots;
+  if (pl.paired) longest = mean;  // (equal pairs)
+  const double items = (pl.paired ? 2.0 : 1.0) * item;
+  if (wgs <= cus) return longest * step + items;
+  // (tail_bh: the launch ends with single q-tiles, about two steps uneven)
+  const double steps =
+      pl.tail_bh > 0 ? 1.05 * mean * wgs / cus + 2
+      : longest <= 1.1 * mean ? std::ceil(wgs / cus) * longest : mean * wgs / cus + longest / 2;
+  return steps * step + items * wgs / cus;
+}
+
+// The plan of a call. Launches of the 16-bit kernels at D = 64 and 128 that
+// leave CUs empty (one workgroup per CU) may cut the waves of a workgroup into
+// 2 or 4 key groups: q-tiles of 128 or 64 rows, so 2 or 4 times the
+// workgroups, each wave a half or a quarter of every tile's keys, the groups'
+// results merged in LDS. Causal bf16 forward with 1 / 2 / 4 groups, (batch, S,
+// heads, D): (1, 777, 32, 128) 26.9 / 20.4 / 29.1 us, (2, 2048, 16, 128) 55.4 /
+// 47.6 / 72.4, (1, 1024, 16, 128) 34.9 / 30.7 / 19.4 (the first two split the
+// keys), (2, 1024, 16, 64) 27.8 / 15.8 / 17.6; one query of (8, 32, 128) over
+// 2048 keys 56.8 / 35.1 / 27.9; (4, 2048, 32, 128), a full launch, 152 / 181 /
+// 277. The line between them is an estimate (plan_time), not a size.
+Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
+               int window_right, int dtype, int max_tiles_per_split = 1 << 30,
+               bool paged = false, int bs_log2 = -1, bool alibi = false) {
+  auto plan = [&](int kg) {
+    return plan_for(kg, B, H, Sq, Sk, D, causal, window_left, window_right, dtype,
+                    max_tiles_per_split, paged, bs_log2, alibi);
+  };
+  Plan best = plan(1);
+  const long bh = (long)B * H;
+  if (dtype == MPX_F32 || (D != 64 && D != 128) || !MPX_FA_DIRECT ||
+      bh * best.n_qtiles > 2 * kNumCUs)
+    return best;
+  double t = plan_time(best, bh, Sq, Sk, D);
+  for (int kg = 2; kg <= (best.BN == 128 ? 4 : 2); kg *= 2) {
+    const Plan pl = plan(kg);
+    const double tk = plan_time(pl, bh, Sq, Sk, D);
+    if (tk < 0.97 * t) {
+      best = pl;
+      t = tk;
+    }
+  }
+  return best;
+}
+
 // BIG: 16-bit paged pools of 4 GiB and more (p.pool_bytes == 0).
 template <int D, int BN, bool F32, bool BF16, bool PAGED, bool BIG = false>
-hipError_t launch_fwd(const FwdParams& p, int grid, hipStream_t stream) {
+hipError_t launch_fwd(const FwdParams& p, int kg, int grid, hipStream_t stream) {
+#define MPX_FWD16(KG)                                                                          \
+  hipLaunchKernelGGL((fa_fwd16_kernel<D, BN, kNumWaves16, BF16, PAGED, BIG, KG>), dim3(grid), \
+                     dim3(64 * kNumWaves16), 0, stream, p)
   if constexpr (F32) {
     hipLaunchKernelGGL((fa_fwd32_kernel<D, BN, kNumWaves32, PAGED>), dim3(grid),
                        dim3(64 * kNumWaves32), 0, stream, p);
+  } else if constexpr (D >= 64) {
+    if (kg == 1) MPX_FWD16(1);
+    if (kg == 2) MPX_FWD16(2);
+    if constexpr (BN == 128) {
+      if (kg == 4) MPX_FWD16(4);
+    }
   } else {
-    hipLaunchKernelGGL((fa_fwd16_kernel<D, BN, kNumWaves16, BF16, PAGED, BIG>), dim3(grid),
-                       dim3(64 * kNumWaves16), 0, stream, p);
+    MPX_FWD16(1);
   }
+#undef MPX_FWD16
   return hipGetLastError();
 }
 
 template <bool PAGED, bool BIG = false>
-hipError_t dispatch_fwd(const FwdParams& p, int D, int dtype, int grid, hipStream_t st) {
+hipError_t dispatch_fwd(const FwdParams& p, int D, int dtype, int kg, int grid, hipStream_t st) {
   if constexpr (PAGED && !BIG) {
     // 16-bit pools of 4 GiB and more: the 64-bit address forms
-    if (dtype != MPX_F32 && p.pool_bytes == 0) return dispatch_fwd<true, true>(p, D, dtype, grid, st);
+    if (dtype != MPX_F32 && p.pool_bytes == 0) return dispatch_fwd<true, true>(p, D, dtype, kg, grid, st);
   }
   if (D == 256) {
     // (16-bit: 64-key DMA-staged tiles dense, 32-key register-staged paged)
     constexpr int kBNw = PAGED ? 32 : 64;
-    if (dtype == MPX_F32) return launch_fwd<256, 32, true, false, PAGED>(p, grid, st);
+    if (dtype == MPX_F32) return launch_fwd<256, 32, true, false, PAGED>(p, kg, grid, st);
     if (dtype == MPX_BF16)
       hipLaunchKernelGGL((fa_fwd16_wide_kernel<256, kBNw, kNumWavesWide, true, PAGED, false, BIG>),
                          dim3(grid), dim3(64 * kNumWavesWide), 0, st, p);
@@ -165,27 +244,27 @@ hipError_t dispatch_fwd(const FwdParams& p, int D, int dtype, int grid, hipStrea
   }
   if constexpr (PAGED) {
     if (paged_wide_tiles(D, dtype, p.bs_log2, p.slopes != nullptr)) {
-      return dtype == MPX_BF16 ? launch_fwd<128, 128, false, true, true, BIG>(p, grid, st)
-                               : launch_fwd<128, 128, false, false, true, BIG>(p, grid, st);
+      return dtype == MPX_BF16 ? launch_fwd<128, 128, false, true, true, BIG>(p, kg, grid, st)
+                               : launch_fwd<128, 128, false, false, true, BIG>(p, kg, grid, st);
     }
   }
   if (dtype == MPX_F32) {
     switch (D) {
-      case 32: return launch_fwd<32, 64, true, false, PAGED>(p, grid, st);
-      case 64: return launch_fwd<64, 64, true, false, PAGED>(p, grid, st);
-      default: return launch_fwd<128, 32, true, false, PAGED>(p, grid, st);
+      case 32: return launch_fwd<32, 64, true, false, PAGED>(p, kg, grid, st);
+      case 64: return launch_fwd<64, 64, true, false, PAGED>(p, kg, grid, st);
+      default: return launch_fwd<128, 32, true, false, PAGED>(p, kg, grid, st);
     }
   } else if (dtype == MPX_BF16) {
     switch (D) {
-      case 32: return launch_fwd<32, kBN16<PAGED, 32>, false, true, PAGED, BIG>(p, grid, st);
-      case 64: return launch_fwd<64, kBN16<PAGED, 64>, false, true, PAGED, BIG>(p, grid, st);
-      default: return launch_fwd<128, kBN16<PAGED, 128>, false, true, PAGED, BIG>(p, grid, st);
+      case 32: return launch_fwd<32, kBN16<PAGED, 32>, false, true, PAGED, BIG>(p, kg, grid, st);
+      case 64: return launch_fwd<64, kBN16<PAGED, 64>, false, true, PAGED, BIG>(p, kg, grid, st);
+      default: return launch_fwd<128, kBN16<PAGED, 128>, false, true, PAGED, BIG>(p, kg, grid, st);
     }
   } else {
     switch (D) {
-      case 32: return launch_fwd<32, kBN16<PAGED, 32>, false, false, PAGED, BIG>(p, grid, st);
-      case 64: return launch_fwd<64, kBN16<PAGED, 64>, false, false, PAGED, BIG>(p, grid, st);
-      default: return launch_fwd<128, kBN16<PAGED, 128>, false, false, PAGED, BIG>(p, grid, st);
+      case 32: return launch_fwd<32, kBN16<PAGED, 32>, false, false, PAGED, BIG>(p, kg, grid, st);
+      case 64: return launch_fwd<64, kBN16<PAGED, 64>, false, false, PAGED, BIG>(p, kg, grid, st);
+      default: return launch_fwd<128, kBN16<PAGED, 128>, false, false, PAGED, BIG>(p, kg, grid, st);
     }
   }
 }
@@ -208,9 +287,9 @@ int run_fwd(FwdParams& p, const Plan& pl, int D, int dtype, void* workspace, hip
           : (long)p.B * p.H * (pl.var_split > 0 ? pl.var_split : (long)pl.n_slots * pl.splits);
   MPX_CHECK_ARG(grid_l < (1L << 31), "attention: problem too large");
   if (!PAGED && drop)
-    MPX_CHECK_HIP(dispatch_fwd_drop(p, D, dtype, (int)grid_l, st));
+    MPX_CHECK_HIP(dispatch_fwd_drop(p, D, dtype, pl.kg, (int)grid_l, st));
   else
-    MPX_CHECK_HIP(dispatch_fwd<PAGED>(p, D, dtype, (int)grid_l, st));
+    MPX_CHECK_HIP(dispatch_fwd<PAGED>(p, D, dtype, pl.kg, (int)grid_l, st));
   if (pl.splits > 1) {
     const MergeShape ms = {pl.var_split, pl.BM, pl.BN, p.Sk, pl.win_left, pl.win_right,
                            pl.tiles_per_split};

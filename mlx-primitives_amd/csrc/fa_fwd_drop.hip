@@ -7,10 +7,17 @@
 namespace mpx {
 
 // The dropout kernels (dense K/V, D = 64, 128 or 256).
-hipError_t dispatch_fwd_drop(const FwdParams& p, int D, int dtype, int grid, hipStream_t st) {
-#define MPX_DROP16(DD, BF)                                                                  \
-  hipLaunchKernelGGL((fa_fwd16_drop_kernel<DD, kBN16<false, DD>, kNumWaves16, BF>), dim3(grid), \
-                     dim3(64 * kNumWaves16), 0, st, p)
+hipError_t dispatch_fwd_drop(const FwdParams& p, int D, int dtype, int kg, int grid,
+                             hipStream_t st) {
+#define MPX_DROP16K(DD, BF, KG)                                                            \
+  hipLaunchKernelGGL((fa_fwd16_drop_kernel<DD, kBN16<false, DD>, kNumWaves16, BF, KG>),   \
+                     dim3(grid), dim3(64 * kNumWaves16), 0, st, p)
+#define MPX_DROP16(DD, BF)                                                                 \
+  do {                                                                                     \
+    if (kg == 1) MPX_DROP16K(DD, BF, 1);                                                   \
+    if (kg == 2) MPX_DROP16K(DD, BF, 2);                                                   \
+    if (kg == 4) MPX_DROP16K(DD, BF, 4);                                                   \
+  } while (0)
   if (D == 256) {
     if (dtype == MPX_F32)
       hipLaunchKernelGGL((fa_fwd32_kernel<256, 32, kNumWaves32, false, true>), dim3(grid),
@@ -36,6 +43,7 @@ hipError_t dispatch_fwd_drop(const FwdParams& p, int D, int dtype, int grid, hip
     if (D == 64) MPX_DROP16(64, false); else MPX_DROP16(128, false);
   }
 #undef MPX_DROP16
+#undef MPX_DROP16K
   return hipGetLastError();
 }
 

@@ -903,15 +903,18 @@ __device__ __forceinline__ int swz64(int r) { return (((r >> 1) & 1) << 2) | ((r
 // 64-bit address form (rows without a page from kZeroChunk) instead of 32-bit
 // buffer offsets.
 template <int D, int BN, int NW, bool BF16, int NST, bool PAGED, bool DROP = false,
-          bool BIG = false>
+          bool BIG = false, int KG = 1>
 __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const WorkItem wi,
                                                  unsigned char* __restrict__ st0,
                                                  unsigned char* __restrict__ st1,
                                                  unsigned char* __restrict__ st2,
                                                  unsigned char* __restrict__ st3,
                                                  int* __restrict__ pages) {
-  constexpr int BM = 32 * NW;
-  constexpr int NB = BN / 32, NSL = BN / 16, NKS = D / 16, NDB = D / 32;
+  // KG key groups: wave w = row group w % NR, key group w / NR, computes its 32
+  // rows against keys [BNW kg, +BNW) of every tile.
+  constexpr int NR = NW / KG, BM = 32 * NR, BNW = BN / KG;
+  constexpr int NB = BNW / 32, NSL = BNW / 16, NKS = D / 16, NDB = D / 32;
+  static_assert(NR * KG == NW && NB >= 1 && NB * KG * 32 == BN, "key groups");
   // Paged, 64-key tiles: the item's page ids are staged in LDS (any page
   // size, ALiBi). Paged, 128-key tiles: page ids come from the block table,
   // one per DMA instruction of a wave; the host picks this form for
@@ -976,7 +979,8 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
     __syncthreads();
   }
 
-  const int wq0 = q0 + wave * 32;
+  const int rg = KG == 1 ? wave : wave % NR, kg = KG == 1 ? 0 : wave / NR;
+  const int wq0 = q0 + rg * 32;
   const int myq = wq0 + j;
   // Dropout: this row's key of the keep-mask hash.
   const u32 drop_rk =
@@ -1374,17 +1378,21 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
     l_run += lsum[0] + lsum[1];
   };
 
-  auto compute_tile = [&](const unsigned char* Kb, int kv0) __attribute__((always_inline)) {
+  // (key groups: the tile's page masks are made by waves of every group)
+  auto compute_tile = [&](const unsigned char* Kt, int kvt) __attribute__((always_inline)) {
     bool skip, full;
-    classify_tile<BN>(p, kv0, wq0, wq0 + 31, skip, full);
+    const int kv0 = kvt + kg * BNW;
+    const unsigned char* const Kb = Kt + kg * BNW * ROWB;
+    classify_tile<BNW>(p, kv0, wq0, wq0 + 31, skip, full);
     if (skip) return;
     bool pmask = false;
     if constexpr (kSlice) {
       // Lane l checks key kv0 + l (one 64-bit ballot per tile).
-      const int key = kv0 + lane;
+      const int key = kvt + lane;
       bool ok = key < p.Sk;
       if (ok) ok = pages[page_of(p, key) - pg_first] >= 0;
       vmask = __ballot(ok);
+      if constexpr (KG > 1) vmask = (vmask >> (kg * BNW)) | (BNW < 64 ? ~0ull << (BNW & 63) : 0);
       pmask = vmask != ~0ull || alibi != 0.f;
     }
     if constexpr (kChecked) {
@@ -1392,12 +1400,14 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
         // Lane l checks keys kv0 + l and kv0 + 64 + l against the table. The
         // loads are waited for here (vmcnt(0)), so the tile waits below
         // still count DMA loads only.
-        const int k0 = kv0 + lane, k1 = k0 + 64;
+        const int k0 = kvt + lane, k1 = k0 + 64;
         const int b0 = bt_row[min(k0, p.Sk - 1) >> p.bs_log2];
         const int b1 = bt_row[min(k1, p.Sk - 1) >> p.bs_log2];
         __builtin_amdgcn_s_waitcnt(0x0F70);
         vmask = __ballot((k0 < p.Sk) & (b0 >= 0) & (b0 < p.num_blocks));
         vmask_hi = __ballot((k1 < p.Sk) & (b1 >= 0) & (b1 < p.num_blocks));
+        // (this wave's keys in the low bits)
+        if constexpr (KG > 1) vmask = (kg * BNW >= 64 ? vmask_hi : vmask) >> (kg * BNW & 63);
       } else {
         vmask = vmask_hi = ~0ull;  // (a previous tile may have set them)
       }
@@ -1463,6 +1473,59 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
     if (NST == 4 && i + 3 < n_tiles) step(i + 3, Const<3 % NST>{});
   }
 
+  // Key groups: groups 1 .. KG - 1 leave their (O, m_run, m_max, l_run) in the
+  // idle stages and group 0 adds them up (the online-softmax merge); the region
+  // a wave of group 0 reads is also the one its output rows go through.
+  constexpr int kRegB = NDB * 16 * 64 * 4;       // a wave's O (float32)
+  constexpr int kRegPer = STAGEB / kRegB > 0 ? STAGEB / kRegB : 1;  // regions per stage
+  auto region = [&](int r) __attribute__((always_inline)) -> unsigned char* {
+    const int st = r / kRegPer;
+    unsigned char* const b = st == 0 ? st0 : (st == 1 ? st1 : (st == 2 ? st2 : st3));
+    return b + (r - st * kRegPer) * kRegB;
+  };
+  if constexpr (KG > 1) {
+    static_assert((KG - 1) * NR <= kRegPer * NST, "a region per wave of groups 1 ..");
+    // (each wave's m_run, m_max and l_run, past the regions)
+    float(*const kg_ml)[3][64] =
+        (float(*)[3][64])((NST >= 3 ? st2 : st1) + STAGEB - NW * 3 * 64 * 4);
+    static_assert(NST >= 3 ? (KG - 1) * NR <= 2 * kRegPer
+                           : ((KG - 1) * NR - kRegPer) * kRegB + NW * 768 <= STAGEB,
+                  "the regions end below kg_ml");
+    if (kg > 0) {
+      f32x4* const dst = (f32x4*)region((kg - 1) * NR + rg) + lane;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4)
+          dst[(4 * db + e4) * 64] = (f32x4){o[db][4 * e4], o[db][4 * e4 + 1], o[db][4 * e4 + 2],
+                                            o[db][4 * e4 + 3]};
+      kg_ml[wave][0][lane] = m_run;
+      kg_ml[wave][1][lane] = m_max;
+      kg_ml[wave][2][lane] = l_run;
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int k = 1; k < KG; ++k) {
+        const float mr = kg_ml[k * NR + rg][0][lane], lr_ = kg_ml[k * NR + rg][2][lane];
+        m_max = fmaxf(m_max, kg_ml[k * NR + rg][1][lane]);
+        const float mn = fmaxf(m_run, mr);
+        const float a0 = m_run == -INFINITY ? 0.f : fast_exp2(m_run - mn);
+        const float a1 = mr == -INFINITY ? 0.f : fast_exp2(mr - mn);
+        l_run = l_run * a0 + lr_ * a1;
+        m_run = mn;
+        const f32x4* const src = (const f32x4*)region((k - 1) * NR + rg) + lane;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int e4 = 0; e4 < 4; ++e4) {
+            const f32x4 x = src[(4 * db + e4) * 64];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[db][4 * e4 + i] = o[db][4 * e4 + i] * a0 + x[i] * a1;
+          }
+      }
+    }
+  }
   const float l_tot = pair_sum32(l_run);
   const float f = m_max == -INFINITY ? 0.f : fast_exp2(m_run - m_max);
   // (dropout: kept weights times 1 / (1 - p); the row sums stay unscaled)
@@ -1477,15 +1540,17 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
     // chunk) and the row reads are free of bank conflicts.
     constexpr int CPR = ROWB / 16, RPI = 64 / CPR, OWB = 32 * ROWB;
     auto oswz = [](int r) { return CPR >= 16 ? (r & 15) : ((r >> 1) & 7); };
-    unsigned char* const eb = NW * OWB <= STAGEB
-                                  ? st0 + wave * OWB
-                                  : (wave < NW / 2 ? st0 : st1) + (wave % (NW / 2)) * OWB;
+    unsigned char* const eb =
+        KG > 1 ? region(rg)
+               : (NW * OWB <= STAGEB ? st0 + wave * OWB
+                                     : (wave < NW / 2 ? st0 : st1) + (wave % (NW / 2)) * OWB);
+    static_assert(KG == 1 || OWB <= kRegB, "output rows fit a region");
     // (the lane index taken afresh: addresses derived from it are not hoisted
     // into registers the tile loop needs)
     int ln = lane;
     asm volatile("" : "+v"(ln));
     const int jr = ln & 31, gr = ln >> 5;
-    if (myq < p.Sq) {
+    if (kg == 0 && myq < p.Sq) {
       const float inv = m_max == -INFINITY ? (p.nan_empty ? __builtin_nanf("") : 0.f)
                                            : fo / (l_tot * f + p.eps);
       if (p.lse && g == 0)
@@ -1503,15 +1568,17 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
         }
     }
     uint16_t* const Ob = (uint16_t*)p.o + wi.b * p.o_sb + wi.h * p.o_sh;
+    if (kg == 0) {
 #pragma unroll
-    for (int i = 0; i < 32 / RPI; ++i) {
-      const int r = RPI * i + ln / CPR, c = ln % CPR;
-      const u32x4 val = *(const u32x4*)(eb + r * ROWB + (c ^ oswz(r)) * 16);
-      if (wq0 + r < p.Sq) *(u32x4*)(Ob + (int64_t)(wq0 + r) * p.o_ss + 8 * c) = val;
+      for (int i = 0; i < 32 / RPI; ++i) {
+        const int r = RPI * i + ln / CPR, c = ln % CPR;
+        const u32x4 val = *(const u32x4*)(eb + r * ROWB + (c ^ oswz(r)) * 16);
+        if (wq0 + r < p.Sq) *(u32x4*)(Ob + (int64_t)(wq0 + r) * p.o_ss + 8 * c) = val;
+      }
     }
     stage_barrier();  // every wave's rows read before the next item restages LDS
   } else if (p.num_splits == 1) {
-    if (myq < p.Sq) {
+    if (kg == 0 && myq < p.Sq) {
       const float inv = m_max == -INFINITY ? (p.nan_empty ? __builtin_nanf("") : 0.f)
                                            : fo / (l_tot * f + p.eps);
       if (p.lse && g == 0)
@@ -1528,7 +1595,7 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
           *(u32x2*)(Op + d) = val;
         }
     }
-  } else if (myq < p.Sq) {
+  } else if (kg == 0 && myq < p.Sq) {
     const int64_t row = (((int64_t)wi.split * p.B + wi.b) * p.H + wi.h) * p.Sq + myq;
     float* wo = p.ws_o + row * D;
 #pragma unroll
@@ -1546,7 +1613,7 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
   }
 }
 
-template <int D, int BN, int NW, bool BF16, bool PAGED, bool BIG = false>
+template <int D, int BN, int NW, bool BF16, bool PAGED, bool BIG = false, int KG = 1>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MPX_FA_WAVES_PER_EU)))
 void fa_fwd16_kernel(FwdParams p) {
   // Stay within 128 KB of LDS per workgroup (a 136 KB configuration gave wrong
@@ -1580,7 +1647,7 @@ void fa_fwd16_kernel(FwdParams p) {
 #pragma nounroll
   for (int item = 0; item < n_items; ++item) {
     if constexpr (kDirect)
-      fa16_rows_direct<D, BN, NW, BF16, kDStages, PAGED, false, BIG>(
+      fa16_rows_direct<D, BN, NW, BF16, kDStages, PAGED, false, BIG, KG>(
           p, slot_item(p, ws, item), dst0, dst1, dst2, dst3, pages);
     else
       fa16_rows<D, BN, NW, BF16, PAGED, false, BIG>(p, slot_item(p, ws, item), smem, pages);
@@ -1589,7 +1656,7 @@ void fa_fwd16_kernel(FwdParams p) {
 
 // The same with dropout on the weights (dense K/V, D = 64 or 128: the direct
 // kernels).
-template <int D, int BN, int NW, bool BF16>
+template <int D, int BN, int NW, bool BF16, int KG = 1>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MPX_FA_WAVES_PER_EU)))
 void fa_fwd16_drop_kernel(FwdParams p) {
   constexpr int kDStages = MPX_FA_DSTAGES > 0 ? MPX_FA_DSTAGES
@@ -1606,8 +1673,8 @@ void fa_fwd16_drop_kernel(FwdParams p) {
   const int n_items = slot_items(p, ws);
 #pragma nounroll
   for (int item = 0; item < n_items; ++item)
-    fa16_rows_direct<D, BN, NW, BF16, kDStages, false, true>(p, slot_item(p, ws, item), dst0, dst1,
-                                                             dst2, dst3, nullptr);
+    fa16_rows_direct<D, BN, NW, BF16, kDStages, false, true, false, KG>(
+        p, slot_item(p, ws, item), dst0, dst1, dst2, dst3, nullptr);
 }
 
 // Head dims 129 .. 256 (zero-padded to 256): four waves of one wave per SIMD,

@@ -1,0 +1,157 @@
+"""GPU parity of the forward launches that cut a workgroup's waves into key
+groups (q-tiles of 128 or 64 rows, every wave a part of each key tile, results
+merged in LDS): sizes around the row groups, the key parts and the tiles, with
+rows whose keys all lie in one group, against the float64 oracle. Bars: 2e-2
+absolute, the repository's 16-bit forward bar."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from mlx_primitives import _native
+from mlx_primitives.attention import flash_attention, sliding_window_attention
+from mlx_primitives.cache import paged_attention
+from mlx_primitives.kernels import fused_rope_attention, precompute_rope_cache, rope
+from oracle import attention as oa
+from oracle import paged as op
+
+pytestmark = pytest.mark.gpu
+
+
+def rnd(shape, seed, dtype):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def dense(q, k, v, left, right):
+    """float64 attention, BSHD, query i seeing keys i - left .. i + right."""
+    q, k, v = (x.double().numpy() for x in (q, k, v))
+    g = q.shape[2] // k.shape[2]
+    k, v = np.repeat(k, g, 2), np.repeat(v, g, 2)
+    s = np.einsum("bqhd,bkhd->bhqk", q, k) / math.sqrt(q.shape[-1])
+    i, j = np.arange(q.shape[1])[:, None], np.arange(k.shape[1])[None, :]
+    keep = np.ones(s.shape[-2:], bool)
+    if left is not None:
+        keep &= j >= i - left
+    if right is not None:
+        keep &= j <= i + right
+    s = np.where(keep, s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True) + 1e-6
+    return np.einsum("bhqk,bkhd->bqhd", p, v)
+
+
+SIZES = [  # B, H, H_kv, Sq, Sk
+    (1, 2, 2, 1, 1), (1, 2, 1, 1, 2048), (2, 8, 2, 3, 700), (1, 4, 4, 31, 33), (1, 4, 4, 65, 127),
+    (1, 8, 8, 64, 129), (1, 16, 16, 257, 257), (1, 4, 2, 300, 300), (2, 16, 16, 512, 512),
+    (1, 16, 16, 1000, 1000), (1, 8, 8, 1025, 1025), (2, 8, 8, 130, 1100), (1, 3, 1, 777, 777),
+]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("causal", [True, False])
+def test_dense(device, size, dtype, D, causal):
+    B, H, H_kv, Sq, Sk = size
+    q = rnd((B, Sq, H, D), 1, dtype)
+    k, v = rnd((B, Sk, H_kv, D), 2, dtype), rnd((B, Sk, H_kv, D), 3, dtype)
+    out = flash_attention(*(x.to(device) for x in (q, k, v)), causal=causal, enable_gqa=H != H_kv)
+    want = dense(q, k, v, None, max(0, Sk - Sq) if causal else None)
+    np.testing.assert_allclose(out.double().cpu().numpy(), want, rtol=0, atol=2e-2)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S,W,causal", [(700, 0, True), (700, 30, True), (1000, 63, False),
+                                        (513, 200, True), (300, 299, False)])
+def test_window(device, S, W, causal, D):
+    q, k, v = (rnd((1, S, 12, D), i, torch.bfloat16) for i in range(3))
+    out = sliding_window_attention(*(x.to(device) for x in (q, k, v)), W, causal=causal)
+    np.testing.assert_allclose(out.double().cpu().numpy(),
+                               dense(q, k, v, W, 0 if causal else W), rtol=0, atol=2e-2)
+
+
+@pytest.mark.parametrize("D,scale,mult", [(128, -0.2, 1.0), (64, 0.125, 3.0), (128, 0.001, 1.0)])
+def test_scales(device, D, scale, mult):
+    # Negative, larger and near-zero scores. The kernels round Q times the scale
+    # to bfloat16, an error of 2^-9 / sqrt(3) of a score's spread, which is at
+    # most 3 here: 3.4e-3 of a weight, well inside the bar. (A spread of 80, D =
+    # 64 at scale 1 and inputs times 10, moves weights by a third with any tile.)
+    q, k, v = (rnd((1, 400, 8, D), i + 5, torch.bfloat16) for i in range(3))
+    q = q * mult
+    out = flash_attention(*(x.to(device) for x in (q, k, v)), scale=scale, causal=True)
+    want = oa.flash_attention(*(x.double().numpy() for x in (q, k, v)), scale=scale, causal=True)
+    np.testing.assert_allclose(out.double().cpu().numpy(), want, rtol=0, atol=2e-2)
+
+
+def test_one_group_dominates(device):
+    # All the weight on one key, in each 32-key part of the tile in turn: the
+    # merge rescales the other groups' sums to nothing.
+    S, D = 512, 128
+    for at in (0, 33, 70, 127, 128, 255, 511):
+        k = torch.zeros(1, S, 4, D)
+        k[:, at] = 30.0
+        q = torch.ones(1, S, 4, D)
+        v = rnd((1, S, 4, D), at, torch.float16)
+        out = flash_attention(*(x.half().to(device) for x in (q, k, v)), causal=False)
+        want = v[:, at:at + 1].expand(1, S, 4, D)
+        assert float((out.cpu().float() - want.float()).abs().max()) <= 2e-3, at
+
+
+@pytest.mark.parametrize("bs", [16, 24, 64])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("alibi", [False, True])
+def test_paged_prefill_missing_pages(device, D, bs, alibi):
+    B, Sq, H, H_kv = 3, 400, 8, 4
+    lens = [400, 333, 0]
+    pages = -(-Sq // bs) + 1
+    g = torch.Generator().manual_seed(bs)
+    tables = torch.randperm(B * pages, generator=g).to(torch.int32).reshape(B, pages)
+    tables[0, 1] = -1             # one page of the first tile
+    tables[1, 128 // bs] = B * pages + 7  # an id past the pool in the second tile
+    q = rnd((B, Sq, H, D), 1, torch.float16)
+    kp, vp = (rnd((B * pages, bs, H_kv, D), s, torch.float16) for s in (2, 3))
+    cl = torch.tensor(lens, dtype=torch.int32)
+    slopes = torch.rand(H, generator=g) * 0.1 if alibi else None
+    out = paged_attention(*(x.to(device) for x in (q, kp, vp, tables, cl)), block_size=bs,
+                          alibi_slopes=None if slopes is None else slopes.to(device),
+                          enable_gqa=True)
+    tb = tables.clone()
+    tb[tb >= B * pages] = -1
+    rep = lambda x: x.double().repeat_interleave(H // H_kv, dim=2).numpy()
+    want = op.paged_attention_prefill(q.double().numpy(), rep(kp), rep(vp), tb.numpy(), cl.numpy(),
+                                      1 / math.sqrt(D), bs, True,
+                                      None if slopes is None else slopes.double().numpy())
+    got = out.double().cpu().numpy()
+    assert (np.isnan(got) == np.isnan(want)).all() and np.isnan(got[2]).all()
+    np.testing.assert_allclose(got[:2], want[:2], rtol=0, atol=2e-2)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_rope_on_load_equals_rope_first(device, D):
+    # Q rotated by every key group: bit-identical to rotating it first.
+    q, k, v = (rnd((1, 300, 8, D), i, torch.bfloat16).to(device) for i in range(3))
+    cos, sin = precompute_rope_cache(400, D, dtype=torch.bfloat16, device=device)
+    out = fused_rope_attention(q, k, v, cos_cache=cos, sin_cache=sin, q_offset=40, kv_offset=40,
+                               causal=True)
+    want = flash_attention(rope(q, cos, sin, 40), rope(k, cos, sin, 40), v, causal=True)
+    assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("S,H", [(300, 8), (1000, 16), (777, 12)])
+def test_lse_of_key_groups(device, S, H):
+    # The saved log-sum-exp (base 2) and the keep mask do not depend on the
+    # groups: lse against float64, dropout's forward against the oracle's mask is
+    # covered by the dropout tests at these sizes.
+    D = 128
+    q, k, v = (rnd((1, S, H, D), i, torch.float16).to(device) for i in range(3))
+    o, lse = torch.empty_like(q), torch.empty(1, H, S, device=device)
+    bhs = lambda x: (x.stride(0), x.stride(2), x.stride(1))
+    _native.attn_fwd(q, k, v, o, bhs(q), bhs(k), bhs(v), bhs(o), 1, H, S, S, D, D ** -0.5, True,
+                     lse=lse)
+    s = torch.einsum("bqhd,bkhd->bhqk", q.double().cpu(), k.double().cpu()) * D ** -0.5
+    s.masked_fill_(~torch.ones(S, S, dtype=torch.bool).tril(), -math.inf)
+    want = torch.logsumexp(s, -1) / math.log(2)
+    # scores of products of float16: Q times the scale is rounded to float16 (2^-11 of ~5)
+    assert float((lse.double().cpu() - want).abs().max()) <= 1e-2
