@@ -146,30 +146,6 @@ __device__ __forceinline__ void store_row(uint16_t* row, int g, const f32x16 (&a
     }
 }
 
-// One key's dK (times scale) and dV (times mul_v) as float32 sums of a part of
-// the K/V head's query heads (BwdParams::dkv_part).
-template <int NDB>
-__device__ __forceinline__ void store_part(const BwdParams& p, int bhk, int part, int key, int g,
-                                           const f32x16 (&dk)[NDB], const f32x16 (&dv)[NDB],
-                                           float mul_v) {
-  constexpr int D = 32 * NDB;
-  const int64_t plane = (int64_t)p.B * p.H_kv * p.kv_parts * p.Sk * D;
-  float* row = p.dkv_part + (((int64_t)bhk * p.kv_parts + part) * p.Sk + key) * D + 4 * g;
-#pragma unroll
-  for (int db = 0; db < NDB; ++db)
-#pragma unroll
-    for (int e4 = 0; e4 < 4; ++e4) {
-      f32x4 a, c;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[i] = dk[db][4 * e4 + i] * p.scale;
-        c[i] = dv[db][4 * e4 + i] * mul_v;
-      }
-      *(f32x4*)(row + db * 32 + 8 * e4) = a;
-      *(f32x4*)(row + plane + db * 32 + 8 * e4) = c;
-    }
-}
-
 // dK (blockIdx.y == 0) or dV = the parts' float32 sums added up, rounded once:
 // four dims of one key per thread.
 template <int D, bool BF16>
@@ -1236,54 +1212,30 @@ void fa_bwd_dq_ds_kernel(BwdParams p) {
 // launches against one: (2, 2048, 16, 128) 167 -> 147 us, (1, 1024, 16, 128)
 // 98 -> 64, (4, 1000, 12, 64) 67 -> 44, (1, 300, 8, 128) 46 -> 26.
 // ---------------------------------------------------------------------------
-// The heads go in chunks of chunk_heads (batch, K/V head)s, chunk_wgs
-// workgroups each. Within a chunk, entry i of the order covers the workgroups
-// first[i] .. first[i + 1] - 1: dK/dV of key tile code >> 1 (code & 1; one per
-// K/V head and part) or dQ of query tile code >> 1 (one per query head).
-constexpr int kMaxOrder = 128;
-struct BwdOrder {
-  int n, chunk_heads, chunk_wgs;
-  int first[kMaxOrder + 1];
-  uint16_t code[kMaxOrder];
-};
-
 template <int D, bool BF16, bool DROP, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fa_bwd_joint_kernel(BwdParams p, BwdOrder order) {
   constexpr int kLds = D == 128 ? kFusedLds : kDkdvLds<D>;
   static_assert(kLds >= kDqLds<D>, "dQ stages");
   __shared__ __align__(1024) uint16_t lds[kLds];
-  const int chunk = blockIdx.x / order.chunk_wgs, wg = blockIdx.x - chunk * order.chunk_wgs;
-  int lo = 0, hi = order.n;  // first[lo] <= wg < first[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (order.first[mid] <= wg)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  const int code = order.code[lo], tile = code >> 1;
-  // K/V heads fastest: with a multiple of 8 heads in a chunk every entry starts
-  // on XCD 0, and a K/V head and its query heads stay on XCD head % 8 through
-  // all their tiles.
-  const int i = wg - order.first[lo];
-  const int sub = i / order.chunk_heads;  // part, or query head of the group
-  const int bhk = chunk * order.chunk_heads + (i - sub * order.chunk_heads);
-  if (code & 1) {
+  const BwdWork w = joint_work(order);
+  if (w.kind != kTileDq) {
     if constexpr (D == 128)
-      bwd_dkdv_fused_tiles<BF16, DROP, false, SPLIT>(p, lds, bhk, sub, tile, -1);
+      bwd_dkdv_fused_tiles<BF16, DROP, false, SPLIT>(p, lds, w.bhk, w.sub, w.tile, -1);
     else
-      bwd_dkdv_tile<D, BF16, kBoth, DROP, SPLIT>(p, lds, bhk, sub, tile);
+      bwd_dkdv_tile<D, BF16, kBoth, DROP, SPLIT>(p, lds, w.bhk, w.sub, w.tile);
   } else {
-    bwd_dq_tiles<D, BF16, DROP>(p, lds, bhk * p.kv_group + sub, tile, -1, false);
+    bwd_dq_tiles<D, BF16, DROP>(p, lds, w.bhk * p.kv_group + w.sub, w.tile, -1, false);
   }
 }
 
-// Rows (or keys) the masks of tile `t` of n_own reach among n_other: keys per
-// query tile (left = win_left, right = win_right) or, with the two swapped,
-// queries per key tile.
-int tile_reach(int t, int n_own, int n_other, int left, int right) {
-  const int o0 = t * kBwdOwn, o1 = std::min(o0 + kBwdOwn, n_own) - 1;
+constexpr int kDqDsQB = 2;  // query blocks per wave of fa_bwd_dq_ds_kernel
+
+// Rows (or keys) the masks of tile `t` of `own` rows of n_own reach among
+// n_other: keys per query tile (left = win_left, right = win_right) or, with
+// the two swapped, queries per key tile.
+static int tile_reach(int t, int own, int n_own, int n_other, int left, int right) {
+  const int o0 = t * own, o1 = std::min(o0 + own, n_own) - 1;
   const int lo = left >= 0 ? std::max(0, o0 - left) : 0;
   const int hi = right >= 0 ? std::min(n_other, o1 + right + 1) : n_other;
   return std::max(0, hi - lo);
@@ -1296,25 +1248,30 @@ int tile_reach(int t, int n_own, int n_other, int left, int right) {
 // 298 / 319 us.
 constexpr int kChunkWgs = 128;
 
-// The order of a joint launch: tiles by cost, products per row of the streamed
-// side (dK/dV: 4 for every query head of the part, dQ: 3), largest first.
-// (bwd_joint: the tiles of a head fit an order.)
-void make_order(const BwdParams& p, BwdOrder& order) {
-  const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn, n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn;
+void make_order(const BwdParams& p, int own, bool split, BwdOrder& order) {
+  const int n_qt = (p.Sq + own - 1) / own, n_kt = (p.Sk + own - 1) / own;
   struct Item {
     int64_t cost;
     int code;
   } items[kMaxOrder];
   int n = 0;
-  for (int t = 0; t < n_kt; ++t)
-    items[n++] = {4LL * (p.kv_group / p.kv_parts) *
-                      tile_reach(t, p.Sk, p.Sq, p.win_right, p.win_left),
-                  2 * t + 1};
+  for (int t = 0; t < n_kt; ++t) {
+    const int64_t rows = (int64_t)(p.kv_group / p.kv_parts) *
+                         tile_reach(t, own, p.Sk, p.Sq, p.win_right, p.win_left);
+    if (split) {
+      items[n++] = {3 * rows, 4 * t + kTileDk};
+      items[n++] = {2 * rows, 4 * t + kTileDv};
+    } else {
+      items[n++] = {4 * rows, 4 * t + kTileDkDv};
+    }
+  }
   for (int t = 0; t < n_qt; ++t)
-    items[n++] = {3LL * tile_reach(t, p.Sq, p.Sk, p.win_left, p.win_right), 2 * t};
+    items[n++] = {3LL * tile_reach(t, own, p.Sq, p.Sk, p.win_left, p.win_right),
+                  4 * t + kTileDq};
   std::stable_sort(items, items + n,
                    [](const Item& a, const Item& b) { return a.cost > b.cost; });
-  const int heads = p.B * p.H_kv, per_head = n_kt * p.kv_parts + n_qt * p.kv_group;
+  const int heads = p.B * p.H_kv, kv_tiles = split ? 2 * n_kt : n_kt;
+  const int per_head = kv_tiles * p.kv_parts + n_qt * p.kv_group;
   order.chunk_heads = heads;
   if (heads % 8 == 0)
     for (int m = 1; m < heads / 8; ++m)
@@ -1327,12 +1284,10 @@ void make_order(const BwdParams& p, BwdOrder& order) {
   for (int i = 0; i < n; ++i) {
     order.first[i] = at;
     order.code[i] = (uint16_t)items[i].code;
-    at += order.chunk_heads * ((items[i].code & 1) ? p.kv_parts : p.kv_group);
+    at += order.chunk_heads * ((items[i].code & 3) == kTileDq ? p.kv_group : p.kv_parts);
   }
   order.first[n] = order.chunk_wgs = at;
 }
-
-constexpr int kDqDsQB = 2;  // query blocks per wave of fa_bwd_dq_ds_kernel
 
 // One joint launch (fa_bwd_joint_kernel) instead of a dQ and a dK/dV launch:
 // while the pairs of one side do not fill the 512 slots, that is below 2048
@@ -1352,19 +1307,22 @@ bool bwd_joint(int B, int H, int Sq, int Sk, int D, int win_left) {
 }
 
 // Parts that a K/V head's query heads are cut into (1: none) for the grouped
-// 16-bit backward at D <= 128: the fewest (a divisor of the group) that give
-// the dK/dV side a workgroup for each of the chip's 512 slots. Causal bf16
-// (1, 2048, 32 heads over 8, 128): 409 -> 158 us with 4 parts in the joint
-// launch; (8, 1024, 32 over 4, 128): 488 -> 325 us with 4 parts of paired
-// tiles. The parts' sums are at most 512 + 511 tiles of 128 keys (256 MB).
+// backward at D <= 128: the fewest (a divisor of the group) that give the
+// dK/dV side a workgroup for each of the chip's slots (512; 256 in float32, at
+// one wave per SIMD). Causal bf16 (1, 2048, 32 heads over 8, 128): 409 -> 158
+// us with 4 parts in the joint launch; (8, 1024, 32 over 4, 128): 488 -> 325 us
+// with 4 parts of paired tiles. The parts' sums are at most 512 + 511 tiles of
+// 128 keys (256 MB).
 int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, int dtype) {
   const int group = H / H_kv;
-  if (group == 1 || dtype == MPX_F32 || D > 128) return 1;
-  const int n_kt = (Sk + kBwdOwn - 1) / kBwdOwn;
-  const bool pairs = D == 128 && !bwd_joint(B, H, Sq, Sk, D, win_left);
-  const long wgs = (long)B * H_kv * (pairs ? (n_kt + 1) / 2 : n_kt);
+  if (group == 1 || D > 128) return 1;
+  const bool f32 = dtype == MPX_F32;
+  const bool pairs = !f32 && D == 128 && !bwd_joint(B, H, Sq, Sk, D, win_left);
+  const int own = pairs ? 2 * kBwdOwn
+                        : (f32 && bwd32_joint(B, H, Sq, Sk, D) ? kBwdOwn / 2 : kBwdOwn);
+  const long wgs = (long)B * H_kv * ((Sk + own - 1) / own), slots = f32 ? 256 : 512;
   for (int parts = 1; parts < group; ++parts)
-    if (group % parts == 0 && wgs * parts >= 512) return parts;
+    if (group % parts == 0 && wgs * parts >= slots) return parts;
   return group;
 }
 
@@ -1395,7 +1353,7 @@ hipError_t launch_bwd(const BwdParams& p, hipStream_t st) {
   if constexpr (D <= 128) {
     BwdOrder order;
     if (bwd_joint(p.B, p.H, p.Sq, p.Sk, D, p.win_left)) {
-      make_order(p, order);
+      make_order(p, kBwdOwn, false, order);
       const long rows = (long)p.B * p.H * p.Sq, rpb = 256 / (D / 8);
       const long tiles = (long)p.B * p.H * n_qt + (long)p.B * p.H_kv * p.kv_parts * n_kt;
       hipLaunchKernelGGL((fa_bwd_dvec_kernel<D, BF16>), dim3((rows + rpb - 1) / rpb), dim3(256), 0,

@@ -47,11 +47,11 @@ __global__ __launch_bounds__(256) void fa_bwd32_dvec_kernel(BwdParams p) {
   if (row < rows && l == 0) p.dvec[row] = acc;
 }
 
-// 32 rows of a float32 (rows, D) slice through 256 threads: global ->
+// 32 KG rows of a float32 (rows, D) slice through 256 threads: global ->
 // registers (rows past `rows` re-read the last one) -> LDS rows of stride D + 4.
-template <int D>
+template <int D, int KG = 1>
 struct Stage32 {
-  static constexpr int CPR = D / 4, PER_T = kB32Tile * CPR / 256, RS = D + 4;
+  static constexpr int CPR = D / 4, PER_T = KG * kB32Tile * CPR / 256, RS = D + 4;
   f32x4 r[PER_T];
   __device__ __forceinline__ void load(const float* base, int64_t row_stride, int row0,
                                        int rows) {
@@ -102,22 +102,73 @@ __device__ __forceinline__ constexpr int crow(int e, int g) {
 // per 32-key tile: S^T = K Q^T, dP^T = V dO^T, dS^T = P^T (dP^T - Dvec),
 // dQ^T += K^T dS^T.
 // ---------------------------------------------------------------------------
-template <int D, bool DROP = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void fa_bwd32_dq_kernel(BwdParams p) {
-  constexpr int NQ4 = D / 8, NDB = D / 32, RS = D + 4, TILE = kB32Tile * RS;
-  // D = 256: one LDS stage (two would be 133 KB); the next tile is loaded
-  // after the barrier that ends the current one.
-  constexpr int NSTG = D > 128 ? 1 : 2;
-  __shared__ __align__(16) float lds[NSTG][2][TILE];  // [stage][K, V]
+// D = 256: one LDS stage (two would be 133 KB); the next tile is loaded after
+// the barrier that ends the current one.
+template <int D>
+constexpr int kStages32 = D > 128 ? 1 : 2;
+// LDS floats: [stage][K, V (or Q, dO)][32 KG rows], then lse and Dvec rows per stage.
+template <int D, int KG>
+constexpr int kLds32 = kStages32<D> * 2 * KG * kB32Tile * (D + 4) + 2 * 2 * KG * kB32Tile;
 
-  const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn;
-  const int qt = n_qt - 1 - (int)(blockIdx.x / (p.B * p.H));
-  const int bh = blockIdx.x % (p.B * p.H);
+// KG key groups: the workgroup's waves are 4 / KG row groups of 32 (so it owns
+// 128 / KG rows), and wave group kg takes tile KG t + kg of step t; the groups'
+// sums meet in LDS at the end. One wave's chain of tiles bounds small calls
+// (each tile is 96 products of 64 cycles at D = 64, on one wave per SIMD), and
+// this halves it.
+template <int KG>
+struct Groups32 {
+  int rg, kg;  // row group, key group of the wave
+  __device__ __forceinline__ Groups32(int wave) {
+    constexpr int NR = kBwdWaves / KG;
+    rg = KG == 1 ? wave : wave % NR;
+    kg = KG == 1 ? 0 : wave / NR;
+  }
+};
+
+// Adds the accumulators of wave groups 1 .. KG - 1 to those of group 0 (lds is
+// free: every wave is past its last read).
+template <int KG, int NDB>
+__device__ __forceinline__ void sum_groups32(float* lds, const Groups32<KG>& gr, int lane,
+                                             f32x16 (&acc)[NDB]) {
+  if constexpr (KG > 1) {
+    constexpr int NR = kBwdWaves / KG;
+    f32x4* const at = (f32x4*)lds + lane;
+    __syncthreads();
+    if (gr.kg > 0) {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4)
+          at[(((gr.kg - 1) * NR + gr.rg) * NDB * 4 + 4 * db + e4) * 64] =
+              (f32x4){acc[db][4 * e4], acc[db][4 * e4 + 1], acc[db][4 * e4 + 2],
+                      acc[db][4 * e4 + 3]};
+    }
+    __syncthreads();
+    if (gr.kg == 0) {
+#pragma unroll
+      for (int k = 1; k < KG; ++k)
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int e4 = 0; e4 < 4; ++e4) {
+            const f32x4 x = at[(((k - 1) * NR + gr.rg) * NDB * 4 + 4 * db + e4) * 64];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[db][4 * e4 + i] += x[i];
+          }
+    }
+  }
+}
+
+template <int D, bool DROP, int KG>
+__device__ __forceinline__ void bwd32_dq_tile(const BwdParams& p, float* smem, int bh, int qt) {
+  constexpr int NQ4 = D / 8, NDB = D / 32, RS = D + 4, TILE = KG * kB32Tile * RS;
+  constexpr int NSTG = kStages32<D>, OWN = kBwdOwn / KG;
+  float(*lds)[2][TILE] = (float(*)[2][TILE])smem;  // [stage][K, V]
   const int b = bh / p.H, h = bh % p.H;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 31, g = lane >> 5;
-  const int q0 = qt * kBwdOwn, wq0 = q0 + wave * 32, myq = wq0 + j;
+  const Groups32<KG> gr(wave);
+  const int q0 = qt * OWN, wq0 = q0 + gr.rg * 32, myq = wq0 + j;
   const int qrow = min(myq, p.Sq - 1);
 
   const int kvh = h / p.kv_group;
@@ -136,17 +187,18 @@ void fa_bwd32_dq_kernel(BwdParams p) {
   const int kv_first = p.win_left >= 0 ? myq - p.win_left : -(1 << 30);
   const int kv_last = min(p.win_right >= 0 ? myq + p.win_right : (1 << 30), p.Sk - 1);
 
-  const int q_last = min(q0 + kBwdOwn, p.Sq) - 1;
+  const int q_last = min(q0 + OWN, p.Sq) - 1;
   const int kv_lo = p.win_left >= 0 ? max(0, q0 - p.win_left) : 0;
   const int kv_hi = p.win_right >= 0 ? min(p.Sk, q_last + p.win_right + 1) : p.Sk;
+  // (steps of KG tiles)
   const int t0 = kv_lo / kB32Tile;
-  const int n_t = kv_hi > kv_lo ? (kv_hi - 1) / kB32Tile - t0 + 1 : 0;
+  const int n_t = kv_hi > kv_lo ? ((kv_hi - 1) / kB32Tile - t0) / KG + 1 : 0;
 
   f32x16 dq[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) dq[db] = (f32x16){};
 
-  Stage32<D> kst, vst;
+  Stage32<D, KG> kst, vst;
   if (n_t > 0) {
     kst.load(K, p.k_ss, t0 * kB32Tile, p.Sk);
     vst.load(V, p.v_ss, t0 * kB32Tile, p.Sk);
@@ -156,20 +208,21 @@ void fa_bwd32_dq_kernel(BwdParams p) {
   __syncthreads();
   for (int t = 0; t < n_t; ++t) {
     const int S = NSTG == 1 ? 0 : t & 1;
-    const int kv0 = (t0 + t) * kB32Tile;
+    const int kvs = (t0 + KG * t) * kB32Tile;  // the step's first key
     if (NSTG == 2 && t + 1 < n_t) {
-      kst.load(K, p.k_ss, kv0 + kB32Tile, p.Sk);
-      vst.load(V, p.v_ss, kv0 + kB32Tile, p.Sk);
+      kst.load(K, p.k_ss, kvs + KG * kB32Tile, p.Sk);
+      vst.load(V, p.v_ss, kvs + KG * kB32Tile, p.Sk);
     }
-    const bool skip = wq0 >= p.Sq ||
+    const int kv0 = kvs + gr.kg * kB32Tile;
+    const bool skip = wq0 >= p.Sq || (KG > 1 && kv0 >= p.Sk) ||
                       (p.win_right >= 0 && kv0 > wq0 + 31 + p.win_right) ||
                       (p.win_left >= 0 && kv0 + kB32Tile - 1 < wq0 - p.win_left);
     const bool full = kv0 + kB32Tile <= p.Sk &&
                       (p.win_right < 0 || kv0 + kB32Tile - 1 <= wq0 + p.win_right) &&
                       (p.win_left < 0 || kv0 >= wq0 + 31 - p.win_left);
     if (!skip) {
-      const float* Kt = lds[S][0];
-      const float* Vt = lds[S][1];
+      const float* Kt = lds[S][0] + gr.kg * kB32Tile * RS;
+      const float* Vt = lds[S][1] + gr.kg * kB32Tile * RS;
       f32x16 sb = {}, dpb = {};
       const f32x4* kp = (const f32x4*)(Kt + j * RS) + g;
       const f32x4* vp = (const f32x4*)(Vt + j * RS) + g;
@@ -213,17 +266,28 @@ void fa_bwd32_dq_kernel(BwdParams p) {
     if (t + 1 < n_t) {
       if constexpr (NSTG == 1) {
         __syncthreads();
-        kst.load(K, p.k_ss, kv0 + kB32Tile, p.Sk);
-        vst.load(V, p.v_ss, kv0 + kB32Tile, p.Sk);
+        kst.load(K, p.k_ss, kvs + KG * kB32Tile, p.Sk);
+        vst.load(V, p.v_ss, kvs + KG * kB32Tile, p.Sk);
       }
       kst.store(lds[NSTG == 1 ? 0 : S ^ 1][0]);
       vst.store(lds[NSTG == 1 ? 0 : S ^ 1][1]);
     }
     __syncthreads();
   }
-  if (myq < p.Sq)
+  static_assert(KG == 1 || (KG - 1) * (kBwdWaves / KG) * NDB * 1024 <= kLds32<D, KG>, "LDS");
+  sum_groups32<KG>(smem, gr, lane, dq);
+  if (gr.kg == 0 && myq < p.Sq)
     store_row32<NDB>((float*)p.dq + b * p.dq_sb + h * p.dq_sh + (int64_t)myq * p.dq_ss, g, dq,
                      p.scale);
+}
+
+template <int D, bool DROP = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void fa_bwd32_dq_kernel(BwdParams p) {
+  __shared__ __align__(16) float lds[kLds32<D, 1>];
+  const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn;
+  bwd32_dq_tile<D, DROP, 1>(p, lds, blockIdx.x % (p.B * p.H),
+                            n_qt - 1 - (int)(blockIdx.x / (p.B * p.H)));
 }
 
 // ---------------------------------------------------------------------------
@@ -234,22 +298,19 @@ void fa_bwd32_dq_kernel(BwdParams p) {
 // accumulator sets do not fit one wave's registers, so dK and dV run as two
 // kernels (the dV one recomputes S and needs neither dP nor V).
 // ---------------------------------------------------------------------------
-template <int D, bool WANT_K, bool WANT_V, bool DROP = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void fa_bwd32_dkdv_kernel(BwdParams p) {
-  constexpr int NQ4 = D / 8, NDB = D / 32, RS = D + 4, TILE = kB32Tile * RS;
-  // D = 256: one LDS stage, as in the dQ kernel.
-  constexpr int NSTG = D > 128 ? 1 : 2;
-  __shared__ __align__(16) float lds[NSTG][2][TILE];  // [stage][Q, dO]
-  __shared__ __align__(16) float lse_lds[2][kB32Tile];
-  __shared__ __align__(16) float dvc_lds[2][kB32Tile];
-
-  const int kt = (int)(blockIdx.x / (p.B * p.H_kv));
-  const int bhk = blockIdx.x % (p.B * p.H_kv);
+template <int D, bool WANT_K, bool WANT_V, bool DROP, int KG>
+__device__ __forceinline__ void bwd32_dkdv_tile(const BwdParams& p, float* smem, int bhk, int part,
+                                                int kt) {
+  constexpr int NQ4 = D / 8, NDB = D / 32, RS = D + 4, TILE = KG * kB32Tile * RS;
+  constexpr int NSTG = kStages32<D>, OWN = kBwdOwn / KG, ROWS = KG * kB32Tile;
+  float(*lds)[2][TILE] = (float(*)[2][TILE])smem;  // [stage][Q, dO]
+  float(*lse_lds)[ROWS] = (float(*)[ROWS])(smem + NSTG * 2 * TILE);
+  float(*dvc_lds)[ROWS] = lse_lds + 2;
   const int b = bhk / p.H_kv, hk = bhk % p.H_kv;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 31, g = lane >> 5;
-  const int k0 = kt * kBwdOwn, wk0 = k0 + wave * 32, mykey = wk0 + j;
+  const Groups32<KG> gr(wave);
+  const int k0 = kt * OWN, wk0 = k0 + gr.rg * 32, mykey = wk0 + j;
   const int krow = min(mykey, p.Sk - 1);
   const int q_first = p.win_right >= 0 ? mykey - p.win_right : -(1 << 30);
   const int q_last = p.win_left >= 0 ? mykey + p.win_left : (1 << 30);
@@ -265,12 +326,14 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
   load_row32<D>(K + (int64_t)krow * p.k_ss, g, kf);
   if constexpr (WANT_K) load_row32<D>(V + (int64_t)krow * p.v_ss, g, vf);
 
-  const int k_last = min(k0 + kBwdOwn, p.Sk) - 1;
+  const int k_last = min(k0 + OWN, p.Sk) - 1;
   const int q_lo = p.win_right >= 0 ? max(0, k0 - p.win_right) : 0;
   const int q_hi = p.win_left >= 0 ? min(p.Sq, k_last + p.win_left + 1) : p.Sq;
+  // (steps of KG tiles of one head)
   const int t0 = q_lo / kB32Tile;
-  const int n_t = q_hi > q_lo ? (q_hi - 1) / kB32Tile - t0 + 1 : 0;
-  const int n_steps = n_t * p.kv_group;
+  const int n_t = q_hi > q_lo ? ((q_hi - 1) / kB32Tile - t0) / KG + 1 : 0;
+  const int heads = p.kv_group / p.kv_parts, h0 = hk * p.kv_group + part * heads;
+  const int n_steps = n_t * heads;
 
   f32x16 dk[NDB], dv[NDB];
 #pragma unroll
@@ -279,14 +342,14 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
     dv[db] = (f32x16){};
   }
 
-  Stage32<D> qst, dst;
+  Stage32<D, KG> qst, dst;
   float lse_r = 0.f, dvc_r = 0.f;
   auto load = [&](int u) __attribute__((always_inline)) {
-    const int h = hk * p.kv_group + u / n_t;
-    const int row0 = (t0 + u % n_t) * kB32Tile;
+    const int h = h0 + u / n_t;
+    const int row0 = (t0 + KG * (u % n_t)) * kB32Tile;
     qst.load((const float*)p.q + b * p.q_sb + h * p.q_sh, p.q_ss, row0, p.Sq);
     dst.load((const float*)p.dout + b * p.do_sb + h * p.do_sh, p.do_ss, row0, p.Sq);
-    if (threadIdx.x < kB32Tile) {
+    if (threadIdx.x < ROWS) {
       const int r = row0 + threadIdx.x;
       const int64_t rix = ((int64_t)b * p.H + h) * p.Sq + r;
       lse_r = r < p.Sq ? p.lse[rix] : INFINITY;
@@ -296,7 +359,7 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
   auto store = [&](int S) __attribute__((always_inline)) {
     qst.store(lds[S][0]);
     dst.store(lds[S][1]);
-    if (threadIdx.x < kB32Tile) {
+    if (threadIdx.x < ROWS) {
       lse_lds[S][threadIdx.x] = lse_r;
       dvc_lds[S][threadIdx.x] = dvc_r;
     }
@@ -309,15 +372,17 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
   for (int u = 0; u < n_steps; ++u) {
     const int S = NSTG == 1 ? 0 : u & 1;
     if (NSTG == 2 && u + 1 < n_steps) load(u + 1);
-    const int qr0 = (t0 + u % n_t) * kB32Tile;
-    const bool skip = wk0 >= p.Sk ||
+    const int qr0 = (t0 + KG * (u % n_t) + gr.kg) * kB32Tile;
+    const bool skip = wk0 >= p.Sk || (KG > 1 && qr0 >= p.Sq) ||
                       (p.win_right >= 0 && wk0 > qr0 + kB32Tile - 1 + p.win_right) ||
                       (p.win_left >= 0 && wk0 + 31 < qr0 - p.win_left);
     const bool full = (p.win_right < 0 || wk0 + 31 <= qr0 + p.win_right) &&
                       (p.win_left < 0 || wk0 >= qr0 + kB32Tile - 1 - p.win_left);
     if (!skip) {
-      const float* Qt = lds[S][0];
-      const float* Dt = lds[S][1];
+      const float* Qt = lds[S][0] + gr.kg * kB32Tile * RS;
+      const float* Dt = lds[S][1] + gr.kg * kB32Tile * RS;
+      const float* lsv = lse_lds[S] + gr.kg * kB32Tile;
+      const float* dvv = dvc_lds[S] + gr.kg * kB32Tile;
       f32x16 sb = {}, dpb = {};
       const f32x4* qp = (const f32x4*)(Qt + j * RS) + g;
       const f32x4* dp = (const f32x4*)(Dt + j * RS) + g;
@@ -340,8 +405,8 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
       f32x16 pr, ds;
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
-        const f32x4 lv = *(const f32x4*)(&lse_lds[S][8 * e4 + 4 * g]);
-        const f32x4 dv4 = *(const f32x4*)(&dvc_lds[S][8 * e4 + 4 * g]);
+        const f32x4 lv = *(const f32x4*)(lsv + 8 * e4 + 4 * g);
+        const f32x4 dv4 = *(const f32x4*)(dvv + 8 * e4 + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int e = 4 * e4 + i;
@@ -349,7 +414,7 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
           if constexpr (DROP) {
             // Row qr0 + crow(e, g) of this step's head (u / n_t of the group).
             const u32 rk = drop_row_key(
-                (u32)(((int64_t)b * p.H + hk * p.kv_group + u / n_t) * p.Sq + qr0 + crow(e, g)),
+                (u32)(((int64_t)b * p.H + h0 + u / n_t) * p.Sq + qr0 + crow(e, g)),
                 p.seed0);
             const bool keep = drop_keep(drop_bits(rk, drop_pk), drop_hm, drop_ht);
             if constexpr (WANT_K) ds[e] = pr[e] * ((keep ? dpb[e] * p.drop_scale : 0.f) - dv4[i]);
@@ -377,7 +442,12 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
     }
     __syncthreads();
   }
-  if (mykey < p.Sk) {
+  if constexpr (WANT_K) sum_groups32<KG>(smem, gr, lane, dk);
+  if constexpr (WANT_V) sum_groups32<KG>(smem, gr, lane, dv);
+  if (gr.kg != 0 || mykey >= p.Sk) return;
+  if (p.kv_parts > 1) {
+    store_part<NDB, WANT_K, WANT_V>(p, bhk, part, mykey, g, dk, dv, DROP ? p.drop_scale : 1.f);
+  } else {
     if constexpr (WANT_K)
       store_row32<NDB>((float*)p.dk + b * p.dk_sb + hk * p.dk_sh + (int64_t)mykey * p.dk_ss, g,
                        dk, p.scale);
@@ -387,20 +457,103 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
   }
 }
 
+template <int D, bool WANT_K, bool WANT_V, bool DROP = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void fa_bwd32_dkdv_kernel(BwdParams p) {
+  __shared__ __align__(16) float lds[kLds32<D, 1>];
+  const int heads = p.B * p.H_kv, i = blockIdx.x % (heads * p.kv_parts);
+  bwd32_dkdv_tile<D, WANT_K, WANT_V, DROP, 1>(p, lds, i % heads, i / heads,
+                                              (int)(blockIdx.x / (heads * p.kv_parts)));
+}
+
+// dQ and dK/dV tiles in one launch, one tile of 64 rows or keys per workgroup,
+// the longest first.
+template <int D, bool DROP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void fa_bwd32_joint_kernel(BwdParams p, BwdOrder order) {
+  __shared__ __align__(16) float lds[kLds32<D, 2>];
+  const BwdWork w = joint_work(order);
+  if (w.kind == kTileDq) {
+    bwd32_dq_tile<D, DROP, 2>(p, lds, w.bhk * p.kv_group + w.sub, w.tile);
+  } else if constexpr (D >= 128) {
+    if (w.kind == kTileDk)
+      bwd32_dkdv_tile<D, true, false, DROP, 2>(p, lds, w.bhk, w.sub, w.tile);
+    else
+      bwd32_dkdv_tile<D, false, true, DROP, 2>(p, lds, w.bhk, w.sub, w.tile);
+  } else {
+    bwd32_dkdv_tile<D, true, true, DROP, 2>(p, lds, w.bhk, w.sub, w.tile);
+  }
+}
+
+// dK (blockIdx.y == 0) or dV = the parts' sums added up: four dims of one key
+// per thread.
+template <int D>
+__global__ __launch_bounds__(256) void fa_bwd32_dkv_sum_kernel(BwdParams p) {
+  const int64_t n = (int64_t)p.B * p.H_kv * p.Sk * (D / 4);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int d = (int)(i % (D / 4)) * 4;
+  const int64_t row = i / (D / 4), bhk = row / p.Sk;
+  const int key = (int)(row - bhk * p.Sk), b = (int)(bhk / p.H_kv), hk = (int)(bhk % p.H_kv);
+  const float* src = p.dkv_part + ((bhk * p.kv_parts + (int64_t)p.B * p.H_kv * p.kv_parts *
+                                    blockIdx.y) * p.Sk + key) * D + d;
+  f32x4 sum = *(const f32x4*)src;
+  for (int k = 1; k < p.kv_parts; ++k) sum += *(const f32x4*)(src + (int64_t)k * p.Sk * D);
+  float* dst = blockIdx.y == 0
+                   ? (float*)p.dk + b * p.dk_sb + hk * p.dk_sh + (int64_t)key * p.dk_ss
+                   : (float*)p.dv + b * p.dv_sb + hk * p.dv_sh + (int64_t)key * p.dv_ss;
+  *(f32x4*)(dst + d) = sum;
+}
+
+// Below 2048 tiles of 64 rows over both sides: the two (at D = 128 three)
+// launches of 128-row tiles then leave SIMDs empty or end on a few long waves.
+// Causal backward of (batch, S, heads, D), launches of their own against one:
+// (2, 1024, 12, 64) 266 -> 133 us, (1, 512, 8, 64) 138 -> 46, (2, 1024, 12,
+// 128) 576 -> 277, (1, 2048, 16, 128), 1536 tiles, 1125 -> 654; (2, 2048, 16,
+// 64), 2048 tiles, 565 against 598, (4, 4096, 16, 64) 4237 against 4516 (half
+// the rows a workgroup means twice the streamed tiles).
+bool bwd32_joint(int B, int H, int Sq, int Sk, int D) {
+  constexpr int own = kBwdOwn / 2;
+  const int n_qt = (Sq + own - 1) / own, n_kt = (Sk + own - 1) / own;
+  const int per_kv = D >= 128 ? 2 : 1;  // dK and dV tiles
+  return D <= 128 && n_qt < kMaxOrder && n_kt < kMaxOrder &&
+         n_qt + per_kv * n_kt <= kMaxOrder && (long)B * H * (n_qt + per_kv * n_kt) < 2048;
+}
+
+template <int D>
+void launch_sum32(const BwdParams& p, hipStream_t st) {
+  const long n = (long)p.B * p.H_kv * p.Sk * (D / 4);
+  hipLaunchKernelGGL((fa_bwd32_dkv_sum_kernel<D>), dim3((unsigned)((n + 255) / 256), 2), dim3(256),
+                     0, st, p);
+}
+
 template <int D, bool DROP>
 hipError_t launch_bwd32_d(const BwdParams& p, hipStream_t st) {
   const int64_t rows = (int64_t)p.B * p.H * p.Sq;
   hipLaunchKernelGGL((fa_bwd32_dvec_kernel<D>), dim3((unsigned)((rows * (D / 4) + 255) / 256)),
                      dim3(256), 0, st, p);
+  if constexpr (D <= 128) {
+    if (bwd32_joint(p.B, p.H, p.Sq, p.Sk, D)) {
+      constexpr int own = kBwdOwn / 2;
+      BwdOrder order;
+      make_order(p, own, D >= 128, order);
+      const long wgs = (long)(p.B * p.H_kv / order.chunk_heads) * order.chunk_wgs;
+      hipLaunchKernelGGL((fa_bwd32_joint_kernel<D, DROP>), dim3((unsigned)wgs), dim3(256), 0, st, p,
+                         order);
+      if (p.kv_parts > 1) launch_sum32<D>(p, st);
+      return hipGetLastError();
+    }
+  }
   const int n_qt = (p.Sq + kBwdOwn - 1) / kBwdOwn, n_kt = (p.Sk + kBwdOwn - 1) / kBwdOwn;
   hipLaunchKernelGGL((fa_bwd32_dq_kernel<D, DROP>), dim3(p.B * p.H * n_qt), dim3(256), 0, st, p);
-  const dim3 grid_kv(p.B * p.H_kv * n_kt);
+  const dim3 grid_kv(p.B * p.H_kv * p.kv_parts * n_kt);
   if constexpr (D >= 128) {
     hipLaunchKernelGGL((fa_bwd32_dkdv_kernel<D, true, false, DROP>), grid_kv, dim3(256), 0, st, p);
     hipLaunchKernelGGL((fa_bwd32_dkdv_kernel<D, false, true, DROP>), grid_kv, dim3(256), 0, st, p);
   } else {
     hipLaunchKernelGGL((fa_bwd32_dkdv_kernel<D, true, true, DROP>), grid_kv, dim3(256), 0, st, p);
   }
+  if (p.kv_parts > 1) launch_sum32<D>(p, st);
   return hipGetLastError();
 }
 

@@ -3,9 +3,9 @@ of the grouped backward that cuts a K/V head's query heads into parts, at the
 sizes where their launch rules and tile orders change: gradients against a
 float64 evaluation of the closed form, itself pinned to the oracle on the CPU.
 
-Tolerance: normwise ||g - ref|| / ||ref||, 2e-3 (float16) and 1.5e-2 (bfloat16),
-the bars of test_gpu_attention_bwd.py (a few units of the rounding of P, dS and
-the result to dtype).
+Tolerance: normwise ||g - ref|| / ||ref||, 2e-3 (float16), 1.5e-2 (bfloat16)
+and 2e-5 (float32), the bars of test_gpu_attention_bwd.py (a few units of the
+rounding of P, dS and the result to dtype; float32 sums).
 """
 
 import math
@@ -18,7 +18,7 @@ from mlx_primitives import _native
 from mlx_primitives.attention import _launch, flash_attention, sliding_window_attention
 from oracle import attention_grad as oag
 
-NREL = {torch.float16: 2e-3, torch.bfloat16: 1.5e-2}
+NREL = {torch.float16: 2e-3, torch.bfloat16: 1.5e-2, torch.float32: 2e-5}
 
 
 def rnd(shape, seed, dtype):
@@ -111,6 +111,30 @@ def test_joint_backward(device, dtype, case):
         assert err <= NREL[dtype] * float(w.norm()) + 1e-2 * (Sk == 1), (name, err)
 
 
+CASES32 = [  # float32: tiles of 64 rows, two key groups of 32
+    (1, 1, 1, 1, 1, 64, True, None),
+    (1, 3, 3, 31, 33, 64, False, None),
+    (1, 8, 8, 65, 97, 128, False, None),
+    (2, 4, 4, 97, 65, 64, True, None),
+    (1, 8, 2, 130, 200, 128, False, None),       # 4 parts
+    (1, 6, 2, 257, 257, 64, True, None),         # group of 3
+    (1, 5, 5, 300, 300, 128, True, 40),
+    (2, 3, 3, 300, 300, 64, False, 33),
+    (1, 1, 1, 64, 8128, 64, False, None),        # 1 + 127 tiles: the longest order
+    (1, 1, 1, 64, 8129, 64, False, None),
+    (1, 1, 1, 128, 4032, 128, False, None),      # 2 + 2 x 63 tiles
+    (1, 4, 1, 64, 6000, 128, False, None),       # too many for an order: parts alone
+    (1, 31, 31, 2112, 2112, 64, True, None),     # 2046 tiles: joint
+    (1, 32, 8, 2048, 2048, 64, True, None),      # 2048: launches of their own, 2 parts
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES32)
+def test_joint_backward_float32(device, case):
+    test_joint_backward(device, torch.float32, case)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,H_kv,S", [(4, 4, 300), (8, 2, 257), (16, 16, 2000)])
 def test_joint_dropout_agrees_with_stored_schedule(device, monkeypatch, H, H_kv, S):
@@ -159,7 +183,9 @@ def test_grouped_workspace_bytes():
     plain = lib.mpx_attn_bwd_workspace_bytes(1, 8, 300)
     assert ws(1, 8, 8, 300, 300, 128, 2, -1) == plain       # no groups
     assert ws(1, 8, 2, 300, 300, 256, 2, -1) == plain       # no parts at head dim 256
-    assert ws(1, 8, 2, 300, 300, 128, 0, -1) == plain       # nor in float32
+    # float32: tiles of 64 keys, parts up to 256 workgroups
+    assert ws(1, 8, 2, 300, 300, 128, 0, -1) == -(-plain // 256) * 256 + 2 * 8 * 300 * 128 * 4
+    assert ws(8, 8, 4, 512, 512, 64, 0, -1) == lib.mpx_attn_bwd_workspace_bytes(8, 8, 512)
     # 4 parts of 2 K/V heads, dK and dV sums in float32
     assert ws(1, 8, 2, 300, 300, 128, 2, -1) == -(-plain // 256) * 256 + 2 * 8 * 300 * 128 * 4
     assert ws(1, 8, 3, 300, 300, 128, 2, -1) == 0
