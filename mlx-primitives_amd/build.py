@@ -23,6 +23,8 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 LIB_DIR = os.path.join(HERE, "mlx_primitives", "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmpx_attn.so")
+HOST_SOURCE = "host.cpp"  # the native host path (a Python extension over torch's C++ API)
+HOST_PATH = os.path.join(LIB_DIR, "_mpx_host.so")
 
 SOURCES = ["abi.hip", "fa_fwd.hip", "fa_fwd_drop.hip", "fa_bwd.hip", "fa_bwd32.hip",
            "paged_decode.hip", "kv_cache.hip", "rope.hip"]
@@ -77,8 +79,25 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(err, file=sys.stderr)
 
 
+def host_command(out: str) -> list[str]:
+    """The host compiler's command for the Python extension (no device code)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return ([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+             "-I" + INCLUDE, "-I" + sysconfig.get_paths()["include"]]
+            + ["-isystem" + d for d in cpp_extension.include_paths()]
+            + [os.path.join(CSRC, HOST_SOURCE), "-o", out, "-L" + torch_lib, "-ltorch_python",
+               "-ltorch_cpu", "-lc10"])
+
+
 def build(verbose: bool = False) -> str:
-    """Compile every source to an object (in parallel), then link the library."""
+    """Compile every source to an object (in parallel), then link the library;
+    beside it, the Python extension."""
     os.makedirs(LIB_DIR, exist_ok=True)
     with tempfile.TemporaryDirectory(prefix="mpx_build.") as tmpdir:
         jobs = []
@@ -87,10 +106,13 @@ def build(verbose: bool = False) -> str:
             cmd = ([hipcc()] + compile_flags() + EXTRA_FLAGS.get(src, [])
                    + ["-c", os.path.join(CSRC, src), "-o", obj])
             jobs.append((cmd, obj))
-        workers = min(len(jobs), max(1, (os.cpu_count() or 1)), 8)
+        host_tmp = os.path.join(tmpdir, "_mpx_host.so")
+        workers = min(len(jobs) + 1, max(1, (os.cpu_count() or 1)), 8)
         with ThreadPoolExecutor(max_workers=workers) as ex:
-            for f in [ex.submit(_run, cmd, verbose) for cmd, _ in jobs]:
+            for f in [ex.submit(_run, cmd, verbose)
+                      for cmd in [host_command(host_tmp)] + [cmd for cmd, _ in jobs]]:
                 f.result()
+        shutil.copyfile(host_tmp, HOST_PATH + ".tmp")
         fd, tmp = tempfile.mkstemp(prefix="libmpx_attn.", suffix=".so.tmp", dir=LIB_DIR)
         os.close(fd)
         try:
@@ -99,6 +121,7 @@ def build(verbose: bool = False) -> str:
         except Exception:
             os.unlink(tmp)
             raise
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
     os.replace(tmp, LIB_PATH)
     return LIB_PATH
 

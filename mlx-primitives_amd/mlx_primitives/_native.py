@@ -13,6 +13,8 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from typing import Optional, Sequence
@@ -30,7 +32,11 @@ MPX_EHIP = -3
 
 DTYPE_CODES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
+# The native host path (csrc/host.cpp), built beside the library.
+_HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "_mpx_host.so")
+
 _lib: Optional[ctypes.CDLL] = None
+_host = None
 _lock = threading.Lock()
 
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -175,8 +181,25 @@ def load() -> ctypes.CDLL:
             ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
             ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
         ]
+        global _host
+        _host = _load_host(lib)
         _lib = lib
         return lib
+
+
+def _load_host(lib: ctypes.CDLL):
+    """The host extension, bound to lib's entries."""
+    if not os.path.exists(_HOST_PATH):
+        raise RuntimeError(
+            f"_mpx_host.so not found at {_HOST_PATH}; build it with "
+            "`python mlx-primitives_amd/build.py`")
+    loader = importlib.machinery.ExtensionFileLoader("_mpx_host", _HOST_PATH)
+    host = importlib.util.module_from_spec(
+        importlib.util.spec_from_file_location("_mpx_host", _HOST_PATH, loader=loader))
+    loader.exec_module(host)
+    host.init({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+               for name in host.entries()})
+    return host
 
 
 def _check(rc: int, what: str) -> None:
@@ -239,6 +262,44 @@ def _stream_ptr(dev: torch.device) -> int:
     if _raw_stream is not None:
         return _raw_stream(dev.index if dev.index is not None else torch.cuda.current_device())
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+def host():
+    """The host extension (loads the library first)."""
+    if _host is None:
+        load()
+    return _host
+
+
+def attn_fwd_new(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bshd: bool, D: int,
+                 scale: float, causal: bool, window_left: int, window_right: int, want_lse: bool,
+                 dropout: Optional[tuple]):
+    """The forward into new tensors through the host extension: o, or (o, lse)
+    with want_lse. None where it leaves the call to the general path (layouts
+    that need a copy or padding, wrapped tensors)."""
+    p, seed = dropout if dropout is not None else (-1.0, 0)
+    r = host().attn_fwd(q, k, v, bshd, D, float(scale), causal, window_left, window_right,
+                        want_lse, p, seed, _stream_ptr(q.device) if q.is_cuda else 0)
+    if r.__class__ is int:
+        _check(r, "mpx_attn_fwd failed")
+    return r
+
+
+def attn_bwd_new(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
+                 dout: torch.Tensor, lse: torch.Tensor, bshd: bool, scale: float, causal: bool,
+                 window_left: int, window_right: int, dropout: Optional[tuple],
+                 stored_ds: Optional[bool]):
+    """attn_bwd into new dq, dk, dv through the host extension; None where the
+    call is left to the general path (also for the stored-dS schedule)."""
+    if stored_ds:
+        return None
+    p, seed = dropout if dropout is not None else (-1.0, 0)
+    r = host().attn_bwd(q, k, v, o, dout, lse, bshd, float(scale), causal, window_left,
+                        window_right, p, seed, stored_ds is None,
+                        _stream_ptr(q.device) if q.is_cuda else 0)
+    if r.__class__ is int:
+        _check(r, "mpx_attn_bwd failed")
+    return r
 
 
 @functools.lru_cache(maxsize=1024)
@@ -408,6 +469,18 @@ def paged_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     _check(rc, "mpx_paged_decode failed")
 
 
+def paged_decode_new(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                     block_tables: torch.Tensor, context_lens: torch.Tensor,
+                     alibi_slopes: Optional[torch.Tensor], scale: float):
+    """paged_decode into a new tensor through the host extension (None: the
+    general path)."""
+    r = host().paged_decode(q, k_pool, v_pool, block_tables, context_lens, alibi_slopes,
+                            float(scale), _stream_ptr(q.device) if q.is_cuda else 0)
+    if r.__class__ is int:
+        _check(r, "mpx_paged_decode failed")
+    return r
+
+
 def paged_prefill(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
                   block_tables: torch.Tensor, context_lens: torch.Tensor,
                   alibi_slopes: Optional[torch.Tensor], o: torch.Tensor,
@@ -463,6 +536,31 @@ def kv_append_rope(k: torch.Tensor, v: torch.Tensor, k_pool: torch.Tensor, v_poo
         dtype_code(k_pool.dtype), cos_cache.data_ptr(), sin_cache.data_ptr(),
         cos_cache.shape[0], dtype_code(cos_cache.dtype), errors.data_ptr(), _stream_ptr(dev))
     _check(rc, "mpx_kv_append_rope failed")
+
+
+def kv_append_clear(k: torch.Tensor, v: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                    block_tables: torch.Tensor, start_pos: torch.Tensor, n_tokens: torch.Tensor,
+                    errors: torch.Tensor, rope: Optional[tuple]) -> bool:
+    """Clear errors and enqueue kv_append (kv_append_rope with rope = (cos,
+    sin)) through the host extension; False: the general path, nothing done."""
+    cos, sin = rope if rope is not None else (None, None)
+    r = host().kv_append(k, v, k_pool, v_pool, block_tables, start_pos, n_tokens, errors, cos, sin,
+                         _stream_ptr(k.device) if k.is_cuda else 0)
+    if r is None:
+        return False
+    _check(r, "mpx_kv_append failed")
+    return True
+
+
+def rope_at_new(x: torch.Tensor, cos_cache: torch.Tensor, sin_cache: torch.Tensor,
+                positions: torch.Tensor, errors: torch.Tensor):
+    """Clear errors and enqueue rope_at into a new tensor through the host
+    extension (None: the general path, nothing done)."""
+    r = host().rope_at(x, cos_cache, sin_cache, positions, errors,
+                       _stream_ptr(x.device) if x.is_cuda else 0)
+    if r.__class__ is int:
+        _check(r, "mpx_rope_at failed")
+    return r
 
 
 def rope_at(x: torch.Tensor, out: torch.Tensor, cos_cache: torch.Tensor, sin_cache: torch.Tensor,

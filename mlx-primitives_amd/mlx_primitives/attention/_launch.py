@@ -72,12 +72,17 @@ class _FlashAttentionFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, layout, scale, causal, window_left, window_right, dropout):
-        B, H, H_kv, Sq, Sk, D = _dims(q, k, layout)
-        o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        lse = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
-        _native.attn_fwd(q, k, v, o, _bhs(q, layout), _bhs(k, layout), _bhs(v, layout),
-                         _bhs(o, layout), B, H, Sq, Sk, D, scale, causal, window_left,
-                         window_right, H_kv=H_kv, lse=lse, dropout=dropout)
+        r = _native.attn_fwd_new(q, k, v, layout == Layout.BSHD, q.shape[-1], scale, causal,
+                                 window_left, window_right, True, dropout)
+        if r is not None:
+            o, lse = r
+        else:
+            B, H, H_kv, Sq, Sk, D = _dims(q, k, layout)
+            o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+            lse = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
+            _native.attn_fwd(q, k, v, o, _bhs(q, layout), _bhs(k, layout), _bhs(v, layout),
+                             _bhs(o, layout), B, H, Sq, Sk, D, scale, causal, window_left,
+                             window_right, H_kv=H_kv, lse=lse, dropout=dropout)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.cfg = (layout, scale, causal, window_left, window_right, dropout)
         return o
@@ -87,6 +92,10 @@ class _FlashAttentionFn(torch.autograd.Function):
     def backward(ctx, dout):
         q, k, v, o, lse = ctx.saved_tensors
         layout, scale, causal, window_left, window_right, dropout = ctx.cfg
+        r = _native.attn_bwd_new(q, k, v, o, dout, lse, layout == Layout.BSHD, scale, causal,
+                                 window_left, window_right, dropout, BWD_STORED_DS)
+        if r is not None:
+            return (*r, None, None, None, None, None, None)
         B, H, H_kv, Sq, Sk, D = _dims(q, k, layout)
         dout = _prepare(dout, D)
         dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
@@ -165,6 +174,11 @@ def run_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: Lay
                                         window_right, dropout)
         # (the dropout kernels take D = 64, 128 or 256)
         dk = 64 if D <= 64 else (128 if D <= 128 else 256)
+    if q_rope is None and dk == D:
+        o = _native.attn_fwd_new(q, k, v, layout == Layout.BSHD, D, scale, causal, window_left,
+                                 window_right, False, dropout)
+        if o is not None:
+            return o
     qk, kk, vk = (_prepare(x, dk) for x in (q, k, v))
     out_shape = list(q.shape)
     out_shape[-1] = dk

@@ -19,6 +19,9 @@ from mlx_primitives import _native
 
 
 def _i32(x, device, n: int, what: str) -> torch.Tensor:
+    if type(x) is int:
+        # filled on the device: a copy from the host would wait for the stream
+        return torch.full((n,), x, dtype=torch.int32, device=device)
     t = torch.as_tensor(x, dtype=torch.int32, device=device).reshape(-1)
     if t.numel() == 1 and n > 1:
         t = t.expand(n)
@@ -132,21 +135,22 @@ def store_kv(
         _native.require_device(cos_cache, sin_cache)
         cos_cache, sin_cache = cos_cache.contiguous(), sin_cache.contiguous()
     if errors is None:
-        errors = torch.zeros(n_err, dtype=torch.int32, device=dev)
-    else:
-        if (errors.dtype != torch.int32 or errors.numel() != n_err or errors.device != dev
-                or not errors.is_contiguous()):
-            raise ValueError(f"errors must be a contiguous int32 tensor of {n_err} entries on "
-                             "the pools' device")
+        errors = torch.empty(n_err, dtype=torch.int32, device=dev)
+    elif (errors.dtype != torch.int32 or errors.numel() != n_err or errors.device != dev
+            or not errors.is_contiguous()):
+        raise ValueError(f"errors must be a contiguous int32 tensor of {n_err} entries on "
+                         "the pools' device")
+    if not _native.kv_append_clear(k, v, k_pool, v_pool, tables, starts, counts, errors,
+                                   None if rope is None else (cos_cache, sin_cache)):
         errors.zero_()
-    if rope is None:
-        _native.kv_append(k, v, k_pool, v_pool, tables, starts, counts, errors, k.stride()[:3],
-                          v.stride()[:3], batch, T, heads, dim, num_blocks, block_size,
-                          tables.shape[1])
-    else:
-        _native.kv_append_rope(k, v, k_pool, v_pool, tables, starts, counts, errors,
-                               k.stride()[:3], v.stride()[:3], batch, T, heads, dim, num_blocks,
-                               block_size, tables.shape[1], cos_cache, sin_cache)
+        if rope is None:
+            _native.kv_append(k, v, k_pool, v_pool, tables, starts, counts, errors,
+                              k.stride()[:3], v.stride()[:3], batch, T, heads, dim, num_blocks,
+                              block_size, tables.shape[1])
+        else:
+            _native.kv_append_rope(k, v, k_pool, v_pool, tables, starts, counts, errors,
+                                   k.stride()[:3], v.stride()[:3], batch, T, heads, dim,
+                                   num_blocks, block_size, tables.shape[1], cos_cache, sin_cache)
     if not check:
         return errors
     _raise_errors(errors.tolist())

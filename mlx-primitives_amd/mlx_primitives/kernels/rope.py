@@ -104,17 +104,20 @@ def rope_at(x: torch.Tensor, cos_cache: torch.Tensor, sin_cache: torch.Tensor,
     vec = 4 if x.dtype == torch.float32 else 8
     if x.stride(-1) != 1 or any(st % vec for st in x.stride()[:3]) or x.data_ptr() % 16:
         x = x.contiguous()
-    if out is None:
-        out = torch.empty((B, S, H, D), dtype=x.dtype, device=x.device)
-    elif out.shape != x.shape or out.dtype != x.dtype or out.stride(-1) != 1:
+    if out is not None and (out.shape != x.shape or out.dtype != x.dtype or out.stride(-1) != 1):
         raise ValueError("out must match x's shape and dtype with a contiguous last dimension")
     if errors is None:
-        errors = torch.zeros(1, dtype=torch.int32, device=dev)
+        errors = torch.empty(1, dtype=torch.int32, device=dev)
+    elif errors.dtype != torch.int32 or errors.numel() != 1 or errors.device != dev:
+        raise ValueError("errors must be an int32 tensor of 1 entry on x's device")
+    made = _native.rope_at_new(x, cos_cache, sin_cache, pos, errors) if out is None else None
+    if made is not None:
+        out = made
     else:
-        if errors.dtype != torch.int32 or errors.numel() != 1 or errors.device != dev:
-            raise ValueError("errors must be an int32 tensor of 1 entry on x's device")
+        if out is None:
+            out = torch.empty((B, S, H, D), dtype=x.dtype, device=x.device)
         errors.zero_()
-    _native.rope_at(x, out, cos_cache, sin_cache, pos, errors)
+        _native.rope_at(x, out, cos_cache, sin_cache, pos, errors)
     if check and int(errors.item()):
         raise ValueError(f"a position in positions .. positions + {S - 1} lies outside the "
                          f"cache's {cos_cache.shape[0]} rows")
