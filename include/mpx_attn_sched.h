@@ -36,8 +36,25 @@ int mpx_attn_bwd_grouped(const void* q, const void* k, const void* v, const void
                          uint64_t seed, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The same call on the stored-dS schedule (mpx_attn_bwd_ds_workspace_bytes),
+ * whatever its size: MPX_EINVAL where the problem has none or the workspace
+ * does not hold it.
+ */
+int mpx_attn_bwd_stored(const void* q, const void* k, const void* v, const void* o,
+                        const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                        const int64_t* q_strides, const int64_t* k_strides,
+                        const int64_t* v_strides, const int64_t* o_strides,
+                        const int64_t* do_strides, const int64_t* dq_strides,
+                        const int64_t* dk_strides, const int64_t* dv_strides,
+                        int B, int H, int H_kv, int Sq, int Sk, int D, float scale, int causal,
+                        int window_left, int window_right, int dtype, float dropout_p,
+                        uint64_t seed, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * 1 when mpx_attn_bwd_dropout runs faster with the stored-dS workspace
- * (mpx_attn_bwd_ds_workspace_bytes) than without it, else 0.
+ * (mpx_attn_bwd_ds_workspace_bytes) than without it, else 0: launches that do
+ * not fill the chip, where it then recomputes whatever the workspace holds, and
+ * grouped heads that run in parts.
  */
 int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk, int D, int dtype,
                               int window_left);

@@ -1443,6 +1443,11 @@ extern "C" int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk,
          bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype) == 1;
 }
 
+// kBySize: stored dS where the workspace holds it (with dropout: and it is the
+// faster schedule); kGrouped: recomputing, in parts where the workspace holds
+// them; kStored: stored dS or an error.
+enum BwdSchedule { kBySize, kGrouped, kStored };
+
 static int attn_bwd_entry(const void* q, const void* k, const void* v, const void* o,
                           const void* dout, const float* lse, void* dq, void* dk, void* dv,
                           const int64_t* q_strides, const int64_t* k_strides,
@@ -1451,7 +1456,7 @@ static int attn_bwd_entry(const void* q, const void* k, const void* v, const voi
                           const int64_t* dk_strides, const int64_t* dv_strides, int B, int H,
                           int H_kv, int Sq, int Sk, int D, float scale, int causal,
                           int window_left, int window_right, int dtype, float dropout_p,
-                          uint64_t seed, bool grouped, void* workspace, size_t workspace_bytes,
+                          uint64_t seed, BwdSchedule schedule, void* workspace, size_t workspace_bytes,
                           void* stream) {
   MPX_CHECK_ARG(dropout_p >= 0.f && dropout_p < 1.f,
                 "mpx_attn_bwd_dropout: dropout_p must be in [0, 1), got %g", (double)dropout_p);
@@ -1524,13 +1529,18 @@ static int attn_bwd_entry(const void* q, const void* k, const void* v, const voi
   // The stored-dS schedule when the workspace holds it.
   const size_t ds_need = mpx_attn_bwd_ds_workspace_bytes(B, H, Sq, Sk, D, dtype, causal,
                                                          window_left, window_right);
-  if (grouped) {
+  MPX_CHECK_ARG(schedule != kStored || (ds_need > 0 && workspace_bytes >= ds_need),
+                "mpx_attn_bwd: the stored-dS schedule needs a workspace of %zu bytes (0: none "
+                "for this problem), %zu given", ds_need, workspace_bytes);
+  if (schedule == kGrouped) {
     if (workspace_bytes >= mpx_attn_bwd_grouped_workspace_bytes(B, H, H_kv, Sq, Sk, D, dtype,
                                                                 window_left)) {
       p.kv_parts = bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype);
       p.dkv_part = (float*)((char*)workspace + dvec_region_bytes(B, H, Sq));
     }
-  } else if (ds_need > 0 && workspace_bytes >= ds_need) {
+  } else if (ds_need > 0 && workspace_bytes >= ds_need &&
+             (schedule == kStored || !drop ||
+              mpx_attn_bwd_ds_preferred(B, H, H_kv, Sq, Sk, D, dtype, window_left))) {
     p.ds = (char*)workspace + dvec_region_bytes(B, H, Sq);
     p.ds_tot = ds_blocks_per_head(Sq, Sk, p.win_left, p.win_right);
   }
@@ -1558,7 +1568,7 @@ extern "C" int mpx_attn_bwd(const void* q, const void* k, const void* v, const v
   clear_error();
   return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
                         o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
-                        Sk, D, scale, causal, window_left, window_right, dtype, 0.f, 0, false,
+                        Sk, D, scale, causal, window_left, window_right, dtype, 0.f, 0, kBySize,
                         workspace, workspace_bytes, stream);
 }
 
@@ -1576,7 +1586,7 @@ extern "C" int mpx_attn_bwd_dropout(const void* q, const void* k, const void* v,
   return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
                         o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
                         Sk, D, scale, causal, window_left, window_right, dtype, dropout_p, seed,
-                        false, workspace, workspace_bytes, stream);
+                        kBySize, workspace, workspace_bytes, stream);
 }
 
 extern "C" int mpx_attn_bwd_grouped(const void* q, const void* k, const void* v, const void* o,
@@ -1593,5 +1603,22 @@ extern "C" int mpx_attn_bwd_grouped(const void* q, const void* k, const void* v,
   return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
                         o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
                         Sk, D, scale, causal, window_left, window_right, dtype, dropout_p, seed,
-                        true, workspace, workspace_bytes, stream);
+                        kGrouped, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mpx_attn_bwd_stored(const void* q, const void* k, const void* v, const void* o,
+                                    const void* dout, const float* lse, void* dq, void* dk,
+                                    void* dv, const int64_t* q_strides,
+                                    const int64_t* k_strides, const int64_t* v_strides,
+                                    const int64_t* o_strides, const int64_t* do_strides,
+                                    const int64_t* dq_strides, const int64_t* dk_strides,
+                                    const int64_t* dv_strides, int B, int H, int H_kv, int Sq,
+                                    int Sk, int D, float scale, int causal, int window_left,
+                                    int window_right, int dtype, float dropout_p, uint64_t seed,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  return attn_bwd_entry(q, k, v, o, dout, lse, dq, dk, dv, q_strides, k_strides, v_strides,
+                        o_strides, do_strides, dq_strides, dk_strides, dv_strides, B, H, H_kv, Sq,
+                        Sk, D, scale, causal, window_left, window_right, dtype, dropout_p, seed,
+                        kStored, workspace, workspace_bytes, stream);
 }

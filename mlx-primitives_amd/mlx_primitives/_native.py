@@ -111,6 +111,8 @@ def load() -> ctypes.CDLL:
         lib.mpx_attn_bwd_grouped.argtypes = lib.mpx_attn_bwd_dropout.argtypes
         lib.mpx_attn_bwd_ds_preferred.restype = ctypes.c_int
         lib.mpx_attn_bwd_ds_preferred.argtypes = [ctypes.c_int] * 8
+        lib.mpx_attn_bwd_stored.restype = ctypes.c_int
+        lib.mpx_attn_bwd_stored.argtypes = lib.mpx_attn_bwd_dropout.argtypes
         lib.mpx_attn_bwd_grouped_workspace_bytes.restype = ctypes.c_size_t
         lib.mpx_attn_bwd_grouped_workspace_bytes.argtypes = [ctypes.c_int] * 8
         lib.mpx_attn_bwd_workspace_bytes.restype = ctypes.c_size_t
@@ -437,9 +439,10 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
             B, H, H_kv, Sq, Sk, D, float(scale), int(causal), int(window_left),
             int(window_right), code)
     tail = (ws.data_ptr(), ws_bytes, _stream_ptr(dev))
-    if grouped:
+    if grouped or stored_ds:
         p, seed = dropout if dropout is not None else (0.0, 0)
-        rc = lib.mpx_attn_bwd_grouped(*args, float(p), int(seed) & (2**64 - 1), *tail)
+        entry = lib.mpx_attn_bwd_grouped if grouped else lib.mpx_attn_bwd_stored
+        rc = entry(*args, float(p), int(seed) & (2**64 - 1), *tail)
     elif dropout is not None:
         p, seed = dropout
         rc = lib.mpx_attn_bwd_dropout(*args, float(p), int(seed) & (2**64 - 1), *tail)
