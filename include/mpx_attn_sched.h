@@ -59,6 +59,29 @@ int mpx_attn_bwd_stored(const void* q, const void* k, const void* v, const void*
 int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk, int D, int dtype,
                               int window_left);
 
+/*
+ * mpx_attn_fwd_rope with K rotated inside the kernel as well: k as given, its
+ * row j at position k_offset + j (the bits of mpx_rope applied to k first, then
+ * mpx_attn_fwd_rope). bfloat16 inputs, 16-bit tables, D = 128; q_offset + Sq and
+ * k_offset + Sk at most n_pos. Workspace: mpx_attn_fwd_workspace_bytes.
+ * Replaces both sides of the reference's fused kernel
+ * (mlx_primitives/kernels/fused_rope_attention.py:766-800).
+ * Available where the launch runs in key groups (calls that leave CUs empty;
+ * elsewhere MPX_EUNSUPPORTED). _preferred: 1 where it is, and is faster than a
+ * pass over K.
+ */
+int mpx_attn_fwd_rope_qk_preferred(int B, int H, int Sq, int Sk, int D, int causal,
+                                   int window_left, int window_right, int dtype, int cache_dtype);
+
+int mpx_attn_fwd_rope_qk(const void* q, const void* k, const void* v, void* o,
+                         const int64_t* q_strides, const int64_t* k_strides,
+                         const int64_t* v_strides, const int64_t* o_strides,
+                         int B, int H, int H_kv, int Sq, int Sk, int D, float scale, int causal,
+                         int window_left, int window_right, int dtype,
+                         const void* cos_cache, const void* sin_cache, int q_offset, int k_offset,
+                         int n_pos, int cache_dtype, void* workspace, size_t workspace_bytes,
+                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

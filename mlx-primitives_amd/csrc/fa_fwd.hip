@@ -3,6 +3,7 @@
 // chunked-cross attention and paged prefill. The kernels and their algorithm
 // are in fa_fwd_kernels.h.
 #include "fa_fwd_kernels.h"
+#include "mpx_attn_sched.h"
 
 namespace mpx {
 
@@ -269,12 +270,27 @@ hipError_t dispatch_fwd(const FwdParams& p, int D, int dtype, int kg, int grid, 
   }
 }
 
+// The ROPEK kernels (bf16, D = 128, dense, 2 or 4 key groups): K rotated in
+// LDS. (With one group the angles do not fit the registers: 71 spilled. In
+// float16 the compiler rounds a rotation's products to float32 first or not,
+// as it picks v_cvt_pk_f16_f32 or v_fma_mixlo_f16, so the bits of a pass of its
+// own would not be kept; bf16 has one conversion.)
+hipError_t dispatch_fwd_ropek(const FwdParams& p, int kg, int grid, hipStream_t st) {
+#define MPX_ROPEK(KG)                                                                        \
+  hipLaunchKernelGGL((fa_fwd16_kernel<128, 128, kNumWaves16, true, false, false, KG, true>), \
+                     dim3(grid), dim3(64 * kNumWaves16), 0, st, p)
+  if (kg == 2) MPX_ROPEK(2);
+  if (kg == 4) MPX_ROPEK(4);
+#undef MPX_ROPEK
+  return hipGetLastError();
+}
+
 // Attention kernel(s) for a prepared FwdParams: the forward launch (with
 // dropout: the dropout kernels), then the split merge when the plan splits
 // the KV range.
 template <bool PAGED>
 int run_fwd(FwdParams& p, const Plan& pl, int D, int dtype, void* workspace, hipStream_t st,
-            bool drop = false) {
+            bool drop = false, bool ropek = false) {
   p.ws_o = pl.splits > 1 ? (float*)workspace : nullptr;
   p.ws_ml = pl.splits > 1 ? (float*)workspace + (size_t)pl.splits * p.B * p.H * p.Sq * D : nullptr;
   p.win_left = pl.win_left; p.win_right = pl.win_right;
@@ -286,7 +302,9 @@ int run_fwd(FwdParams& p, const Plan& pl, int D, int dtype, void* workspace, hip
           ? (long)p.B * p.H * pl.n_slots + (long)kNumXcds * pl.tail_bh * (pl.n_qtiles - pl.n_slots)
           : (long)p.B * p.H * (pl.var_split > 0 ? pl.var_split : (long)pl.n_slots * pl.splits);
   MPX_CHECK_ARG(grid_l < (1L << 31), "attention: problem too large");
-  if (!PAGED && drop)
+  if (!PAGED && ropek)
+    MPX_CHECK_HIP(dispatch_fwd_ropek(p, pl.kg, (int)grid_l, st));
+  else if (!PAGED && drop)
     MPX_CHECK_HIP(dispatch_fwd_drop(p, D, dtype, pl.kg, (int)grid_l, st));
   else
     MPX_CHECK_HIP(dispatch_fwd<PAGED>(p, D, dtype, pl.kg, (int)grid_l, st));
@@ -363,6 +381,8 @@ struct FwdExtras {
   const void* rope_cos = nullptr;
   const void* rope_sin = nullptr;
   int rope_offset = 0, rope_cdt = 0;
+  bool rope_k = false;  // K comes unrotated (the ROPEK kernels)
+  int rope_k_offset = 0;
   bool drop = false;  // dropout on the weights (the fields below)
   uint32_t drop_thresh = 0, seed0 = 0, seed1 = 0;
   float drop_scale = 1.f;
@@ -398,6 +418,10 @@ static int attn_fwd_entry(const void* q, const void* k, const void* v, void* o,
                     "mpx_attn_fwd: strides must be non-negative multiples of %d elements", vec);
 
   const Plan pl = make_plan(B, H, Sq, Sk, D, causal, window_left, window_right, dtype);
+  if (ex.rope_k && pl.kg == 1) {
+    set_error("mpx_attn_fwd_rope_qk: not for a launch of this size (see _preferred)");
+    return MPX_EUNSUPPORTED;
+  }
   if (pl.splits > 1) {
     MPX_CHECK_ARG(workspace != nullptr && workspace_bytes >= pl.ws_bytes,
                   "mpx_attn_fwd: workspace of %zu bytes required, %zu given", pl.ws_bytes,
@@ -431,11 +455,13 @@ static int attn_fwd_entry(const void* q, const void* k, const void* v, void* o,
   p.rope_sin = ex.rope_sin;
   p.rope_offset = ex.rope_offset;
   p.rope_cdt = ex.rope_cdt;
+  p.rope_k_offset = ex.rope_k_offset;
   p.drop_thresh = ex.drop_thresh;
   p.seed0 = ex.seed0;
   p.seed1 = ex.seed1;
   p.drop_scale = ex.drop_scale;
-  return run_fwd<false>(p, pl, D, dtype, workspace, (hipStream_t)stream, ex.drop);
+  return run_fwd<false>(p, pl, D, dtype, workspace, (hipStream_t)stream, ex.drop,
+                        ex.rope_k);
 }
 
 extern "C" int mpx_attn_fwd_lse(const void* q, const void* k, const void* v, void* o,
@@ -512,6 +538,57 @@ extern "C" int mpx_attn_fwd_rope(const void* q, const void* k, const void* v, vo
   ex.rope_sin = sin_cache;
   ex.rope_offset = q_offset;
   ex.rope_cdt = cache_dtype;
+  return attn_fwd_entry(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, H, H_kv, Sq,
+                        Sk, D, scale, causal, window_left, window_right, dtype, workspace,
+                        workspace_bytes, stream, ex);
+}
+
+extern "C" int mpx_attn_fwd_rope_qk_preferred(int B, int H, int Sq, int Sk, int D, int causal,
+                                              int window_left, int window_right, int dtype,
+                                              int cache_dtype) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D != 128 || !MPX_FA_DIRECT ||
+      dtype != MPX_BF16 || (cache_dtype != MPX_F16 && cache_dtype != MPX_BF16))
+    return 0;
+  // K tiles that the q-tiles of a head visit, against those K has: a pass over
+  // K of its own costs about 3 visits' worth of rotations in LDS.
+  const Plan pl = make_plan(B, H, Sq, Sk, D, causal, window_left, window_right, dtype);
+  if (pl.kg == 1) return 0;
+  long visits = 0;
+  for (int t = 0; t < pl.n_qtiles; ++t)
+    visits += qtile_kv_tiles(t, pl.BM, pl.BN, Sq, Sk, pl.win_left, pl.win_right);
+  return visits <= 3L * ((Sk + pl.BN - 1) / pl.BN);
+}
+
+extern "C" int mpx_attn_fwd_rope_qk(const void* q, const void* k, const void* v, void* o,
+                                    const int64_t* q_strides, const int64_t* k_strides,
+                                    const int64_t* v_strides, const int64_t* o_strides, int B,
+                                    int H, int H_kv, int Sq, int Sk, int D, float scale,
+                                    int causal, int window_left, int window_right, int dtype,
+                                    const void* cos_cache, const void* sin_cache, int q_offset,
+                                    int k_offset, int n_pos, int cache_dtype, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (dtype != MPX_BF16 || D != 128 || cache_dtype == MPX_F32) {
+    set_error("mpx_attn_fwd_rope_qk: bfloat16 inputs, 16-bit tables and head_dim 128 only");
+    return MPX_EUNSUPPORTED;
+  }
+  MPX_CHECK_ARG(cache_dtype == MPX_F16 || cache_dtype == MPX_BF16,
+                "mpx_attn_fwd_rope_qk: unknown cache dtype code %d", cache_dtype);
+  MPX_CHECK_ARG(q_offset >= 0 && k_offset >= 0 && (long)q_offset + Sq <= n_pos &&
+                    (long)k_offset + Sk <= n_pos,
+                "mpx_attn_fwd_rope_qk: positions up to %ld exceed the %d-row cos/sin caches",
+                std::max((long)q_offset + Sq, (long)k_offset + Sk) - 1, n_pos);
+  MPX_CHECK_ARG((long)B * H * Sq == 0 || (cos_cache && sin_cache),
+                "mpx_attn_fwd_rope_qk: null cos/sin cache");
+  MPX_CHECK_ARG(aligned16(cos_cache) && aligned16(sin_cache),
+                "mpx_attn_fwd_rope_qk: cos/sin caches must be 16-byte aligned");
+  FwdExtras ex;
+  ex.rope_cos = cos_cache;
+  ex.rope_sin = sin_cache;
+  ex.rope_offset = q_offset;
+  ex.rope_cdt = cache_dtype;
+  ex.rope_k = true;
+  ex.rope_k_offset = k_offset;
   return attn_fwd_entry(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, H, H_kv, Sq,
                         Sk, D, scale, causal, window_left, window_right, dtype, workspace,
                         workspace_bytes, stream, ex);

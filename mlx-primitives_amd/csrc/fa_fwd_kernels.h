@@ -77,6 +77,8 @@ struct FwdParams {
   const void* rope_cos;
   const void* rope_sin;
   int rope_offset, rope_cdt;
+  // ROPEK kernels: K comes unrotated, row j at position rope_k_offset + j.
+  int rope_k_offset;
   // Paged K/V (prefill over a block-table cache; the PAGED kernels only): k
   // and v are the pools (num_blocks, bs, H, D), k_ss / v_ss their token row
   // stride H*D; the rows of batch b come through bt[b, pos / bs].
@@ -903,7 +905,7 @@ __device__ __forceinline__ int swz64(int r) { return (((r >> 1) & 1) << 2) | ((r
 // 64-bit address form (rows without a page from kZeroChunk) instead of 32-bit
 // buffer offsets.
 template <int D, int BN, int NW, bool BF16, int NST, bool PAGED, bool DROP = false,
-          bool BIG = false, int KG = 1>
+          bool BIG = false, int KG = 1, bool ROPEK = false>
 __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const WorkItem wi,
                                                  unsigned char* __restrict__ st0,
                                                  unsigned char* __restrict__ st1,
@@ -1379,6 +1381,58 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
   };
 
   // (key groups: the tile's page masks are made by waves of every group)
+  // ROPEK: the tile's K rows are rotated in place once they have landed, each
+  // (row, 8-dim chunk pair) by one thread, with the RoPE kernel's arithmetic
+  // (rope_pair, one rounding): the bits that a separate pass over K would have
+  // left. The next tile's angles (16-bit tables) are fetched a step ahead, under
+  // the compute, and covered by the step's closing vmcnt(0) (two stages).
+  static_assert(!ROPEK || (D == 128 && NST == 2 && !PAGED && !DROP), "ROPEK layout");
+  constexpr int kRot = ROPEK ? BN * (D / 16) / (64 * NW) : 1;  // chunk pairs per thread
+  u32x4 rcos[kRot], rsin[kRot];
+  auto fetch_angles = [&](int kv0) __attribute__((always_inline)) {
+    if constexpr (ROPEK) {
+#pragma unroll
+      for (int i = 0; i < kRot; ++i) {
+        const int r = (tid + 64 * NW * i) / (D / 16), c = tid % (D / 16);
+        // (rows past the last key hold copies of it)
+        const int64_t idx = (int64_t)(p.rope_k_offset + min(kv0 + r, p.Sk - 1)) * (D / 2) + 8 * c;
+        rcos[i] = *(const u32x4*)((const uint16_t*)p.rope_cos + idx);
+        rsin[i] = *(const u32x4*)((const uint16_t*)p.rope_sin + idx);
+      }
+    }
+  };
+  auto rotate_tile = [&](unsigned char* Kt) __attribute__((always_inline)) {
+    if constexpr (ROPEK) {
+      static_assert(64 * NW % (D / 16) == 0, "a thread keeps its chunk");
+      const bool bf = p.rope_cdt == MPX_BF16;
+      auto ang = [&](u32 w, bool hi) __attribute__((always_inline)) {
+        const uint16_t x = (uint16_t)(hi ? w >> 16 : w & 0xffffu);
+        return bf ? h2f<true>(x) : h2f<false>(x);
+      };
+#pragma unroll
+      for (int i = 0; i < kRot; ++i) {
+        const int r = (tid + 64 * NW * i) / (D / 16), c = tid % (D / 16);
+        u32x4* const lo_p = (u32x4*)(Kt + r * ROWB + (c ^ (r & 15)) * 16);
+        u32x4* const hi_p = (u32x4*)(Kt + r * ROWB + ((c + D / 16) ^ (r & 15)) * 16);
+        u32x4 lo = *lo_p, hi = *hi_p;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          float y1a, y2a, y1b, y2b;
+          rope_pair(h2f<BF16>((uint16_t)(lo[w] & 0xffffu)), h2f<BF16>((uint16_t)(hi[w] & 0xffffu)),
+                    ang(rcos[i][w], false), ang(rsin[i][w], false), y1a, y2a);
+          rope_pair(h2f<BF16>((uint16_t)(lo[w] >> 16)), h2f<BF16>((uint16_t)(hi[w] >> 16)),
+                    ang(rcos[i][w], true), ang(rsin[i][w], true), y1b, y2b);
+          lo[w] = pack2<BF16>(y1a, y1b);
+          hi[w] = pack2<BF16>(y2a, y2b);
+        }
+        *lo_p = lo;
+        *hi_p = hi;
+      }
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's rows are written
+      stage_barrier();
+    }
+  };
+
   auto compute_tile = [&](const unsigned char* Kt, int kvt) __attribute__((always_inline)) {
     bool skip, full;
     const int kv0 = kvt + kg * BNW;
@@ -1441,6 +1495,7 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
     if (n_tiles > 0) fetch_pages(kv_lo + t_begin * BN);
   }
   if (n_tiles > 0) load_tile(kv_lo + t_begin * BN, st0);
+  if (n_tiles > 0) fetch_angles(kv_lo + t_begin * BN);
   if constexpr (kChecked) tile_ok = tile_ok_next;
   if constexpr (kScalarPages) {
     if (n_tiles > 1) fetch_pages(kv_lo + (t_begin + 1) * BN);
@@ -1459,6 +1514,8 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
     if constexpr (kScalarPages) {
       if (i + NST < n_tiles) fetch_pages(kv0 + NST * BN);
     }
+    rotate_tile(stage_ptr(Const<S>{}));
+    if (i + 1 < n_tiles) fetch_angles(kv0 + BN);
     compute_tile(stage_ptr(Const<S>{}), kv0);
     if constexpr (kChecked) tile_ok = tile_ok_next;
     // Tile i+1 must have landed before the barrier that hands it to every
@@ -1613,7 +1670,8 @@ __device__ __forceinline__ void fa16_rows_direct(const FwdParams& pin, const Wor
   }
 }
 
-template <int D, int BN, int NW, bool BF16, bool PAGED, bool BIG = false, int KG = 1>
+template <int D, int BN, int NW, bool BF16, bool PAGED, bool BIG = false, int KG = 1,
+          bool ROPEK = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MPX_FA_WAVES_PER_EU)))
 void fa_fwd16_kernel(FwdParams p) {
   // Stay within 128 KB of LDS per workgroup (a 136 KB configuration gave wrong
@@ -1647,7 +1705,7 @@ void fa_fwd16_kernel(FwdParams p) {
 #pragma nounroll
   for (int item = 0; item < n_items; ++item) {
     if constexpr (kDirect)
-      fa16_rows_direct<D, BN, NW, BF16, kDStages, PAGED, false, BIG, KG>(
+      fa16_rows_direct<D, BN, NW, BF16, kDStages, PAGED, false, BIG, KG, ROPEK>(
           p, slot_item(p, ws, item), dst0, dst1, dst2, dst3, pages);
     else
       fa16_rows<D, BN, NW, BF16, PAGED, false, BIG>(p, slot_item(p, ws, item), smem, pages);

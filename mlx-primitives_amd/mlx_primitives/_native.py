@@ -93,6 +93,13 @@ def load() -> ctypes.CDLL:
                                  ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                  ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
                                  ctypes.c_void_p]
+        lib.mpx_attn_fwd_rope_qk.restype = ctypes.c_int
+        lib.mpx_attn_fwd_rope_qk.argtypes = [ctypes.c_void_p] * 4 + [_i64p] * 4 + [
+            ctypes.c_int] * 6 + [ctypes.c_float] + [ctypes.c_int] * 4 + [
+            ctypes.c_void_p] * 2 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_size_t,
+                                                         ctypes.c_void_p]
+        lib.mpx_attn_fwd_rope_qk_preferred.restype = ctypes.c_int
+        lib.mpx_attn_fwd_rope_qk_preferred.argtypes = [ctypes.c_int] * 10
         lib.mpx_attn_bwd.restype = ctypes.c_int
         lib.mpx_attn_bwd.argtypes = [ctypes.c_void_p] * 9 + [_i64p] * 8 + [
             ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
@@ -326,7 +333,8 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     K/V carry H_kv heads, default H; lse: optional contiguous (B, H, Sq) float32
     that receives each row's base-2 log-sum-exp for the backward). With
     q_rope = (cos_cache, sin_cache, q_offset) the kernel rotates Q on load
-    (mpx_attn_fwd_rope); with dropout = (dropout_p, seed) the weights are
+    (mpx_attn_fwd_rope), with (cos_cache, sin_cache, q_offset, k_offset) K too
+    (mpx_attn_fwd_rope_qk); with dropout = (dropout_p, seed) the weights are
     dropped by the counter-based keep mask (mpx_attn_fwd_dropout)."""
     lib = load()
     dev = require_device(q, k, v, o)
@@ -334,17 +342,18 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     if q_rope is not None:
         if lse is not None:
             raise ValueError("q_rope and lse cannot be combined")
-        cos, sin, q_offset = q_rope
+        cos, sin, *offsets = q_rope
         require_device(q, cos, sin)
         ws_bytes = _fwd_workspace_bytes(B, H, Sq, Sk, D, int(causal), int(window_left),
                                         int(window_right), code)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        rc = lib.mpx_attn_fwd_rope(
+        entry = lib.mpx_attn_fwd_rope if len(offsets) == 1 else lib.mpx_attn_fwd_rope_qk
+        rc = entry(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
             _strides(q_strides), _strides(k_strides), _strides(v_strides), _strides(o_strides),
             B, H, H if H_kv is None else H_kv, Sq, Sk, D, float(scale), int(causal),
             int(window_left), int(window_right), code, cos.data_ptr(), sin.data_ptr(),
-            int(q_offset), int(cos.shape[0]), dtype_code(cos.dtype),
+            *(int(x) for x in offsets), int(cos.shape[0]), dtype_code(cos.dtype),
             ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(dev))
         _check(rc, "mpx_attn_fwd_rope failed")
         return
@@ -367,6 +376,16 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     else:
         rc = lib.mpx_attn_fwd_lse(*args, *tail)
     _check(rc, "mpx_attn_fwd failed")
+
+
+@functools.lru_cache(maxsize=1024)
+def rope_qk_preferred(B: int, H: int, Sq: int, Sk: int, D: int, causal: bool, window_left: int,
+                      window_right: int, dtype: torch.dtype, cache_dtype: torch.dtype) -> bool:
+    """Whether K is better rotated inside the attention kernel than by a pass of
+    its own (a pure function of its arguments)."""
+    return bool(load().mpx_attn_fwd_rope_qk_preferred(
+        B, H, Sq, Sk, D, int(causal), window_left, window_right, dtype_code(dtype),
+        dtype_code(cache_dtype)))
 
 
 _DS_LIMIT: dict = {}

@@ -144,7 +144,8 @@ def run_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: Lay
     """Attention forward on the GPU kernel; returns a new tensor shaped like q.
     When autograd tracks q, k or v, the result is differentiable through the
     gfx950 backward kernels. q_rope = (cos_cache, sin_cache, q_offset) rotates Q
-    inside the kernel (16-bit, D in 32/64/128, no gradients). dropout_p > 0
+    inside the kernel (16-bit, D in 32/64/128, no gradients), with a fourth entry
+    k_offset K too (_native.rope_qk_preferred). dropout_p > 0
     drops attention weights by the kernels' counter-based keep mask, seeded by
     dropout_seed_value or else a fresh dropout_seed(); the backward regenerates
     the same mask."""

@@ -3,7 +3,8 @@
 Drop-in for mlx_primitives/kernels/fused_rope_attention.py:
 ``fast_fused_rope_attention`` (637-733), ``fused_rope_attention`` (939-985)
 and ``FusedRoPEFlashAttention`` (988-1109). K is rotated by the gfx950 RoPE
-kernel into a scratch tensor; for 16-bit inputs with head_dim 32, 64 or 128
+kernel into a scratch tensor, or (bfloat16, head_dim 128, few queries per key)
+by the flash kernel in LDS; for 16-bit inputs with head_dim 32, 64 or 128
 the flash kernel rotates Q itself as it loads it (as the reference's fused
 kernel does, fused_rope_attention.py:766-800), otherwise Q goes through the
 RoPE kernel too. Tensors are (batch, seq, heads, head_dim).
@@ -51,6 +52,25 @@ def _check_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
         raise ValueError(f"Q/K/V dtype mismatch: {q.dtype}, {k.dtype}, {v.dtype}")
 
 
+def _k_in_kernel(q, k, cos_cache, sin_cache, q_offset: int, kv_offset: int, mask: dict) -> bool:
+    """Whether K is rotated by the attention kernel: few q-tiles per K tile
+    (_native.rope_qk_preferred), tables as the kernel reads them, and nothing
+    that the general path would refuse or copy."""
+    half = q.shape[-1] // 2
+    for c in (cos_cache, sin_cache):
+        if (c.ndim != 2 or c.shape[1] != half or c.dtype != cos_cache.dtype
+                or c.dtype not in (torch.float16, torch.bfloat16) or c.device != q.device
+                or not c.is_contiguous() or c.data_ptr() % 16):
+            return False
+    if (cos_cache.shape != sin_cache.shape or cos_cache.requires_grad or sin_cache.requires_grad
+            or not q.is_cuda or q.dtype != torch.bfloat16 or q.numel() == 0 or k.numel() == 0
+            or max(q.shape[1] + q_offset, k.shape[1] + kv_offset) > cos_cache.shape[0]):
+        return False
+    return _native.rope_qk_preferred(
+        q.shape[0], q.shape[2], q.shape[1], k.shape[1], q.shape[3], mask["causal"], -1,
+        mask.get("window_right", -1), q.dtype, cos_cache.dtype)
+
+
 def _rope_attention(q, k, v, scale, cos_cache, sin_cache, rope_base, q_offset, kv_offset,
                     causal, position_rule: bool) -> torch.Tensor:
     """softmax(scale * rope(Q) rope(K)^T + mask) V on the gfx950 kernels, with
@@ -82,10 +102,14 @@ def _rope_attention(q, k, v, scale, cos_cache, sin_cache, rope_base, q_offset, k
                                           rope_base, q_offset + n0, kv_offset, causal,
                                           position_rule)
         return out
-    k_rot = rope(k, cos_cache, sin_cache, kv_offset)
     # kv_offset + j <= q_offset + i  <=>  j <= i + shift
     mask = (dict(causal=False) if not causal else
             dict(causal=True) if shift == 0 else dict(causal=False, window_right=shift))
+    if _k_in_kernel(q, k, cos_cache, sin_cache, q_offset, kv_offset, mask):
+        # K as well, tile by tile in LDS: the same bits without a pass over K.
+        return run_attention(q, k, v, Layout.BSHD, scale,
+                             q_rope=(cos_cache, sin_cache, q_offset, kv_offset), **mask)
+    k_rot = rope(k, cos_cache, sin_cache, kv_offset)
     if q.dtype != torch.float32 and dim in (32, 64, 128):
         # Q is rotated by the attention kernel as it loads it (same arithmetic
         # and rounding as the RoPE kernel); caches go in as given.

@@ -139,6 +139,43 @@ def test_rope_on_load_equals_rope_first(device, D):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Sq,Sk,q_off,kv_off,causal", [
+    (1, 4, 1, 700, 699, 0, True), (2, 32, 65, 4065, 4000, 0, True), (1, 8, 100, 129, 40, 40, False),
+    (1, 3, 33, 128, 97, 2, True), (1, 4, 1, 1, 7, 7, True), (1, 16, 200, 200, 0, 0, True)])
+def test_k_rotated_in_the_kernel_equals_rope_first(device, B, H, Sq, Sk, q_off, kv_off, causal,
+                                                   cache):
+    # The same bits as rotating Q and K first: tiles past the last key, offsets
+    # on either side, splits of the keys, 2 and 4 key groups.
+    D, dtype = 128, torch.bfloat16
+    q = rnd((B, Sq, H, D), 1, dtype).to(device)
+    k, v = (rnd((B, Sk, H, D), s, dtype).to(device) for s in (2, 3))
+    # (the tables end at the last key or query)
+    cos, sin = precompute_rope_cache(max(Sq + q_off, Sk + kv_off), D, dtype=cache, device=device)
+    wr = q_off - kv_off if causal else -1
+    mask = (False, -1, wr) if wr else (True, -1, -1)
+    assert _native.rope_qk_preferred(B, H, Sq, Sk, D, *mask, dtype, cache)
+    out = fused_rope_attention(q, k, v, cos_cache=cos, sin_cache=sin, q_offset=q_off,
+                               kv_offset=kv_off, causal=causal)
+    o = torch.empty_like(q)
+    qr, kr = rope(q, cos, sin, q_off), rope(k, cos, sin, kv_off)
+    bhs = lambda x: (x.stride(0), x.stride(2), x.stride(1))
+    _native.attn_fwd(qr, kr, v, o, bhs(q), bhs(k), bhs(v), bhs(o), B, H, Sq, Sk, D, D ** -0.5,
+                     *mask)
+    assert torch.equal(out, o)
+
+
+def test_k_rotation_left_to_its_own_pass():
+    # full launches, float32 tables, other inputs and head dims
+    pref = _native.rope_qk_preferred
+    b, f = torch.bfloat16, torch.float32
+    assert not pref(2, 32, 65, 4065, 128, False, -1, 4000, torch.float16, b)
+    assert not pref(4, 32, 4096, 4096, 128, True, -1, -1, b, b)
+    assert not pref(2, 32, 65, 4065, 128, False, -1, 4000, b, f)
+    assert not pref(2, 32, 65, 4065, 64, False, -1, 4000, b, b)
+    assert not pref(2, 32, 65, 4065, 128, False, -1, 4000, f, b)
+
+
 @pytest.mark.parametrize("S,H", [(300, 8), (1000, 16), (777, 12)])
 def test_lse_of_key_groups(device, S, H):
     # The saved log-sum-exp (base 2) and the keep mask do not depend on the
