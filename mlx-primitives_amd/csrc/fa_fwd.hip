@@ -34,6 +34,7 @@ struct Plan {
   int kg;  // key groups of a workgroup's waves (make_plan)
   int BM, BN, n_qtiles, splits, tiles_per_split, win_left, win_right;
   int n_slots, paired, win_first;
+  int snake;    // float32 with two key groups: two workgroups per CU, balanced
   int tail_bh;  // paired: (batch, head)s per XCD run as single q-tiles at the end
   int var_split;  // splits per (batch, head) when each q-tile has its own count, else 0
   size_t ws_bytes;
@@ -59,9 +60,10 @@ int tile_n(int D, int dtype, bool paged = false, int bs_log2 = -1, bool alibi = 
 
 Plan plan_for(int kg, int B, int H, int Sq, int Sk, int D, int causal, int window_left,
               int window_right, int dtype, int max_tiles_per_split, bool paged, int bs_log2,
-              bool alibi) {
+              bool alibi, bool may_split = true) {
   Plan pl;
   pl.kg = kg;
+  pl.snake = 0;
   pl.BM = 32 * (dtype == MPX_F32 ? kNumWaves32 : (D > 128 ? kNumWavesWide : kNumWaves16)) / kg;
   pl.BN = tile_n(D, dtype, paged, bs_log2, alibi);
   pl.win_left = window_left < 0 ? -1 : window_left;
@@ -75,7 +77,7 @@ Plan plan_for(int kg, int B, int H, int Sq, int Sk, int D, int causal, int windo
   const long base = (long)B * H * pl.n_qtiles;
   int splits = 1;
   const long target = target_workgroups(D, dtype);
-  if (base > 0 && base < target && max_tiles >= 8) {
+  if (may_split && base > 0 && base < target && max_tiles >= 8) {
     splits = (int)std::min<long>((target + base - 1) / base, max_tiles / 4);
     splits = std::max(splits, 1);
   }
@@ -169,6 +171,33 @@ double plan_time(const Plan& pl, long bh, int Sq, int Sk, int D) {
   return steps * step + items * wgs / cus;
 }
 
+// The same for the float32 kernel at D <= 64 (64-key tiles, two workgroups per
+// CU): the longest item's chain of tiles or the chip's share of them all,
+// whichever takes longer. A 64-key tile of a wave at D = 64 is 128 products of
+// 64 cycles, 3.9 us, and half of it with two key groups; a CU kept busy takes
+// 5.3 and 3.3 us per tile of a workgroup, and about 8 us for each round of
+// items. Causal forward of (batch, S, heads, 64) without and with two groups:
+// (2, 1024, 12) 58 / 54 us (the first splits the keys), (1, 2048, 16) 154 / 94,
+// (2, 2048, 16) 282 / 216, (2, 700, 16) 66 / 37, window 300 (1, 2000, 8) 44 /
+// 23; (8, 512, 16) 80 / 86, (4, 2048, 16) 419 and more.
+double plan_time32(const Plan& pl, long bh, int Sq, int Sk, int D) {
+  const double chain = (pl.kg == 2 ? 2.15 : 3.9) * D / 64, busy = (pl.kg == 2 ? 3.3 : 5.3) * D / 64;
+  double longest = 0, total = 0;
+  for (int t = 0; t < pl.n_qtiles; ++t) {
+    const int n = qtile_kv_tiles(t, pl.BM, pl.BN, Sq, Sk, pl.win_left, pl.win_right);
+    total += n;
+    longest = std::max<double>(longest, std::min(n, pl.splits > 1 ? pl.tiles_per_split : n));
+  }
+  const double wgs = (double)bh * pl.n_qtiles;
+  // (more than one workgroup per CU in the order of the heads: long ones meet)
+  if (pl.splits == 1 && !pl.snake && wgs > kNumCUs) longest *= 2;
+  const double share = total * bh / kNumCUs * busy;
+  if (pl.splits > 1) return std::max(longest * chain, 1.05 * share) + 20.0;
+  // (snake: every CU has at most the longest item and a shortest one)
+  if (pl.snake) return (longest + 1) * 2.65 * D / 64 + 8.0;
+  return std::max(longest * chain, share) + 8.0 * std::ceil(wgs / (2 * kNumCUs));
+}
+
 // The plan of a call. Launches of the 16-bit kernels at D = 64 and 128 that
 // leave CUs empty (one workgroup per CU) may cut the waves of a workgroup into
 // 2 or 4 key groups: q-tiles of 128 or 64 rows, so 2 or 4 times the
@@ -188,6 +217,22 @@ Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
   };
   Plan best = plan(1);
   const long bh = (long)B * H;
+  if (dtype == MPX_F32 && D <= 64 && !paged) {
+    double t = plan_time32(best, bh, Sq, Sk, D);
+    for (bool split : {true, false}) {
+      Plan pl = plan_for(2, B, H, Sq, Sk, D, causal, window_left, window_right, dtype,
+                         max_tiles_per_split, paged, bs_log2, alibi, split);
+      const long per_xcd = bh / kNumXcds * pl.n_qtiles;
+      pl.snake = pl.splits == 1 && pl.win_left < 0 && pl.win_right >= 0 && bh % kNumXcds == 0 &&
+                 per_xcd > kNumCUs / kNumXcds && per_xcd <= 2 * kNumCUs / kNumXcds;
+      const double t2 = plan_time32(pl, bh, Sq, Sk, D);
+      if (t2 < 0.97 * t) {
+        best = pl;
+        t = t2;
+      }
+    }
+    return best;
+  }
   if (dtype == MPX_F32 || (D != 64 && D != 128) || !MPX_FA_DIRECT ||
       bh * best.n_qtiles > 2 * kNumCUs)
     return best;
@@ -210,6 +255,13 @@ hipError_t launch_fwd(const FwdParams& p, int kg, int grid, hipStream_t stream) 
   hipLaunchKernelGGL((fa_fwd16_kernel<D, BN, kNumWaves16, BF16, PAGED, BIG, KG>), dim3(grid), \
                      dim3(64 * kNumWaves16), 0, stream, p)
   if constexpr (F32) {
+    if constexpr (BN == 64 && !PAGED) {
+      if (kg == 2) {
+        hipLaunchKernelGGL((fa_fwd32_kernel<D, BN, kNumWaves32, false, false, 2>), dim3(grid),
+                           dim3(64 * kNumWaves32), 0, stream, p);
+        return hipGetLastError();
+      }
+    }
     hipLaunchKernelGGL((fa_fwd32_kernel<D, BN, kNumWaves32, PAGED>), dim3(grid),
                        dim3(64 * kNumWaves32), 0, stream, p);
   } else if constexpr (D >= 64) {
@@ -295,7 +347,7 @@ int run_fwd(FwdParams& p, const Plan& pl, int D, int dtype, void* workspace, hip
   p.ws_ml = pl.splits > 1 ? (float*)workspace + (size_t)pl.splits * p.B * p.H * p.Sq * D : nullptr;
   p.win_left = pl.win_left; p.win_right = pl.win_right;
   p.n_qtiles = pl.n_qtiles; p.num_splits = pl.splits; p.tiles_per_split = pl.tiles_per_split;
-  p.n_slots = pl.n_slots; p.paired = pl.paired; p.tail_bh = pl.tail_bh;
+  p.n_slots = pl.n_slots; p.paired = pl.paired; p.tail_bh = pl.tail_bh; p.snake = pl.snake;
   p.var_split = pl.var_split; p.bm = pl.BM; p.bn = pl.BN; p.win_first = pl.win_first;
   const long grid_l =
       pl.tail_bh > 0
@@ -371,7 +423,12 @@ using namespace mpx;
 extern "C" size_t mpx_attn_fwd_workspace_bytes(int B, int H, int Sq, int Sk, int D, int causal,
                                                int window_left, int window_right, int dtype) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D <= 0) return 0;
-  return make_plan(B, H, Sq, Sk, D, causal, window_left, window_right, dtype).ws_bytes;
+  // (at least what the launch without key groups takes)
+  return std::max(make_plan(B, H, Sq, Sk, D, causal, window_left, window_right, dtype).ws_bytes,
+                  dtype != MPX_F32 ? 0
+                                   : plan_for(1, B, H, Sq, Sk, D, causal, window_left,
+                                              window_right, dtype, 1 << 30, false, -1, false)
+                                         .ws_bytes);
 }
 
 namespace {

@@ -31,7 +31,10 @@ hipError_t dispatch_fwd_drop(const FwdParams& p, int D, int dtype, int kg, int g
     return hipGetLastError();
   }
   if (dtype == MPX_F32) {
-    if (D == 64)
+    if (D == 64 && kg == 2)
+      hipLaunchKernelGGL((fa_fwd32_kernel<64, 64, kNumWaves32, false, true, 2>), dim3(grid),
+                         dim3(64 * kNumWaves32), 0, st, p);
+    else if (D == 64)
       hipLaunchKernelGGL((fa_fwd32_kernel<64, 64, kNumWaves32, false, true>), dim3(grid),
                          dim3(64 * kNumWaves32), 0, st, p);
     else

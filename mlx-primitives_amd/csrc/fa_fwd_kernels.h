@@ -63,6 +63,7 @@ struct FwdParams {
   // Paired launches, > 0: the last tail_bh (batch, head)s of every XCD's slice
   // run their q-tiles one per workgroup, longest first (B * H % 8 == 0).
   int tail_bh;
+  int snake;    // two workgroups per CU: second half in reverse (decode_slot)
   float c;  // |scale| * log2(e)
   int neg;  // scale < 0: Q is negated on load (exact) and |scale| used
   float eps;      // normaliser epsilon: O / (l + eps)
@@ -259,6 +260,20 @@ __device__ __forceinline__ WorkSlot decode_slot(const FwdParams& p) {
       ws.slot = 0;
       ws.single = p.n_qtiles - 1 - r;
     }
+    return ws;
+  }
+  if (p.snake) {
+    // XCD L % 8 takes B * H / 8 heads' q-tiles, longest first over all its
+    // heads for the first workgroup of each of its 32 CUs, then the rest
+    // shortest first: the second workgroup of a CU is short where its first is
+    // long.
+    const int x = L & 7, idx = L >> 3, hpx = (p.B * p.H) >> 3;
+    const int k = idx < 32 ? idx : hpx * p.n_qtiles - 1 - (idx - 32), r = k / hpx;
+    WorkSlot ws;
+    ws.single = -1;
+    ws.split = 0;
+    ws.slot = r;
+    ws.bh = x * hpx + (k - r * hpx);
     return ws;
   }
   const int w = (N & 7) == 0 ? (L & 7) * (N >> 3) + (L >> 3) : L;
@@ -1775,17 +1790,19 @@ void fa_fwd16_wide_kernel(FwdParams p) {
 // of lane (j, g) holds key 32*nb + 8*(e/4) + 4*g + e%4. PV step (nb, e) has
 // k = g <-> that key, so P^T needs no repacking and V stays row-major in LDS.
 // ---------------------------------------------------------------------------
-template <int D, int BN, int NW, bool PAGED, bool DROP = false>
+// KG key groups as in the 16-bit kernels: the waves are NW / KG row groups, each
+// wave takes BN / KG keys of every tile, and group 0 adds the groups up.
+template <int D, int BN, int NW, bool PAGED, bool DROP = false, int KG = 1>
 __global__ __launch_bounds__(64 * NW) void fa_fwd32_kernel(FwdParams pin) {
-  constexpr int BM = 32 * NW, NT = 64 * NW;
+  constexpr int NR = NW / KG, BM = 32 * NR, NT = 64 * NW, BNW = BN / KG;
   constexpr int KS = D + 4;  // conflict-free 16-byte reads along rows
   constexpr int VS = D + 8;  // rows kv and kv+4 land on opposite bank halves
   constexpr int K_ELEMS = BN * KS, V_ELEMS = BN * VS, STAGE = K_ELEMS + V_ELEMS;
-  constexpr int NB = BN / 32, NDB = D / 32, NQ4 = D / 8;
+  constexpr int NB = BNW / 32, NDB = D / 32, NQ4 = D / 8;
   constexpr int CPR = D / 4;  // 16-byte chunks per row
   constexpr int CHUNKS = BN * CPR;
   constexpr int PER_T = (CHUNKS + NT - 1) / NT;
-  static_assert(D % 32 == 0 && BN % 32 == 0, "tile shape");
+  static_assert(D % 32 == 0 && BNW % 32 == 0 && (KG == 1 || !PAGED), "tile shape");
   // D = 256: one LDS stage (two do not fit 128 KB); the next tile is loaded
   // once every wave has finished reading the current one (not under the
   // compute: its registers would spill).
@@ -1810,7 +1827,8 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd32_kernel(FwdParams pin) {
   const float* __restrict__ Kp = (const float*)p.k + wi.b * p.k_sb + kvh * p.k_sh;
   const float* __restrict__ Vp = (const float*)p.v + wi.b * p.v_sb + kvh * p.v_sh;
 
-  const int wq0 = q0 + wave * 32;
+  const int rg = KG == 1 ? wave : wave % NR, kg = KG == 1 ? 0 : wave / NR;
+  const int wq0 = q0 + rg * 32;
   const int myq = wq0 + j;
   // Dropout: this row's key of the keep-mask hash.
   const u32 drop_rk =
@@ -1909,12 +1927,12 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd32_kernel(FwdParams pin) {
 
   for (int t = t_begin; t < t_end; ++t) {
     const int stage = NSTG == 1 ? 0 : (t - t_begin) & 1;
-    const int kv0 = kv_lo + t * BN;
+    const int kvt = kv_lo + t * BN, kv0 = kvt + kg * BNW;
     const bool has_next = t + 1 < t_end;
-    if (NSTG == 2 && has_next) load_tile(kv0 + BN);
+    if (NSTG == 2 && has_next) load_tile(kvt + BN);
 
     bool skip, full;
-    classify_tile<BN>(p, kv0, wq0, wq0 + 31, skip, full);
+    classify_tile<BNW>(p, kv0, wq0, wq0 + 31, skip, full);
     uint64_t vmask = ~0ull;
     if constexpr (PAGED) {
       if (!skip) {
@@ -1927,8 +1945,8 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd32_kernel(FwdParams pin) {
       }
     }
     if (!skip) {
-      const float* Ks = smem + stage * STAGE;
-      const float* Vs = Ks + K_ELEMS;
+      const float* Ks = smem + stage * STAGE + kg * BNW * KS;
+      const float* Vs = smem + stage * STAGE + K_ELEMS + kg * BNW * VS;
 
       f32x16 s[NB];
 #pragma unroll
@@ -2020,13 +2038,52 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd32_kernel(FwdParams pin) {
     if (has_next) {
       if constexpr (NSTG == 1) {
         __syncthreads();
-        load_tile(kv0 + BN);
+        load_tile(kvt + BN);
       }
       store_tile(NSTG == 1 ? 0 : stage ^ 1);
     }
     __syncthreads();
   }
 
+  if constexpr (KG > 1) {
+    // (every wave is past its last read of the stages)
+    static_assert((KG - 1) * NR * (NDB * 1024 + 192) <= NSTG * STAGE, "LDS");
+    f32x4* const at = (f32x4*)smem + lane;
+    float* const ml = smem + (KG - 1) * NR * NDB * 1024 + lane;
+    if (kg > 0) {
+      const int r = (kg - 1) * NR + rg;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4)
+          at[(r * NDB * 4 + 4 * db + e4) * 64] = (f32x4){o[db][4 * e4], o[db][4 * e4 + 1],
+                                                         o[db][4 * e4 + 2], o[db][4 * e4 + 3]};
+      ml[r * 192] = m_run;
+      ml[r * 192 + 64] = m_max;
+      ml[r * 192 + 128] = l_run;
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int k = 1; k < KG; ++k) {
+      const int r = (k - 1) * NR + rg;
+      const float mr = ml[r * 192], lr = ml[r * 192 + 128];
+      m_max = fmaxf(m_max, ml[r * 192 + 64]);
+      const float mn = fmaxf(m_run, mr);
+      const float a0 = m_run == -INFINITY ? 0.f : fast_exp2(m_run - mn);
+      const float a1 = mr == -INFINITY ? 0.f : fast_exp2(mr - mn);
+      l_run = l_run * a0 + lr * a1;
+      m_run = mn;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+          const f32x4 x = at[(r * NDB * 4 + 4 * db + e4) * 64];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[db][4 * e4 + i] = o[db][4 * e4 + i] * a0 + x[i] * a1;
+        }
+    }
+  }
   const float l_tot = pair_sum32(l_run);
   const float f = m_max == -INFINITY ? 0.f : fast_exp2(m_run - m_max);
   // (dropout: kept weights times 1 / (1 - p); the row sums stay unscaled)

@@ -192,3 +192,23 @@ def test_lse_of_key_groups(device, S, H):
     want = torch.logsumexp(s, -1) / math.log(2)
     # scores of products of float16: Q times the scale is rounded to float16 (2^-11 of ~5)
     assert float((lse.double().cpu() - want).abs().max()) <= 1e-2
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("B,H,H_kv,Sq,Sk,causal,W", [
+    (1, 8, 8, 1, 300, False, None), (1, 8, 8, 33, 97, True, None), (1, 8, 2, 300, 300, True, None),
+    (1, 8, 8, 700, 700, True, 100), (2, 16, 16, 300, 300, True, None),  # 10 tiles per XCD
+    (1, 16, 16, 1300, 1300, True, None),   # 42 q-tiles on each XCD: second half reversed
+    (2, 12, 12, 1024, 1024, True, None),   # 48, the training case
+    (1, 3, 1, 500, 500, False, None)])
+def test_float32_key_groups(device, B, H, H_kv, Sq, Sk, causal, W, D):
+    q = rnd((B, Sq, H, D), 1, torch.float32)
+    k, v = rnd((B, Sk, H_kv, D), 2, torch.float32), rnd((B, Sk, H_kv, D), 3, torch.float32)
+    qd, kd, vd = (x.to(device) for x in (q, k, v))
+    if W is None:
+        out = flash_attention(qd, kd, vd, causal=causal, enable_gqa=H != H_kv)
+    else:
+        out = sliding_window_attention(qd, kd, vd, W, causal=causal)
+    want = dense(q, k, v, W, max(0, Sk - Sq) if causal else None)
+    # the repository's float32 forward bar
+    np.testing.assert_allclose(out.double().cpu().numpy(), want, rtol=1e-4, atol=1e-5)
