@@ -1,4 +1,5 @@
-// Attention backward for gfx950 (MI355X), bf16 / f16, head_dim 64 or 128.
+// Attention backward for gfx950 (MI355X), bf16 / f16, head_dim 64,
+// 128 or 256.
 //
 // Gradients of O = softmax(scale * Q K^T + mask) V (with the forward's
 // O / (l + eps) normaliser) for mlx_primitives' flash_attention
@@ -10,7 +11,8 @@
 //   dQ = scale * dS K                                 (fa_bwd_dq_kernel)
 //   dV = P^T dO,  dK = scale * dS^T Q                 (fa_bwd_dkdv_kernel,
 //                                                      fa_bwd_dkdv_fused_kernel)
-// Two MFMA kernels, no atomics: dQ is query-parallel (each workgroup owns 128
+// Two kinds of tiles, no atomics (a launch of each, or both in one:
+// fa_bwd_joint_kernel, with Dvec by a launch of its own): dQ is query-parallel (each workgroup owns 128
 // query rows and streams K and V; it also writes Dvec), dK/dV key-parallel
 // (each workgroup owns 128 keys and streams Q and dO). Both recompute S and
 // dP; tiles go from HBM straight into LDS (buffer_load ... lds), double

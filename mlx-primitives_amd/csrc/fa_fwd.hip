@@ -143,8 +143,8 @@ Plan plan_for(int kg, int B, int H, int Sq, int Sk, int D, int causal, int windo
 // items (Q, filling the DMA pipeline, the epilogue) and the split merge.
 // A step of 128 keys takes 3.5 / 2.3 / 1.8 us with 1 / 2 / 4 key groups at
 // D = 128 and 2.3 / 1.25 / 0.8 at D = 64 (a workgroup's row count halves each
-// time, but its tile still has to come in), an item about 6 us, splitting and
-// merging about 14.
+// time, but its tile still has to come in), an item 6 us (7.2 with
+// groups to merge), splitting and merging about 14.
 double plan_time(const Plan& pl, long bh, int Sq, int Sk, int D) {
   static const double kStep[2][3] = {{2.3, 1.25, 0.8}, {3.5, 2.3, 1.8}};
   const double step = kStep[D == 128][pl.kg == 4 ? 2 : pl.kg - 1] * pl.BN / 128;
@@ -217,7 +217,10 @@ Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
   };
   Plan best = plan(1);
   const long bh = (long)B * H;
-  if (dtype == MPX_F32 && D <= 64 && !paged) {
+  // Up to 8 q-tiles per CU: a busy chip runs two groups' twice as many 64-row
+  // tiles at 6.6 us for one group's 5.3, so past that there is nothing to find
+  // and the walk over the tiles is host time lost.
+  if (dtype == MPX_F32 && D <= 64 && !paged && bh * best.n_qtiles <= 8 * kNumCUs) {
     double t = plan_time32(best, bh, Sq, Sk, D);
     for (bool split : {true, false}) {
       Plan pl = plan_for(2, B, H, Sq, Sk, D, causal, window_left, window_right, dtype,
@@ -239,7 +242,9 @@ Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
   double t = plan_time(best, bh, Sq, Sk, D);
   for (int kg = 2; kg <= (best.BN == 128 ? 4 : 2); kg *= 2) {
     const Plan pl = plan(kg);
-    const double tk = plan_time(pl, bh, Sq, Sk, D);
+    // (paged items pay more for four groups: one 128-key step alone, (2, 74, 32,
+    // 128), takes 10.4 us with one group and 11.3 with four)
+    const double tk = plan_time(pl, bh, Sq, Sk, D) + (paged && kg == 4 ? 0.8 : 0.0);
     if (tk < 0.97 * t) {
       best = pl;
       t = tk;

@@ -35,6 +35,8 @@ namespace {
   X(mpx_attn_bwd_ds_preferred)                                                              \
   X(mpx_paged_decode_gqa)                                                                   \
   X(mpx_paged_decode_workspace_bytes)                                                       \
+  X(mpx_paged_prefill_gqa)                                                                  \
+  X(mpx_paged_prefill_workspace_bytes)                                                      \
   X(mpx_kv_append)                                                                          \
   X(mpx_kv_append_rope)                                                                     \
   X(mpx_rope_at)
@@ -236,11 +238,12 @@ PyObject* attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// paged_decode(q, k_pool, v_pool, tables, lens, slopes or None, scale, stream)
-//   -> o, an error code, or None; the caller has checked the shapes
-PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
+// paged_attend(q, k_pool, v_pool, tables, lens, slopes or None, scale, causal,
+//   stream) -> o, an error code, or None; the caller has checked the shapes.
+// Decode for one query per sequence, else prefill (head dims of the kernels).
+PyObject* paged_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (wrong_count(n, 8)) return nullptr;
+  if (wrong_count(n, 9)) return nullptr;
   const at::Tensor* t[6];
   for (int i = 0; i < 6; ++i) {
     t[i] = nullptr;
@@ -257,17 +260,27 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       (t[5] && (t[5]->scalar_type() != at::kFloat || !t[5]->is_contiguous())))
     Py_RETURN_NONE;
   const double scale = as_float(a[6]);
-  void* stream = PyLong_AsVoidPtr(a[7]);
+  const int causal = PyObject_IsTrue(a[7]);
+  void* stream = PyLong_AsVoidPtr(a[8]);
   if (PyErr_Occurred()) return nullptr;
-  const int B = (int)q.size(0), H = (int)q.size(2), D = (int)q.size(3);
+  const int B = (int)q.size(0), Sq = (int)q.size(1), H = (int)q.size(2), D = (int)q.size(3);
   const int nb = (int)kp.size(0), bs = (int)kp.size(1), H_kv = (int)kp.size(2);
   const int mb = (int)bt.size(1);
   at::Tensor o = at::empty(q.sizes(), q.options());
-  const size_t need = api.mpx_paged_decode_workspace_bytes(B, H, D, bs, mb);
+  const size_t need =
+      Sq == 1 ? api.mpx_paged_decode_workspace_bytes(B, H, D, bs, mb)
+              : api.mpx_paged_prefill_workspace_bytes(B, Sq, H, D, bs, mb, causal, code);
   at::Tensor ws = bytes(need, q);
-  const int64_t qs[2] = {q.stride(0), q.stride(2)}, os[2] = {o.stride(0), o.stride(2)};
+  const int64_t qs[3] = {q.stride(0), q.stride(2), q.stride(1)};
+  const int64_t os[3] = {o.stride(0), o.stride(2), o.stride(1)};
   const float* const sl = t[5] ? t[5]->data_ptr<float>() : nullptr;
   const int rc = call([&] {
+    if (Sq != 1)
+      return api.mpx_paged_prefill_gqa(q.data_ptr(), kp.data_ptr(), vp.data_ptr(),
+                                       bt.data_ptr<int32_t>(), cl.data_ptr<int32_t>(), sl,
+                                       o.data_ptr(), qs, os, B, Sq, H, H_kv, D, nb, bs, mb,
+                                       (float)scale, causal, code, ws.data_ptr(),
+                                       (size_t)ws.numel(), stream);
     return api.mpx_paged_decode_gqa(q.data_ptr(), kp.data_ptr(), vp.data_ptr(),
                                     bt.data_ptr<int32_t>(), cl.data_ptr<int32_t>(), sl,
                                     o.data_ptr(), qs, os, B, H, H_kv, D, nb, bs, mb, (float)scale,
@@ -392,7 +405,7 @@ PyObject* entries(PyObject*, PyObject*) {
 }
 
 #define FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(attn_fwd),  FAST(attn_bwd), FAST(paged_decode),
+PyMethodDef methods[] = {FAST(attn_fwd),  FAST(attn_bwd), FAST(paged_attend),
                          FAST(kv_append), FAST(rope_at),  {"init", init, METH_O, nullptr},
                          {"entries", entries, METH_NOARGS, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

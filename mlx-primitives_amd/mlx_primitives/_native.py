@@ -491,15 +491,15 @@ def paged_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     _check(rc, "mpx_paged_decode failed")
 
 
-def paged_decode_new(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+def paged_attend_new(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
                      block_tables: torch.Tensor, context_lens: torch.Tensor,
-                     alibi_slopes: Optional[torch.Tensor], scale: float):
-    """paged_decode into a new tensor through the host extension (None: the
-    general path)."""
-    r = host().paged_decode(q, k_pool, v_pool, block_tables, context_lens, alibi_slopes,
-                            float(scale), _stream_ptr(q.device) if q.is_cuda else 0)
+                     alibi_slopes: Optional[torch.Tensor], scale: float, causal: bool):
+    """paged_decode (one query per sequence) or paged_prefill into a new tensor
+    through the host extension (None: the general path)."""
+    r = host().paged_attend(q, k_pool, v_pool, block_tables, context_lens, alibi_slopes,
+                            float(scale), causal, _stream_ptr(q.device) if q.is_cuda else 0)
     if r.__class__ is int:
-        _check(r, "mpx_paged_decode failed")
+        _check(r, "mpx_paged_decode failed" if q.shape[1] == 1 else "mpx_paged_prefill failed")
     return r
 
 

@@ -58,9 +58,9 @@ def _dims(q: torch.Tensor, k: torch.Tensor, layout: Layout):
     return B, H, k.shape[1], Sq, k.shape[2], D
 
 
-# The backward's schedule (_native.attn_bwd's stored_ds): None = the stored-dS
-# schedule for the dropout backward where it applies and its workspace fits,
-# True = the stored-dS schedule, False = recompute S and dP for dQ.
+# The backward's schedule (_native.attn_bwd's stored_ds): None = chosen by the
+# launch's size (large dropout backwards whose workspace fits store dS, the rest
+# recompute S and dP), True = the stored-dS schedule, False = recompute.
 BWD_STORED_DS: Optional[bool] = None
 
 

@@ -19,7 +19,7 @@ from mlx_primitives import _native
 
 
 def _i32(x, device, n: int, what: str) -> torch.Tensor:
-    if type(x) is int:
+    if type(x) is int and n > 0:
         # filled on the device: a copy from the host would wait for the stream
         return torch.full((n,), x, dtype=torch.int32, device=device)
     t = torch.as_tensor(x, dtype=torch.int32, device=device).reshape(-1)

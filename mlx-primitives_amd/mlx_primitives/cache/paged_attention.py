@@ -116,8 +116,9 @@ def paged_attention(
         q = q.contiguous()
     tables = _as_i32(block_tables)
     lens = _as_i32(context_lens)
-    if seq_q == 1 and dk == dim:
-        out = _native.paged_decode_new(q, k_pool, v_pool, tables, lens, alibi_slopes, scale)
+    if dk == dim:
+        out = _native.paged_attend_new(q, k_pool, v_pool, tables, lens, alibi_slopes, scale,
+                                       causal)
         if out is not None:
             return out
     out = torch.empty((batch, seq_q, heads, dk), dtype=q.dtype, device=q.device)

@@ -157,6 +157,24 @@ def test_decode(device, monkeypatch, H, H_kv, D, dtype, alibi):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,H_kv,D,dtype", [(8, 2, 128, torch.bfloat16), (4, 4, 64, torch.float32),
+                                            (4, 4, 72, torch.float16)])
+@pytest.mark.parametrize("causal,alibi", [(True, False), (False, True)])
+@pytest.mark.parametrize("S", [0, 2, 40])
+def test_prefill(device, monkeypatch, H, H_kv, D, dtype, causal, alibi, S):
+    kp, vp = (rnd(9, 16, H_kv, D, dtype=dtype, seed=s).to(device) for s in (1, 2))
+    q = rnd(3, S, H, D, dtype=dtype, seed=3).to(device)
+    tables = torch.tensor([[0, 3, 5], [1, 2, -1], [4, 8, 7]], device=device)
+    lens = torch.tensor([40, 0, 33], device=device)
+    slopes = get_alibi_slopes(H, device=device) if alibi else None
+    for it in (torch.int32, torch.int64):
+        for view in (lambda x: x, lambda x: x.transpose(1, 2).contiguous().transpose(1, 2)):
+            both(monkeypatch, lambda: [paged_attention(view(q), kp, vp, tables.to(it), lens.to(it),
+                                                       causal=causal, alibi_slopes=slopes,
+                                                       enable_gqa=True)])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rope", [False, True])
 @pytest.mark.parametrize("counts", [None, 1, "tensor"])
 def test_append_and_rope_at(device, monkeypatch, rope, counts):
