@@ -104,8 +104,17 @@ int call(F&& f) {
   return rc;
 }
 
-// Argument i as a C value; the Python layer passes plain ints and floats.
-int64_t as_int(PyObject* o) { return PyLong_AsLongLong(o); }
+// An argument as the general path's int(...) and ctypes read it: what has
+// __int__, __index__ or __trunc__ (masks and windows come as the user gave
+// them: floats, numpy scalars), of which the low bits count.
+int64_t as_int(PyObject* o) {
+  if (PyLong_Check(o)) return (int64_t)PyLong_AsUnsignedLongLongMask(o);
+  PyObject* const x = PyNumber_Long(o);
+  if (!x) return -1;
+  const int64_t v = (int64_t)PyLong_AsUnsignedLongLongMask(x);
+  Py_DECREF(x);
+  return v;
+}
 double as_float(PyObject* o) { return PyFloat_AsDouble(o); }
 
 bool wrong_count(Py_ssize_t n, Py_ssize_t want) {
@@ -260,10 +269,10 @@ PyObject* paged_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
       (t[5] && (t[5]->scalar_type() != at::kFloat || !t[5]->is_contiguous())))
     Py_RETURN_NONE;
   const double scale = as_float(a[6]);
-  const int causal = PyObject_IsTrue(a[7]);
+  const int B = (int)q.size(0), Sq = (int)q.size(1), H = (int)q.size(2), D = (int)q.size(3);
+  const int causal = Sq == 1 ? 0 : (int)as_int(a[7]);  // (decode takes no mask)
   void* stream = PyLong_AsVoidPtr(a[8]);
   if (PyErr_Occurred()) return nullptr;
-  const int B = (int)q.size(0), Sq = (int)q.size(1), H = (int)q.size(2), D = (int)q.size(3);
   const int nb = (int)kp.size(0), bs = (int)kp.size(1), H_kv = (int)kp.size(2);
   const int mb = (int)bt.size(1);
   at::Tensor o = at::empty(q.sizes(), q.options());

@@ -2,6 +2,7 @@
 calls with the extension answering None give the same bits, over the layouts
 that it takes and those that it leaves."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -138,6 +139,52 @@ def test_dropout_window_and_second_derivative(device, monkeypatch, layout):
                                create_graph=True)
     with pytest.raises(RuntimeError):
         g.sum().backward()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80])
+def test_windows_and_masks_as_int_reads_them(device, monkeypatch, D):
+    # whatever int(...) takes, with its value: floats, numpy scalars, 0-dim
+    # tensors; what int(...) refuses is refused
+    q, k, v = (rnd(1, 70, 4, D, seed=s).to(device) for s in range(3))
+    want = sliding_window_attention(q, k, v, 20)
+
+    for W in (20.0, 20.9, np.float32(20), np.int64(20), torch.tensor(20)):
+        def fn():
+            a = q.detach().requires_grad_(True)
+            o = sliding_window_attention(a, k, v, W)
+            return [sliding_window_attention(q, k, v, W), o.detach(),
+                    *torch.autograd.grad(o, a, torch.ones_like(o))]
+        assert torch.equal(both(monkeypatch, fn)[0], want)
+    for causal in (1.0, 2, np.True_, 0.5, np.float64(0.5), 0, "1"):
+        (out,) = both(monkeypatch, lambda: [flash_attention(q, k, v, causal=causal)])
+        assert torch.equal(out, flash_attention(q, k, v, causal=int(causal) != 0))
+    for bad in (None, [], "x"):
+        def refused():
+            with pytest.raises((TypeError, ValueError)):
+                flash_attention(q, k, v, causal=bad)
+            return []
+        both(monkeypatch, refused)
+
+
+@pytest.mark.gpu
+def test_paged_masks_as_int_reads_them(device, monkeypatch):
+    kp, vp, q = (rnd(*n, 2, 64, seed=1).to(device) for n in ((3, 16), (3, 16), (1, 40)))
+    tables = torch.tensor([[0, 2, 1]], dtype=torch.int32, device=device)
+    lens = torch.tensor([40], dtype=torch.int32, device=device)
+    for causal in (1.0, 2, np.True_, 0.5, 0):
+        (out,) = both(monkeypatch,
+                      lambda: [paged_attention(q, kp, vp, tables, lens, causal=causal)])
+        assert torch.equal(out, paged_attention(q, kp, vp, tables, lens,
+                                                causal=int(causal) != 0))
+    # decode ignores it
+    both(monkeypatch, lambda: [paged_attention(q[:, :1], kp, vp, tables, lens, causal=None)])
+
+    def refused():
+        with pytest.raises(TypeError):
+            paged_attention(q, kp, vp, tables, lens, causal=None)
+        return []
+    both(monkeypatch, refused)
 
 
 @pytest.mark.gpu
