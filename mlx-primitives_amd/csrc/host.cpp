@@ -95,13 +95,15 @@ at::Tensor bytes(size_t n, const at::Tensor& like) {
   return at::empty({(int64_t)(n < 16 ? 16 : n)}, like.options().dtype(at::kByte));
 }
 
+// f() without the GIL, which is taken back also when f throws (data_ptr() of
+// some tensors does).
 template <class F>
 int call(F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = f();
-  Py_END_ALLOW_THREADS;
-  return rc;
+  struct Released {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return f();
 }
 
 // An argument as the general path's int(...) and ctypes read it: what has

@@ -123,6 +123,22 @@ def test_which_calls_are_taken(device, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_tensors_that_refuse_their_address(device, monkeypatch):
+    # data_ptr() throws while the GIL is released: the general path's error
+    q = rnd(1, 1, 2, 128).to(device)
+    kp, vp = (rnd(4, 16, 2, 128, seed=s).to(device) for s in (1, 2))
+    torch._C._set_throw_on_mutable_data_ptr(vp)
+    tables = torch.zeros(1, 1, dtype=torch.int32, device=device)
+    lens = torch.ones(1, dtype=torch.int32, device=device)
+
+    def fn():
+        with pytest.raises(RuntimeError, match="data pointer"):
+            paged_attention(q, kp, vp, tables, lens)
+        return []
+    both(monkeypatch, fn)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["BSHD", "BHSD"])
 def test_dropout_window_and_second_derivative(device, monkeypatch, layout):
     q, k, v = (rnd(1, 130, 8, 64, seed=s).to(device) for s in range(3))
