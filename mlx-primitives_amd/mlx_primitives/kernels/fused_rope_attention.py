@@ -68,7 +68,7 @@ def _k_in_kernel(q, k, cos_cache, sin_cache, q_offset: int, kv_offset: int, mask
         return False
     return _native.rope_qk_preferred(
         q.shape[0], q.shape[2], q.shape[1], k.shape[1], q.shape[3], mask["causal"], -1,
-        mask.get("window_right", -1), q.dtype, cos_cache.dtype)
+        int(mask.get("window_right", -1)), q.dtype, cos_cache.dtype)
 
 
 def _rope_attention(q, k, v, scale, cos_cache, sin_cache, rope_base, q_offset, kv_offset,

@@ -165,6 +165,18 @@ def test_k_rotated_in_the_kernel_equals_rope_first(device, B, H, Sq, Sk, q_off, 
     assert torch.equal(out, o)
 
 
+@pytest.mark.parametrize("offset", [40.0, np.float32(40), np.int64(40), torch.tensor(40)])
+def test_offsets_as_int_reads_them(device, offset):
+    # Where K is rotated in the kernel (Sq = 3) and where it is not (Sq = 700).
+    cos, sin = precompute_rope_cache(800, 128, dtype=torch.bfloat16, device=device)
+    k, v = (rnd((1, 700, 4, 128), s, torch.bfloat16).to(device) for s in (2, 3))
+    for Sq in (3, 700):
+        q = rnd((1, Sq, 4, 128), 1, torch.bfloat16).to(device)
+        a, b = (fused_rope_attention(q, k, v, cos_cache=cos, sin_cache=sin, q_offset=o,
+                                     kv_offset=0, causal=True) for o in (offset, 40))
+        assert torch.equal(a, b)
+
+
 def test_k_rotation_left_to_its_own_pass():
     # full launches, float32 tables, other inputs and head dims
     pref = _native.rope_qk_preferred
