@@ -19,8 +19,9 @@ from mlx_primitives import _native
 
 
 def _i32(x, device, n: int, what: str) -> torch.Tensor:
-    if type(x) is int and n > 0:
+    if type(x) is int and n > 0 and -2**31 <= x < 2**31:
         # filled on the device: a copy from the host would wait for the stream
+        # (as_tensor refuses what int32 does not hold)
         return torch.full((n,), x, dtype=torch.int32, device=device)
     t = torch.as_tensor(x, dtype=torch.int32, device=device).reshape(-1)
     if t.numel() == 1 and n > 1:

@@ -9,6 +9,7 @@ import torch
 from mlx_primitives import _native
 from mlx_primitives.attention import flash_attention, sliding_window_attention
 from mlx_primitives.cache import get_alibi_slopes, paged_attention, store_kv
+from mlx_primitives.cache.kv_store import _i32
 from mlx_primitives.kernels import precompute_rope_cache, rope_at
 
 
@@ -68,6 +69,25 @@ def test_entries_are_the_librarys():
     with pytest.raises(KeyError):
         _native.host().init({})
     assert _native._load_host(lib) is not None  # (binds the entries again)
+
+
+@pytest.mark.parametrize("x", [2**31 - 1, -2**31, 2**31, 2**63, -2**31 - 1, True])
+@pytest.mark.parametrize("n", [0, 1, 3])
+def test_int_positions_are_refused_as_as_tensor_does(x, n):
+    def general():
+        t = torch.as_tensor(x, dtype=torch.int32).reshape(-1)
+        t = t.expand(n) if n > 1 else t
+        if t.numel() != n:
+            raise ValueError
+        return t
+    try:
+        want = general()
+    except Exception as e:
+        with pytest.raises(type(e)):
+            _i32(x, "cpu", n, "x")
+    else:
+        got = _i32(x, "cpu", n, "x")
+        assert got.dtype == torch.int32 and got.tolist() == want.tolist()
 
 
 @pytest.mark.gpu
