@@ -58,6 +58,14 @@ __host__ __device__ inline void ds_key_tile(int Sq, int Sk, int win_left, int wi
   nt = q_hi > q_lo ? (q_hi - 1) / 32 - t0 + 1 : 0;
 }
 
+// The query heads of part `part` of a K/V head, counted within its group: as
+// even as the parts divide it, the first ones a head longer.
+__device__ __forceinline__ void part_heads(const BwdParams& p, int part, int& first, int& n) {
+  const int least = p.kv_group / p.kv_parts, more = p.kv_group - least * p.kv_parts;
+  first = part * least + min(part, more);
+  n = least + (part < more ? 1 : 0);
+}
+
 // One key's dK (times scale) and dV (times mul_v) as float32 sums of a part of
 // the K/V head's query heads (BwdParams::dkv_part).
 // WANT_K / WANT_V: the outputs that the caller has.

@@ -531,8 +531,9 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdParams& p, uint16_t* lds,
   const int q_hi = p.win_left >= 0 ? min(p.Sq, k_last + p.win_left + 1) : p.Sq;
   const int t0 = q_lo / ROWS;
   const int n_t = q_hi > q_lo ? (q_hi - 1) / ROWS - t0 + 1 : 0;
-  const int heads = SPLIT ? p.kv_group / p.kv_parts : p.kv_group;
-  const int h0 = hk * p.kv_group + (SPLIT ? part * heads : 0);
+  int h0 = 0, heads = p.kv_group;
+  if constexpr (SPLIT) part_heads(p, part, h0, heads);
+  h0 += hk * p.kv_group;
   const int n_steps = n_t * heads;
 
   Addr<D> ad;
@@ -798,8 +799,9 @@ __device__ __forceinline__ void bwd_dkdv_fused_tiles(const BwdParams& p, uint16_
     const int q_hi = p.win_left >= 0 ? min(p.Sq, k_last + p.win_left + 1) : p.Sq;
     const int t0 = q_lo / kFusedTile;
     const int n_t = q_hi > q_lo ? (q_hi - 1) / kFusedTile - t0 + 1 : 0;
-    const int heads = SPLIT ? p.kv_group / p.kv_parts : p.kv_group;
-    const int h0 = hk * p.kv_group + (SPLIT ? part * heads : 0);
+    int h0 = 0, heads = p.kv_group;
+    if constexpr (SPLIT) part_heads(p, part, h0, heads);
+    h0 += hk * p.kv_group;
     const int n_steps = n_t * heads;
 
     f32x16 dk[NDB], dv[NDB];
@@ -1258,7 +1260,7 @@ void make_order(const BwdParams& p, int own, bool split, BwdOrder& order) {
   } items[kMaxOrder];
   int n = 0;
   for (int t = 0; t < n_kt; ++t) {
-    const int64_t rows = (int64_t)(p.kv_group / p.kv_parts) *
+    const int64_t rows = (int64_t)((p.kv_group + p.kv_parts - 1) / p.kv_parts) *
                          tile_reach(t, own, p.Sk, p.Sq, p.win_right, p.win_left);
     if (split) {
       items[n++] = {3 * rows, 4 * t + kTileDk};
@@ -1309,12 +1311,23 @@ bool bwd_joint(int B, int H, int Sq, int Sk, int D, int win_left) {
 }
 
 // Parts that a K/V head's query heads are cut into (1: none) for the grouped
-// backward at D <= 128: the fewest (a divisor of the group) that give the
-// dK/dV side a workgroup for each of the chip's slots (512; 256 in float32, at
-// one wave per SIMD). Causal bf16 (1, 2048, 32 heads over 8, 128): 409 -> 158
+// backward at D <= 128: the fewest equal ones (a divisor of the group) that give
+// the dK/dV side a workgroup for each of the chip's slots (512; 256 in float32,
+// at one wave per SIMD). Causal bf16 (1, 2048, 32 heads over 8, 128): 409 -> 158
 // us with 4 parts in the joint launch; (8, 1024, 32 over 4, 128): 488 -> 325 us
-// with 4 parts of paired tiles. The parts' sums are at most 512 + 511 tiles of
-// 128 keys (256 MB).
+// with 4 parts of paired tiles. Where the next divisor is far (groups like 7:
+// from 1 to 7) its sums can be large; above kMaxPartBytes the group is cut into
+// as many parts as that holds, some a head longer, which is still a workgroup
+// per slot: `need` parts are below 1024 workgroups, 256 MiB of pairs at D = 128.
+// Causal bf16 forward and backward, the divisor's sums against these: (4, 4000,
+// 28 over 4, 128) 439 MiB 2.12 ms, 250 MiB 2.07; (15, 4096, 71 over 1, 64) 2.1
+// GiB 13.0 ms, 240 MiB 12.2.
+constexpr size_t kMaxPartBytes = 256u << 20;
+
+size_t part_bytes(int B, int H_kv, int Sk, int D, int parts) {
+  return (size_t)2 * B * H_kv * parts * Sk * D * sizeof(float);
+}
+
 int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, int dtype) {
   const int group = H / H_kv;
   if (group == 1 || D > 128) return 1;
@@ -1323,9 +1336,12 @@ int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, in
   const int own = pairs ? 2 * kBwdOwn
                         : (f32 && bwd32_joint(B, H, Sq, Sk, D) ? kBwdOwn / 2 : kBwdOwn);
   const long wgs = (long)B * H_kv * ((Sk + own - 1) / own), slots = f32 ? 256 : 512;
-  for (int parts = 1; parts < group; ++parts)
-    if (group % parts == 0 && wgs * parts >= slots) return parts;
-  return group;
+  const long need = (slots + wgs - 1) / wgs;
+  if (need >= group) return group;
+  int parts = (int)need;
+  while (group % parts != 0) ++parts;
+  if (parts == 1 || part_bytes(B, H_kv, Sk, D, parts) <= kMaxPartBytes) return parts;
+  return (int)(kMaxPartBytes / part_bytes(B, H_kv, Sk, D, 1));
 }
 
 template <int D, bool BF16>
@@ -1435,7 +1451,7 @@ extern "C" size_t mpx_attn_bwd_grouped_workspace_bytes(int B, int H, int H_kv, i
   if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || Sq <= 0 || Sk <= 0 || D <= 0) return 0;
   const int parts = bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype);
   if (parts == 1) return mpx_attn_bwd_workspace_bytes(B, H, Sq);
-  return dvec_region_bytes(B, H, Sq) + (size_t)2 * B * H_kv * parts * Sk * D * sizeof(float);
+  return dvec_region_bytes(B, H, Sq) + part_bytes(B, H_kv, Sk, D, parts);
 }
 
 extern "C" int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk, int D, int dtype,

@@ -332,7 +332,9 @@ __device__ __forceinline__ void bwd32_dkdv_tile(const BwdParams& p, float* smem,
   // (steps of KG tiles of one head)
   const int t0 = q_lo / kB32Tile;
   const int n_t = q_hi > q_lo ? ((q_hi - 1) / kB32Tile - t0) / KG + 1 : 0;
-  const int heads = p.kv_group / p.kv_parts, h0 = hk * p.kv_group + part * heads;
+  int h0, heads;
+  part_heads(p, part, h0, heads);
+  h0 += hk * p.kv_group;
   const int n_steps = n_t * heads;
 
   f32x16 dk[NDB], dv[NDB];

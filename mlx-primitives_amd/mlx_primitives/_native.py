@@ -441,8 +441,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     grouped = False
     if ws is None and H_kv != H:
         # room for the parts that a K/V head's query heads are cut into (at
-        # most about a quarter of a GiB: the parts stop at one workgroup per
-        # slot of the chip); without it each head's group is one part
+        # most 256 MiB of sums); without it each head's group is one part
         part_bytes = int(lib.mpx_attn_bwd_grouped_workspace_bytes(
             B, H, H_kv, Sq, Sk, D, code, int(window_left)))
         try:

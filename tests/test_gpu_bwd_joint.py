@@ -90,6 +90,9 @@ CASES = [
     (2, 16, 16, 4096, 200, 128, False, None),    # 32 x 34 tiles: joint
     (1, 32, 4, 4096, 4096, 128, True, None),     # 2048 tiles: paired, 4 parts
     (1, 31, 31, 4100, 4100, 128, True, None),    # 2046 tiles: joint
+    (1, 20, 4, 64, 16384, 128, True, None),      # 5 heads in 4 parts: paired tiles
+    (1, 33, 3, 64, 16384, 64, False, None),      # 11 in 10, two launches at D = 64
+    (1, 4, 2, 64, 16384, 64, True, None),        # 2 parts of one head, two launches
 ]
 
 
@@ -126,6 +129,8 @@ CASES32 = [  # float32: tiles of 64 rows, two key groups of 32
     (1, 4, 1, 64, 6000, 128, False, None),       # too many for an order: parts alone
     (1, 31, 31, 2112, 2112, 64, True, None),     # 2046 tiles: joint
     (1, 32, 8, 2048, 2048, 64, True, None),      # 2048: launches of their own, 2 parts
+    (1, 74, 2, 64, 8256, 64, False, None),       # 37 heads in 31 parts, own launches
+    (1, 34, 2, 64, 8256, 128, True, None),       # 17 in 15
 ]
 
 
@@ -147,6 +152,23 @@ def test_joint_dropout_agrees_with_stored_schedule(device, monkeypatch, H, H_kv,
         monkeypatch.setattr(_launch, "BWD_STORED_DS", stored)
         torch.manual_seed(5)
         got[stored] = run(device, q, k, v, d, dropout=0.2)
+    for name, a, b in zip(("dq", "dk", "dv"), got[True], got[None]):
+        rel = float((a.double() - b.double()).norm() / a.double().norm())
+        assert rel <= 4e-3, (name, rel)
+
+
+@pytest.mark.gpu
+def test_uneven_parts_with_dropout(device, monkeypatch):
+    # The keep mask of every head where one part holds a head more than the
+    # others, against the stored-dS schedule, which has no parts.
+    H, H_kv, Sk = 20, 4, 16384
+    q, d = rnd((1, 64, H, 128), 1, torch.bfloat16), rnd((1, 64, H, 128), 2, torch.bfloat16)
+    k, v = rnd((1, Sk, H_kv, 128), 3, torch.bfloat16), rnd((1, Sk, H_kv, 128), 4, torch.bfloat16)
+    got = {}
+    for stored in (True, None):
+        monkeypatch.setattr(_launch, "BWD_STORED_DS", stored)
+        torch.manual_seed(5)
+        got[stored] = run(device, q, k, v, d, causal=False, dropout=0.2)
     for name, a, b in zip(("dq", "dk", "dv"), got[True], got[None]):
         rel = float((a.double() - b.double()).norm() / a.double().norm())
         assert rel <= 4e-3, (name, rel)
@@ -191,3 +213,31 @@ def test_grouped_workspace_bytes():
     assert ws(1, 8, 3, 300, 300, 128, 2, -1) == 0
     # parts stop at one workgroup per slot of the chip
     assert ws(4, 32, 8, 4096, 4096, 128, 2, -1) == lib.mpx_attn_bwd_workspace_bytes(4, 32, 4096)
+
+
+@pytest.mark.parametrize("group", [2, 3, 4, 5, 6, 7, 8, 11, 12, 28, 31, 64, 71])
+def test_grouped_workspace_is_bounded(group):
+    # also where the group has no divisor near the count that fills the chip
+    lib = _native.load()
+    most = 0
+    for B in (1, 2, 3, 4, 7, 8, 15, 16):
+        for H_kv in (1, 2, 4, 8):
+            for S in (64, 300, 1024, 2048, 4000, 4096, 4608, 8192, 16384, 32768, 65000):
+                for D in (64, 128):
+                    for dtype in (0, 2):
+                        need = lib.mpx_attn_bwd_grouped_workspace_bytes(
+                            B, H_kv * group, H_kv, S, S, D, dtype, -1)
+                        plain = lib.mpx_attn_bwd_workspace_bytes(B, H_kv * group, S)
+                        most = max(most, need - -(-plain // 256) * 256)
+    assert most <= 256 << 20
+
+
+@pytest.mark.parametrize("H,H_kv,Sk,D,dtype,parts", [
+    (20, 4, 16384, 128, 2, 4), (33, 3, 16384, 64, 2, 10), (4, 2, 16384, 64, 2, 2),
+    (74, 2, 8256, 64, 0, 31), (34, 2, 8256, 128, 0, 15), (56, 8, 4096, 128, 2, 7)])
+def test_parts_of_a_group(H, H_kv, Sk, D, dtype, parts):
+    # the parts that the cases above mean
+    lib = _native.load()
+    plain = -(-lib.mpx_attn_bwd_workspace_bytes(1, H, 64) // 256) * 256
+    assert lib.mpx_attn_bwd_grouped_workspace_bytes(1, H, H_kv, 64, Sk, D, dtype, -1) \
+        == plain + 2 * H_kv * parts * Sk * D * 4
