@@ -316,8 +316,10 @@ int mpx_attn_fwd_rope(const void* q, const void* k, const void* v, void* o,
  * (per-row rowsum(dout * o)). A workspace of at least
  * mpx_attn_bwd_ds_workspace_bytes(...) bytes (same problem arguments; 0 when
  * the problem has no such schedule: float32, or D other than 128) selects the
- * stored-dS schedule (mpx_attn_bwd_dropout: in launches that fill the chip,
- * 2048 tiles of 128 rows or more): the dK/dV kernel stores dS (16-bit, only the 32 x 32
+ * stored-dS schedule (mpx_attn_bwd_dropout: in launches that fill the chip;
+ * below, that is with fewer than 2048 query and key tiles of 128 rows over all
+ * B * H heads, or up to 4096 with window_left >= 0, and at most 128 of them per
+ * head, it recomputes): the dK/dV kernel stores dS (16-bit, only the 32 x 32
  * blocks the mask leaves, about B * H * Sq * Sk bytes under a causal mask)
  * and dQ is computed from it instead of recomputing S and dP (and, with
  * dropout, the keep mask). On MI355X it is the faster schedule for

@@ -51,10 +51,12 @@ int mpx_attn_bwd_stored(const void* q, const void* k, const void* v, const void*
                         uint64_t seed, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * 1 when mpx_attn_bwd_dropout runs faster with the stored-dS workspace
- * (mpx_attn_bwd_ds_workspace_bytes) than without it, else 0: launches that do
- * not fill the chip, where it then recomputes whatever the workspace holds, and
- * grouped heads that run in parts.
+ * 1 when the dropout backward runs faster on the stored-dS schedule
+ * (mpx_attn_bwd_dropout with mpx_attn_bwd_ds_workspace_bytes) than recomputing
+ * (mpx_attn_bwd_grouped for grouped heads), else 0: launches that do not fill
+ * the chip, where mpx_attn_bwd_dropout recomputes whatever the workspace holds,
+ * and grouped heads that mpx_attn_bwd_grouped runs in parts (which
+ * mpx_attn_bwd_dropout does not: with that workspace it stores dS).
  */
 int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk, int D, int dtype,
                               int window_left);

@@ -1461,8 +1461,9 @@ extern "C" int mpx_attn_bwd_ds_preferred(int B, int H, int H_kv, int Sq, int Sk,
          bwd_kv_parts(B, H, H_kv, Sq, Sk, D, window_left, dtype) == 1;
 }
 
-// kBySize: stored dS where the workspace holds it (with dropout: and it is the
-// faster schedule); kGrouped: recomputing, in parts where the workspace holds
+// kBySize: stored dS where the workspace holds it (with dropout: and the launch
+// is not a joint one, which recomputes faster; a group's parts, which do too,
+// are kGrouped's); kGrouped: recomputing, in parts where the workspace holds
 // them; kStored: stored dS or an error.
 enum BwdSchedule { kBySize, kGrouped, kStored };
 
@@ -1557,8 +1558,7 @@ static int attn_bwd_entry(const void* q, const void* k, const void* v, const voi
       p.dkv_part = (float*)((char*)workspace + dvec_region_bytes(B, H, Sq));
     }
   } else if (ds_need > 0 && workspace_bytes >= ds_need &&
-             (schedule == kStored || !drop ||
-              mpx_attn_bwd_ds_preferred(B, H, H_kv, Sq, Sk, D, dtype, window_left))) {
+             (schedule == kStored || !drop || !bwd_joint(B, H, Sq, Sk, D, window_left))) {
     p.ds = (char*)workspace + dvec_region_bytes(B, H, Sq);
     p.ds_tot = ds_blocks_per_head(Sq, Sk, p.win_left, p.win_right);
   }

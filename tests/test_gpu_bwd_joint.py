@@ -199,6 +199,44 @@ def test_grouped_backward_without_room_for_parts(device):
         assert float((a.double() - b.double()).norm() / b.double().norm()) <= 1e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H_kv", [8, 2, 1])
+@pytest.mark.parametrize("Sq,Sk,stored", [(64, 16384, True), (64, 1000, False)])
+def test_dropout_entry_stores_ds_in_large_launches(device, H_kv, Sq, Sk, stored):
+    # mpx_attn_bwd_dropout with the stored-dS workspace, with and without groups:
+    # the bits of mpx_attn_bwd_stored and its dS blocks where the launch is not a
+    # joint one, else nothing but Dvec written.
+    B, H, D = 1, 8, 128
+    q, d = (rnd((B, Sq, H, D), s, torch.bfloat16).to(device) for s in (1, 2))
+    k, v = (rnd((B, Sk, H_kv, D), s, torch.bfloat16).to(device) for s in (3, 4))
+    lib = _native.load()
+    o, lse = torch.empty_like(q), torch.empty(B, H, Sq, device=device)
+    bhs = lambda x: (x.stride(0), x.stride(2), x.stride(1))
+    _native.attn_fwd(q, k, v, o, bhs(q), bhs(k), bhs(v), bhs(o), B, H, Sq, Sk, D, D ** -0.5, False,
+                     H_kv=H_kv, lse=lse, dropout=(0.2, 7))
+    nbytes = lib.mpx_attn_bwd_ds_workspace_bytes(B, H, Sq, Sk, D, 2, 0, -1, -1)
+    outs, left = {}, {}
+    for entry in ("mpx_attn_bwd_dropout", "mpx_attn_bwd_stored"):
+        got = [torch.empty_like(x) for x in (q, k, v)]
+        ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=device)
+        rc = getattr(lib, entry)(
+            *(x.data_ptr() for x in (q, k, v, o, d, lse, *got)),
+            *(_native._strides(bhs(x)) for x in (q, k, v, o, d, *got)), B, H, H_kv, Sq, Sk, D,
+            D ** -0.5, 0, -1, -1, 2, 0.2, 7, ws.data_ptr(), ws.numel(),
+            _native._stream_ptr(device))
+        assert rc == _native.MPX_OK
+        outs[entry] = got
+        left[entry] = int((ws[lib.mpx_attn_bwd_workspace_bytes(B, H, Sq):] == 0xA5).sum())
+    a, b = outs.values()
+    if stored:
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
+        assert left["mpx_attn_bwd_dropout"] == left["mpx_attn_bwd_stored"] < nbytes // 2
+    else:
+        assert left["mpx_attn_bwd_stored"] < nbytes // 2 < left["mpx_attn_bwd_dropout"]
+        for x, y in zip(a, b):
+            assert float((x.double() - y.double()).norm() / y.double().norm()) <= 4e-3
+
+
 def test_grouped_workspace_bytes():
     lib = _native.load()
     ws = lib.mpx_attn_bwd_grouped_workspace_bytes
