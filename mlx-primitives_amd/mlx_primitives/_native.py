@@ -17,6 +17,7 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 from typing import Optional, Sequence
 
 import torch
@@ -191,9 +192,22 @@ def load() -> ctypes.CDLL:
             ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
         ]
         global _host
-        _host = _load_host(lib)
+        try:
+            _host = _load_host(lib)
+        except (ImportError, RuntimeError) as e:
+            # (not built, or built for another Python or torch)
+            warnings.warn(f"mlx_primitives: every call takes its Python path: {e}",
+                          RuntimeWarning, stacklevel=2)
+            _host = _GeneralPath()
         _lib = lib
         return lib
+
+
+class _GeneralPath:
+    """In place of the host extension: leaves each call to the Python path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
 
 
 def _load_host(lib: ctypes.CDLL):

@@ -71,6 +71,20 @@ def test_entries_are_the_librarys():
     assert _native._load_host(lib) is not None  # (binds the entries again)
 
 
+@pytest.mark.parametrize("content", [None, b"", b"\x7fELF of another torch"])
+def test_package_loads_without_the_extension(monkeypatch, tmp_path, content):
+    # missing, empty or unreadable: a warning, and every call left to the Python path
+    path = tmp_path / "_mpx_host.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_native, "_HOST_PATH", str(path))
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "_host", None)
+    with pytest.warns(RuntimeWarning, match="Python path"):
+        assert _native.load().mpx_version() > 0
+    assert _native.host().rope_at(None, None, None, None, None, 0) is None
+
+
 @pytest.mark.parametrize("x", [2**31 - 1, -2**31, 2**31, 2**63, -2**31 - 1, True])
 @pytest.mark.parametrize("n", [0, 1, 3])
 def test_int_positions_are_refused_as_as_tensor_does(x, n):
