@@ -102,8 +102,9 @@ __device__ __forceinline__ constexpr int crow(int e, int g) {
 // per 32-key tile: S^T = K Q^T, dP^T = V dO^T, dS^T = P^T (dP^T - Dvec),
 // dQ^T += K^T dS^T.
 // ---------------------------------------------------------------------------
-// D = 256: one LDS stage (two would be 133 KB); the next tile is loaded after
-// the barrier that ends the current one.
+// D = 256: one LDS stage, the next tile loaded after the barrier that ends the
+// current one: a tile in flight under the compute, for a second stage, has no
+// registers left (491 to 512 are used).
 template <int D>
 constexpr int kStages32 = D > 128 ? 1 : 2;
 // LDS floats: [stage][K, V (or Q, dO)][32 KG rows], then lse and Dvec rows per stage.
@@ -473,6 +474,8 @@ void fa_bwd32_dkdv_kernel(BwdParams p) {
 template <int D, bool DROP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void fa_bwd32_joint_kernel(BwdParams p, BwdOrder order) {
+  // (133 KB at D = 128: no kernel here has more. 353 registers, none spilled.)
+  static_assert(kLds32<D, 2> * 4 <= 160 * 1024, "LDS of a CU");
   __shared__ __align__(16) float lds[kLds32<D, 2>];
   const BwdWork w = joint_work(order);
   if (w.kind == kTileDq) {

@@ -1689,8 +1689,12 @@ template <int D, int BN, int NW, bool BF16, bool PAGED, bool BIG = false, int KG
           bool ROPEK = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MPX_FA_WAVES_PER_EU)))
 void fa_fwd16_kernel(FwdParams p) {
-  // Stay within 128 KB of LDS per workgroup (a 136 KB configuration gave wrong
-  // results on gfx950).
+  // Tiles and page table within 128 KB of LDS per workgroup (a 136 KB
+  // configuration gave wrong results on gfx950). Key groups name every stage, so
+  // that the placeholders of stages past kDStages count too, 16 bytes each:
+  // 131104 bytes at D = 128 with 128-key tiles. (Without them, the stages 32
+  // bytes lower, the RoPE attention of 2 x 65 queries over 4065 keys runs 3%
+  // slower, 52.8 against 51.2 us.)
   constexpr bool kDirect = MPX_FA_DIRECT && (D == 128 || D == 64) && (BN == 64 || BN == 128) &&
                            (NW == 8 || NW == 4);
   // Paged with 64-key tiles: three stages, which leaves room for the
@@ -1702,7 +1706,9 @@ void fa_fwd16_kernel(FwdParams p) {
                                   : (131072 / (4 * BN * D) < 4 ? 131072 / (4 * BN * D) : 4));
   constexpr int kLdsBytes =
       kDirect ? kDStages * 2 * BN * 2 * D : kFa16Stages * fa16_stage_elems<D, BN>() * 2;
-  static_assert(kLdsBytes + (kSlice ? kMaxItemPages * 4 : 0) <= 131072, "LDS budget");
+  constexpr int kPlaceholders = kDirect && KG > 1 ? 16 * (4 - kDStages) : 0;
+  static_assert(kLdsBytes + kPlaceholders + (kSlice ? kMaxItemPages * 4 : 0) <= 131072 + 32,
+                "LDS budget");
   // Direct staging uses three separate stage arrays (so alias analysis can
   // tell a stage being read from the stage a DMA is writing); smem is used by
   // the register-staged path.
@@ -1735,7 +1741,8 @@ void fa_fwd16_drop_kernel(FwdParams p) {
   constexpr int kDStages = MPX_FA_DSTAGES > 0 ? MPX_FA_DSTAGES
                                               : (131072 / (4 * BN * D) < 4 ? 131072 / (4 * BN * D) : 4);
   static_assert(MPX_FA_DIRECT && (D == 128 || D == 64) && (BN == 64 || BN == 128) &&
-                    (NW == 8 || NW == 4) && kDStages * 2 * BN * 2 * D <= 131072,
+                    (NW == 8 || NW == 4) &&
+                    kDStages * 2 * BN * 2 * D + (KG > 1 ? 16 * (4 - kDStages) : 0) <= 131072 + 32,
                 "dropout runs on the direct kernels");
   constexpr int kStageB = 2 * BN * 2 * D;
   __shared__ __align__(16) unsigned char dst0[kStageB];
