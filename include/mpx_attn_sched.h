@@ -84,6 +84,19 @@ int mpx_attn_fwd_rope_qk(const void* q, const void* k, const void* v, void* o,
                          int n_pos, int cache_dtype, void* workspace, size_t workspace_bytes,
                          void* stream);
 
+/*
+ * How a forward call of this size runs, for tests and tuning: *key_groups is
+ * the number of key groups that a workgroup's waves are cut into (1, 2 or 4),
+ * *splits the most ranges that a query tile's keys are split into (1: none),
+ * *balanced 1 where two workgroups per CU take long and short query tiles
+ * together. block_size > 0: paged prefill over tables of Sk tokens (no window)
+ * with pages of that size, `alibi` != 0 with ALiBi slopes. D as the kernels
+ * take it. MPX_EINVAL for empty sizes. No counterpart in the reference.
+ */
+int mpx_attn_fwd_form(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
+                      int window_right, int dtype, int block_size, int alibi, int* key_groups,
+                      int* splits, int* balanced);
+
 #ifdef __cplusplus
 }
 #endif

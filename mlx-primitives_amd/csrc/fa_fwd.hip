@@ -796,3 +796,24 @@ extern "C" int mpx_paged_prefill(const void* q, const void* k_pool, const void* 
                                block_size, max_blocks, scale, causal, dtype, workspace,
                                workspace_bytes, stream);
 }
+
+extern "C" int mpx_attn_fwd_form(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
+                                 int window_right, int dtype, int block_size, int alibi,
+                                 int* key_groups, int* splits, int* balanced) {
+  clear_error();
+  MPX_CHECK_ARG(B > 0 && H > 0 && Sq > 0 && Sk > 0 && D > 0 && key_groups && splits && balanced,
+                "mpx_attn_fwd_form: empty problem or null result");
+  Plan pl;
+  if (block_size > 0) {
+    const int bl = log2_if_pow2(block_size);
+    pl = make_plan(B, H, Sq, Sk, D, causal, -1, -1, dtype,
+                   paged_tile_cap(block_size, tile_n(D, dtype, true, bl, alibi != 0)), true, bl,
+                   alibi != 0);
+  } else {
+    pl = make_plan(B, H, Sq, Sk, D, causal, window_left, window_right, dtype);
+  }
+  *key_groups = pl.kg;
+  *splits = pl.splits;
+  *balanced = pl.snake;
+  return MPX_OK;
+}

@@ -101,6 +101,8 @@ def load() -> ctypes.CDLL:
                                                          ctypes.c_void_p]
         lib.mpx_attn_fwd_rope_qk_preferred.restype = ctypes.c_int
         lib.mpx_attn_fwd_rope_qk_preferred.argtypes = [ctypes.c_int] * 10
+        lib.mpx_attn_fwd_form.restype = ctypes.c_int
+        lib.mpx_attn_fwd_form.argtypes = [ctypes.c_int] * 11 + [ctypes.POINTER(ctypes.c_int)] * 3
         lib.mpx_attn_bwd.restype = ctypes.c_int
         lib.mpx_attn_bwd.argtypes = [ctypes.c_void_p] * 9 + [_i64p] * 8 + [
             ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
@@ -400,6 +402,17 @@ def rope_qk_preferred(B: int, H: int, Sq: int, Sk: int, D: int, causal: bool, wi
     return bool(load().mpx_attn_fwd_rope_qk_preferred(
         B, H, Sq, Sk, D, int(causal), window_left, window_right, dtype_code(dtype),
         dtype_code(cache_dtype)))
+
+
+def fwd_form(B: int, H: int, Sq: int, Sk: int, D: int, causal: bool, window_left: int,
+             window_right: int, dtype: torch.dtype, block_size: int = 0, alibi: bool = False
+             ) -> tuple:
+    """(key groups, key splits, balanced) of a forward call (mpx_attn_fwd_form)."""
+    out = [ctypes.c_int() for _ in range(3)]
+    _check(load().mpx_attn_fwd_form(B, H, Sq, Sk, D, int(causal), window_left, window_right,
+                                    dtype_code(dtype), block_size, int(alibi),
+                                    *(ctypes.byref(x) for x in out)), "mpx_attn_fwd_form failed")
+    return out[0].value, out[1].value, bool(out[2].value)
 
 
 _DS_LIMIT: dict = {}

@@ -40,7 +40,10 @@ def test_header_declares_expected_entry_points():
 
 
 def test_library_exports_every_declared_symbol(lib):
-    for name in declared_functions():
+    sched = open(HEADER.replace("mpx_attn.h", "mpx_attn_sched.h")).read()
+    sched = re.findall(r"\b(mpx_\w+)\(", re.sub(r"/\*.*?\*/", "", sched, flags=re.S))
+    assert len(sched) == 7
+    for name in declared_functions() + sched:
         assert hasattr(lib, name), name
         assert ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
 

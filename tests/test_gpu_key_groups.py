@@ -62,6 +62,93 @@ def test_dense(device, size, dtype, D, causal):
     np.testing.assert_allclose(out.double().cpu().numpy(), want, rtol=0, atol=2e-2)
 
 
+# A size for each form that _native.fwd_form names: key groups, whether the keys
+# are split, and float32's order of two workgroups per CU.
+FORMS = [  # dtype, D, (B, H, H_kv, Sq, Sk), causal, window, (groups, split, balanced)
+    *((dt, D, *c) for dt in (torch.bfloat16, torch.float16) for D in (64, 128) for c in (
+        ((1, 2, 2, 1, 1), True, None, (4, False, False)),
+        ((1, 2, 1, 1, 2048), True, None, (4, True, False)),
+        ((1, 96, 48, 129, 129), True, None, (2, False, False)),
+        ((1, 96, 96, 129, 129), False, None, (2, False, False)),
+        ((1, 5, 1, 65, 16384), True, None, (2, True, False)),
+        ((1, 5, 5, 65, 16384), False, None, (2, True, False)),
+        ((1, 96, 96, 129, 129), True, 30, (2, False, False)),
+        ((1, 12, 12, 1000, 1000), False, 500, (2, True, False)),
+        ((1, 1, 1, 1000, 1000), False, 500, (4, True, False)),
+        ((1, 96, 96, 257, 257), True, None, (1, False, False)))),
+    *((torch.bfloat16, 128, *c) for c in (
+        ((1, 32, 8, 777, 777), True, None, (2, False, False)),
+        ((1, 24, 24, 1300, 1300), True, None, (2, False, False)),
+        ((1, 5, 5, 129, 16384), True, None, (1, True, False)))),
+    *((torch.float32, D, *c) for D in (32, 64) for c in (
+        ((1, 8, 8, 33, 97), True, None, (2, False, False)),
+        ((1, 2, 1, 1, 2048), False, None, (2, True, False)),
+        ((1, 12, 12, *((129, 2048) if D == 32 else (65, 4096))), True, None, (1, True, False)),
+        ((1, 64, 32, 257, 257), True, None, (2, False, True)),   # 40 q-tiles on each XCD
+        ((1, 64, 64, 257, 257), False, None, (1, False, False)))),
+    (torch.float32, 32, (1, 16, 16, 1300, 1300), True, None, (2, False, True)),
+]
+
+
+def form_of(dtype, D, size, causal, W):
+    B, H, _, Sq, Sk = size
+    if W is not None:
+        mask = (causal, W, -1 if causal else W)
+    else:
+        mask = (False, -1, Sk - Sq) if causal and Sk > Sq else (causal, -1, -1)
+    groups, splits, balanced = _native.fwd_form(B, H, Sq, Sk, D, *mask, dtype)
+    return groups, splits > 1, balanced
+
+
+@pytest.mark.parametrize("dtype,D,size,causal,W,form", FORMS)
+def test_each_form(device, dtype, D, size, causal, W, form):
+    assert form_of(dtype, D, size, causal, W) == form
+    B, H, H_kv, Sq, Sk = size
+    q = rnd((B, Sq, H, D), 1, dtype)
+    k, v = rnd((B, Sk, H_kv, D), 2, dtype), rnd((B, Sk, H_kv, D), 3, dtype)
+    qd, kd, vd = (x.to(device) for x in (q, k, v))
+    if W is None:
+        out = flash_attention(qd, kd, vd, causal=causal, enable_gqa=H != H_kv)
+        want = dense(q, k, v, None, max(0, Sk - Sq) if causal else None)
+    else:
+        out = sliding_window_attention(qd, kd, vd, W, causal=causal)
+        want = dense(q, k, v, W, 0 if causal else W)
+    rtol, atol = (1e-4, 1e-5) if dtype == torch.float32 else (0, 2e-2)
+    np.testing.assert_allclose(out.double().cpu().numpy(), want, rtol=rtol, atol=atol)
+
+
+@pytest.mark.parametrize("dtype,D,size", [
+    (torch.bfloat16, 64, (1, 4, 4, 3, 300)), (torch.float16, 128, (1, 4, 4, 3, 300)),
+    (torch.bfloat16, 128, (1, 4, 4, 3, 2048)), (torch.bfloat16, 128, (1, 96, 96, 129, 129)),
+    (torch.float32, 64, (1, 4, 4, 3, 300)), (torch.float32, 32, (1, 2, 2, 1, 2048))])
+@pytest.mark.parametrize("causal", [True, False])
+def test_infinities_and_nan_across_groups(device, dtype, D, size, causal):
+    # Keys of some groups of a tile score -inf or NaN, or +inf (a NaN row, inf -
+    # inf), as the query's first dimension is negative or positive: the same rows
+    # are NaN as in float64, the others agree.
+    B, H, _, Sq, Sk = size
+    assert form_of(dtype, D, size, causal, None)[0] > 1
+    for inf, nan in ((range(32, 64), ()), (range(0, 128), ()), ((5, 70, 127), ()),
+                     ((), (100,)), (range(16, 32), (3,))):
+        q, k, v = (rnd((B, n, H, D), i, dtype) for i, n in enumerate((Sq, Sk, Sk)))
+        q[:, ::2, :, 0] = -q[:, ::2, :, 0].abs() - 1   # even rows: -inf
+        k[:, list(inf), :, 0] = math.inf
+        k[:, list(nan), 0] = math.nan                  # in the first head
+        out = flash_attention(*(x.to(device) for x in (q, k, v)), causal=causal)
+        with np.errstate(invalid="ignore"):
+            want = dense(q, k, v, None, Sk - Sq if causal else None)
+        got = out.double().cpu().numpy()
+        # (a row whose every visible key scores -inf: NaN in the closed form, a
+        # row without keys, 0, in the kernels)
+        blind = np.isnan(want) & (got == 0)
+        if blind.any():
+            assert Sq == Sk and causal and len(inf) >= 32 and not blind[:, 128:].any()
+        assert (np.isnan(got) == np.isnan(want) & ~blind).all()
+        rtol, atol = (1e-4, 1e-5) if dtype == torch.float32 else (0, 2e-2)
+        seen = ~np.isnan(want)
+        np.testing.assert_allclose(got[seen], want[seen], rtol=rtol, atol=atol)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("S,W,causal", [(700, 0, True), (700, 30, True), (1000, 63, False),
                                         (513, 200, True), (300, 299, False)])
@@ -128,6 +215,25 @@ def test_paged_prefill_missing_pages(device, D, bs, alibi):
     np.testing.assert_allclose(got[:2], want[:2], rtol=0, atol=2e-2)
 
 
+@pytest.mark.parametrize("D,H,S,bs,form", [
+    (128, 2, 1, 16, (1, False)), (128, 1, 257, 16, (4, False)), (128, 1, 1000, 16, (4, True)),
+    (128, 12, 1000, 16, (2, True)), (128, 1, 129, 24, (2, False)), (128, 1, 512, 24, (2, True)),
+    (64, 1, 129, 16, (2, False)), (64, 1, 512, 16, (2, True)), (64, 48, 512, 16, (1, True))])
+def test_each_paged_form(device, D, H, S, bs, form):
+    pages = -(-S // bs)
+    got = _native.fwd_form(1, H, max(S, 2), pages * bs, D, True, -1, -1, torch.bfloat16, bs)
+    assert (got[0], got[1] > 1) == form
+    Sq = max(S, 2)   # (one query is a decode)
+    tables = torch.randperm(pages, generator=torch.Generator().manual_seed(1)).to(torch.int32)[None]
+    q = rnd((1, Sq, H, D), 1, torch.bfloat16)
+    kp, vp = (rnd((pages, bs, H, D), s, torch.bfloat16) for s in (2, 3))
+    cl = torch.tensor([S], dtype=torch.int32)
+    out = paged_attention(*(x.to(device) for x in (q, kp, vp, tables, cl)), block_size=bs)
+    want = op.paged_attention_prefill(*(x.double().numpy() for x in (q, kp, vp)), tables.numpy(),
+                                      cl.numpy(), 1 / math.sqrt(D), bs, True, None)
+    np.testing.assert_allclose(out.double().cpu().numpy(), want, rtol=0, atol=2e-2)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_rope_on_load_equals_rope_first(device, D):
     # Q rotated by every key group: bit-identical to rotating it first.
@@ -142,11 +248,12 @@ def test_rope_on_load_equals_rope_first(device, D):
 @pytest.mark.parametrize("cache", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,Sq,Sk,q_off,kv_off,causal", [
     (1, 4, 1, 700, 699, 0, True), (2, 32, 65, 4065, 4000, 0, True), (1, 8, 100, 129, 40, 40, False),
-    (1, 3, 33, 128, 97, 2, True), (1, 4, 1, 1, 7, 7, True), (1, 16, 200, 200, 0, 0, True)])
+    (1, 3, 33, 128, 97, 2, True), (1, 4, 1, 1, 7, 7, True), (1, 16, 200, 200, 0, 0, True),
+    (1, 96, 129, 129, 5, 5, True)])
 def test_k_rotated_in_the_kernel_equals_rope_first(device, B, H, Sq, Sk, q_off, kv_off, causal,
                                                    cache):
     # The same bits as rotating Q and K first: tiles past the last key, offsets
-    # on either side, splits of the keys, 2 and 4 key groups.
+    # on either side, splits of the keys, 2 key groups (32 and 96 heads) and 4.
     D, dtype = 128, torch.bfloat16
     q = rnd((B, Sq, H, D), 1, dtype).to(device)
     k, v = (rnd((B, Sk, H, D), s, dtype).to(device) for s in (2, 3))
@@ -155,6 +262,7 @@ def test_k_rotated_in_the_kernel_equals_rope_first(device, B, H, Sq, Sk, q_off, 
     wr = q_off - kv_off if causal else -1
     mask = (False, -1, wr) if wr else (True, -1, -1)
     assert _native.rope_qk_preferred(B, H, Sq, Sk, D, *mask, dtype, cache)
+    assert _native.fwd_form(B, H, Sq, Sk, D, *mask, dtype)[0] == (2 if H in (32, 96) else 4)
     out = fused_rope_attention(q, k, v, cos_cache=cos, sin_cache=sin, q_offset=q_off,
                                kv_offset=kv_off, causal=causal)
     o = torch.empty_like(q)
@@ -188,11 +296,10 @@ def test_k_rotation_left_to_its_own_pass():
     assert not pref(2, 32, 65, 4065, 128, False, -1, 4000, f, b)
 
 
-@pytest.mark.parametrize("S,H", [(300, 8), (1000, 16), (777, 12)])
+@pytest.mark.parametrize("S,H", [(300, 8), (1000, 16), (777, 12), (129, 96)])
 def test_lse_of_key_groups(device, S, H):
-    # The saved log-sum-exp (base 2) and the keep mask do not depend on the
-    # groups: lse against float64, dropout's forward against the oracle's mask is
-    # covered by the dropout tests at these sizes.
+    # The saved log-sum-exp (base 2) does not depend on the groups: lse against
+    # float64.
     D = 128
     q, k, v = (rnd((1, S, H, D), i, torch.float16).to(device) for i in range(3))
     o, lse = torch.empty_like(q), torch.empty(1, H, S, device=device)
@@ -210,7 +317,7 @@ def test_lse_of_key_groups(device, S, H):
 @pytest.mark.parametrize("B,H,H_kv,Sq,Sk,causal,W", [
     (1, 8, 8, 1, 300, False, None), (1, 8, 8, 33, 97, True, None), (1, 8, 2, 300, 300, True, None),
     (1, 8, 8, 700, 700, True, 100), (2, 16, 16, 300, 300, True, None),  # 10 tiles per XCD
-    (1, 16, 16, 1300, 1300, True, None),   # 42 q-tiles on each XCD: second half reversed
+    (1, 16, 16, 1300, 1300, True, None),   # 42 q-tiles on each XCD (D = 32: second half reversed)
     (2, 12, 12, 1024, 1024, True, None),   # 48, the training case
     (1, 3, 1, 500, 500, False, None)])
 def test_float32_key_groups(device, B, H, H_kv, Sq, Sk, causal, W, D):
