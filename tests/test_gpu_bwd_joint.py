@@ -16,7 +16,9 @@ import torch
 
 from mlx_primitives import _native
 from mlx_primitives.attention import _launch, flash_attention, sliding_window_attention
+from mlx_primitives.constants import Layout
 from oracle import attention_grad as oag
+from oracle import dropout as od
 
 NREL = {torch.float16: 2e-3, torch.bfloat16: 1.5e-2, torch.float32: 2e-5}
 
@@ -138,6 +140,35 @@ CASES32 = [  # float32: tiles of 64 rows, two key groups of 32
 @pytest.mark.parametrize("case", CASES32)
 def test_joint_backward_float32(device, case):
     test_joint_backward(device, torch.float32, case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,D,stored", [
+    (torch.bfloat16, 64, None), (torch.float16, 128, False), (torch.bfloat16, 128, None),
+    (torch.float32, 64, None), (torch.float32, 128, None)])
+@pytest.mark.parametrize("long,p,causal,wl,H_kv", [
+    ("keys", 0.0, False, 300, 4), ("keys", 0.3, True, -1, 4), ("keys", 0.3, False, 300, 2),
+    ("queries", 0.0, True, -1, 4), ("queries", 0.3, False, -1, 2), ("queries", 0.3, False, 300, 4)])
+def test_launches_of_their_own(device, monkeypatch, dtype, D, stored, p, causal, wl, H_kv, long):
+    # A side of 129 tiles is no joint launch at any size: the dQ and dK/dV
+    # launches (paired at D = 128, an odd count), with the masks and the keep
+    # mask; without groups and with them (parts on the side of the keys). At D =
+    # 128 the dropout backward stores dS by default; False recomputes.
+    monkeypatch.setattr(_launch, "BWD_STORED_DS", stored)
+    n = 16400 if dtype != torch.float32 else 8200
+    Sq, Sk = (70, n) if long == "keys" else (n, 200)
+    H, seed = 4, 0xABCDEF0123456789
+    q, d = rnd((1, Sq, H, D), 1, dtype), rnd((1, Sq, H, D), 2, dtype)
+    k, v = rnd((1, Sk, H_kv, D), 3, dtype), rnd((1, Sk, H_kv, D), 4, dtype)
+    a = [x.to(device).requires_grad_(True) for x in (q, k, v)]
+    out = _launch.run_attention(*a, Layout.BSHD, 1 / math.sqrt(D), causal, wl, -1, dropout_p=p,
+                                dropout_seed_value=seed)
+    got = torch.autograd.grad(out, a, d.to(device))
+    want = od.attention_dropout_grad(*(x.double().numpy() for x in (q, k, v, d)), 1 / math.sqrt(D),
+                                     causal, p, seed, wl, keep=None if p else np.ones((1, 1, 1, 1)))
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        err = np.linalg.norm(g.double().cpu().numpy() - w)
+        assert err <= NREL[dtype] * np.linalg.norm(w), (name, err)
 
 
 @pytest.mark.gpu

@@ -29,6 +29,7 @@ import numpy as np
 import pytest
 import torch
 
+from mlx_primitives import _native
 from mlx_primitives.attention import (chunked_cross_attention, flash_attention,
                                       sliding_window_attention)
 from mlx_primitives.attention import _launch
@@ -245,14 +246,33 @@ def test_grad_vs_oracle(device, dtype, D, causal, wl, H_kv):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("causal,wl,H_kv", [(True, -1, 4), (True, 50, 2)])
 def test_grad_vs_oracle_recompute_schedule(device, monkeypatch, dtype, causal, wl, H_kv):
-    # The dropout backward at D = 128 takes the stored-dS schedule by default;
-    # this runs the other one.
+    # The schedule that recomputes dS at D = 128 (also the default at this size).
     monkeypatch.setattr(_launch, "BWD_STORED_DS", False)
     grad_vs_oracle(device, dtype, 128, causal, wl, H_kv)
 
 
-def grad_vs_oracle(device, dtype, D, causal, wl, H_kv):
-    B, Sq, Sk, H, p, seed = 2, 300, 300, 4, 0.2, SEED ^ (D * 31 + H_kv)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal,wl,H_kv", [(True, -1, 4), (False, -1, 4), (True, 50, 4),
+                                            (True, -1, 2)])
+def test_grad_vs_oracle_stored_schedule(device, monkeypatch, dtype, causal, wl, H_kv):
+    # The schedule that stores dS, which larger launches take by default.
+    monkeypatch.setattr(_launch, "BWD_STORED_DS", True)
+    grad_vs_oracle(device, dtype, 128, causal, wl, H_kv)
+
+
+@pytest.mark.parametrize("dtype,B,S,H,D,groups", [
+    (torch.bfloat16, 4, 1000, 12, 64, 2), (torch.float16, 1, 300, 8, 64, 4),
+    (torch.bfloat16, 1, 1000, 16, 128, 4), (torch.float16, 1, 777, 12, 128, 4),
+    (torch.bfloat16, 1, 129, 96, 128, 2), (torch.float32, 2, 300, 16, 64, 2)])
+def test_grad_vs_oracle_key_groups(device, dtype, B, S, H, D, groups):
+    # The keep mask of forwards that run in key groups.
+    assert _native.fwd_form(B, H, S, S, D, True, -1, -1, dtype)[0] == groups
+    grad_vs_oracle(device, dtype, D, True, -1, H, B, S, H)
+
+
+def grad_vs_oracle(device, dtype, D, causal, wl, H_kv, B=2, S=300, H=4):
+    Sq = Sk = S
+    p, seed = 0.2, SEED ^ (D * 31 + H_kv)
     scale = 1 / math.sqrt(D)
     q = rnd((B, Sq, H, D), 10, dtype)
     k = rnd((B, Sk, H_kv, D), 11, dtype)

@@ -275,7 +275,7 @@ def test_stub_fused_rope_matches_api(device):
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
 def test_stub_dropout_matches_api(device, D):
-    # (D = 128: both sides take the stored-dS backward)
+    # (both sides recompute dS at this size)
     from mlx_primitives.attention._launch import run_attention
     from mlx_primitives.constants import Layout
 
