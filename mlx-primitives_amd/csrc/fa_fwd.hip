@@ -138,37 +138,55 @@ Plan plan_for(int kg, int B, int H, int Sq, int Sk, int D, int causal, int windo
   return pl;
 }
 
-// Estimated time of a 16-bit launch at D = 64 or 128, in us: steps of the CU
-// that runs the most of them times a step's time, plus the fixed part of its
-// items (Q, filling the DMA pipeline, the epilogue) and the split merge.
-// A step of 128 keys takes 3.5 / 2.3 / 1.8 us with 1 / 2 / 4 key groups at
-// D = 128 and 2.3 / 1.25 / 0.8 at D = 64 (a workgroup's row count halves each
-// time, but its tile still has to come in), an item 6 us (7.2 with
-// groups to merge), splitting and merging about 14.
-double plan_time(const Plan& pl, long bh, int Sq, int Sk, int D) {
-  static const double kStep[2][3] = {{2.3, 1.25, 0.8}, {3.5, 2.3, 1.8}};
-  const double step = kStep[D == 128][pl.kg == 4 ? 2 : pl.kg - 1] * pl.BN / 128;
-  const double item = pl.kg == 1 ? 6.0 : 7.2;
-  const double cus = kNumCUs;
+// Estimated time of a 16-bit launch at D = 64 or 128, in us: 3 for the launch,
+// then the chain of steps and items (Q, filling the DMA pipeline, the epilogue)
+// of the CU that runs the most, and the merge of split keys (its partial sums
+// written and read back at about 1.8 TB/s). The costs of a step (one KV tile of
+// a workgroup) and an item are fitted to 1500 calls of up to 8 x 128 heads and
+// 6000 keys, each timed in every form (a tenth off in the mean). A workgroup's
+// row count halves with each cut, but its tile still has to come in and the
+// groups' sums to be merged: four groups gain from the third tile on.
+struct TileCost {
+  double step, item;
+};
+
+TileCost tile_cost(int kg, int D, int BN, bool paged) {
+  static const TileCost kCost[5][3] = {
+      {{2.0, 2.2}, {1.3, 2.1}, {0.9, 2.6}},      // D = 64
+      {{3.1, 2.75}, {1.95, 3.5}, {1.35, 5.2}},   // D = 128
+      {{1.55, 3.2}, {1.25, 3.35}, {1.25, 3.35}}, // 64-key tiles (paged), D = 64
+      {{3.0, 2.65}, {2.0, 3.85}, {2.0, 3.85}},   // 64-key tiles (paged), D = 128
+      {{3.3, 3.7}, {2.05, 4.45}, {1.5, 5.7}}};   // paged 128-key tiles, D = 128
+  const int form = BN == 64 ? (D == 64 ? 2 : 3) : paged ? 4 : (D == 64 ? 0 : 1);
+  return kCost[form][kg == 4 ? 2 : kg - 1];
+}
+
+double plan_time(const Plan& pl, long bh, int Sq, int Sk, int D, bool paged) {
+  const TileCost c = tile_cost(pl.kg, D, pl.BN, paged);
+  const double cus = kNumCUs, launch = 3.0;
   if (pl.splits > 1) {
     const double wgs = (double)bh * (pl.var_split > 0 ? pl.var_split : pl.n_qtiles * pl.splits);
-    return std::ceil(wgs / cus) * (pl.tiles_per_split * step + item) + 14.0;
+    return launch + std::ceil(wgs / cus) * (pl.tiles_per_split * c.step + c.item) +
+           (pl.BN == 64 ? 4.0 : 2.0) + 0.55e-6 * pl.ws_bytes;
   }
+  // A workgroup's share: a q-tile, or the pair of them (the middle one alone).
   double longest = 0, total = 0;
-  for (int t = 0; t < pl.n_qtiles; ++t) {
-    const int n = qtile_kv_tiles(t, pl.BM, pl.BN, Sq, Sk, pl.win_left, pl.win_right);
-    total += n;
-    longest = std::max<double>(longest, n);
+  for (int t = 0; t < pl.n_slots; ++t) {
+    double cost = 0;
+    for (int qt : {pl.n_qtiles - 1 - t, t}) {
+      cost += qtile_kv_tiles(qt, pl.BM, pl.BN, Sq, Sk, pl.win_left, pl.win_right) * c.step + c.item;
+      if (!pl.paired || qt == t) break;
+    }
+    total += cost;
+    longest = std::max(longest, cost);
   }
   const double wgs = (double)bh * pl.n_slots, mean = total / pl.n_slots;
-  if (pl.paired) longest = mean;  // (equal pairs)
-  const double items = (pl.paired ? 2.0 : 1.0) * item;
-  if (wgs <= cus) return longest * step + items;
-  // (tail_bh: the launch ends with single q-tiles, about two steps uneven)
-  const double steps =
-      pl.tail_bh > 0 ? 1.05 * mean * wgs / cus + 2
-      : longest <= 1.1 * mean ? std::ceil(wgs / cus) * longest : mean * wgs / cus + longest / 2;
-  return steps * step + items * wgs / cus;
+  if (wgs <= cus) return launch + longest;
+  // (tail_bh: the launch ends with single q-tiles, about two steps uneven;
+  // otherwise whole rounds of equal shares, or half a long one on top of the mean)
+  if (pl.tail_bh > 0) return launch + 1.05 * mean * wgs / cus + 2 * c.step;
+  if (longest <= 1.1 * mean) return launch + std::ceil(wgs / cus) * longest;
+  return launch + mean * wgs / cus + longest / 2;
 }
 
 // The same for the float32 kernel at D <= 64 (64-key tiles, two workgroups per
@@ -192,7 +210,8 @@ double plan_time32(const Plan& pl, long bh, int Sq, int Sk, int D) {
   // (more than one workgroup per CU in the order of the heads: long ones meet)
   if (pl.splits == 1 && !pl.snake && wgs > kNumCUs) longest *= 2;
   const double share = total * bh / kNumCUs * busy;
-  if (pl.splits > 1) return std::max(longest * chain, 1.05 * share) + 20.0;
+  if (pl.splits > 1)  // (and the merge, by its partial sums' bytes)
+    return std::max(longest * chain, 1.05 * share) + 10.0 + 0.35e-6 * pl.ws_bytes;
   // (snake: every CU has at most the longest item and a shortest one)
   if (pl.snake) return (longest + 1) * 2.65 * D / 64 + 8.0;
   return std::max(longest * chain, share) + 8.0 * std::ceil(wgs / (2 * kNumCUs));
@@ -239,13 +258,13 @@ Plan make_plan(int B, int H, int Sq, int Sk, int D, int causal, int window_left,
   if (dtype == MPX_F32 || (D != 64 && D != 128) || !MPX_FA_DIRECT ||
       bh * best.n_qtiles > 2 * kNumCUs)
     return best;
-  double t = plan_time(best, bh, Sq, Sk, D);
+  // (6%: past the estimate's error near the line, where a cut gains little; a
+  // call of one tile stays as it is)
+  double t = 0.94 * plan_time(best, bh, Sq, Sk, D, paged);
   for (int kg = 2; kg <= (best.BN == 128 ? 4 : 2); kg *= 2) {
     const Plan pl = plan(kg);
-    // (paged items pay more for four groups: one 128-key step alone, (2, 74, 32,
-    // 128), takes 10.4 us with one group and 11.3 with four)
-    const double tk = plan_time(pl, bh, Sq, Sk, D) + (paged && kg == 4 ? 0.8 : 0.0);
-    if (tk < 0.97 * t) {
+    const double tk = plan_time(pl, bh, Sq, Sk, D, paged);
+    if (tk < t) {
       best = pl;
       t = tk;
     }

@@ -66,7 +66,8 @@ def test_dense(device, size, dtype, D, causal):
 # are split, and float32's order of two workgroups per CU.
 FORMS = [  # dtype, D, (B, H, H_kv, Sq, Sk), causal, window, (groups, split, balanced)
     *((dt, D, *c) for dt in (torch.bfloat16, torch.float16) for D in (64, 128) for c in (
-        ((1, 2, 2, 1, 1), True, None, (4, False, False)),
+        ((1, 2, 2, 1, 1), True, None, (2 if D == 64 else 1, False, False)),
+        ((1, 4, 4, 3, 300), True, None, (4, False, False)),
         ((1, 2, 1, 1, 2048), True, None, (4, True, False)),
         ((1, 96, 48, 129, 129), True, None, (2, False, False)),
         ((1, 96, 96, 129, 129), False, None, (2, False, False)),
@@ -79,14 +80,13 @@ FORMS = [  # dtype, D, (B, H, H_kv, Sq, Sk), causal, window, (groups, split, bal
     *((torch.bfloat16, 128, *c) for c in (
         ((1, 32, 8, 777, 777), True, None, (2, False, False)),
         ((1, 24, 24, 1300, 1300), True, None, (2, False, False)),
-        ((1, 5, 5, 129, 16384), True, None, (1, True, False)))),
+        ((1, 24, 24, 129, 4065), True, None, (1, True, False)))),
     *((torch.float32, D, *c) for D in (32, 64) for c in (
         ((1, 8, 8, 33, 97), True, None, (2, False, False)),
         ((1, 2, 1, 1, 2048), False, None, (2, True, False)),
-        ((1, 12, 12, *((129, 2048) if D == 32 else (65, 4096))), True, None, (1, True, False)),
+        ((1, 12, 12, 65, 4096), True, None, (1, True, False)),
         ((1, 64, 32, 257, 257), True, None, (2, False, True)),   # 40 q-tiles on each XCD
         ((1, 64, 64, 257, 257), False, None, (1, False, False)))),
-    (torch.float32, 32, (1, 16, 16, 1300, 1300), True, None, (2, False, True)),
 ]
 
 
@@ -246,14 +246,15 @@ def test_rope_on_load_equals_rope_first(device, D):
 
 
 @pytest.mark.parametrize("cache", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("B,H,Sq,Sk,q_off,kv_off,causal", [
-    (1, 4, 1, 700, 699, 0, True), (2, 32, 65, 4065, 4000, 0, True), (1, 8, 100, 129, 40, 40, False),
-    (1, 3, 33, 128, 97, 2, True), (1, 4, 1, 1, 7, 7, True), (1, 16, 200, 200, 0, 0, True),
-    (1, 96, 129, 129, 5, 5, True)])
+@pytest.mark.parametrize("B,H,Sq,Sk,q_off,kv_off,causal,groups", [
+    (1, 4, 1, 700, 699, 0, True, 4), (2, 32, 65, 4065, 4000, 0, True, 2),
+    (1, 8, 100, 129, 40, 40, False, 2), (1, 3, 33, 400, 369, 2, True, 4),
+    (1, 4, 1, 257, 263, 7, True, 4), (1, 16, 200, 200, 0, 0, True, 2),
+    (1, 96, 129, 129, 5, 5, True, 2)])
 def test_k_rotated_in_the_kernel_equals_rope_first(device, B, H, Sq, Sk, q_off, kv_off, causal,
-                                                   cache):
+                                                   groups, cache):
     # The same bits as rotating Q and K first: tiles past the last key, offsets
-    # on either side, splits of the keys, 2 key groups (32 and 96 heads) and 4.
+    # on either side, splits of the keys, 2 and 4 key groups.
     D, dtype = 128, torch.bfloat16
     q = rnd((B, Sq, H, D), 1, dtype).to(device)
     k, v = (rnd((B, Sk, H, D), s, dtype).to(device) for s in (2, 3))
@@ -262,7 +263,7 @@ def test_k_rotated_in_the_kernel_equals_rope_first(device, B, H, Sq, Sk, q_off, 
     wr = q_off - kv_off if causal else -1
     mask = (False, -1, wr) if wr else (True, -1, -1)
     assert _native.rope_qk_preferred(B, H, Sq, Sk, D, *mask, dtype, cache)
-    assert _native.fwd_form(B, H, Sq, Sk, D, *mask, dtype)[0] == (2 if H in (32, 96) else 4)
+    assert _native.fwd_form(B, H, Sq, Sk, D, *mask, dtype)[0] == groups
     out = fused_rope_attention(q, k, v, cos_cache=cos, sin_cache=sin, q_offset=q_off,
                                kv_offset=kv_off, causal=causal)
     o = torch.empty_like(q)
@@ -317,7 +318,7 @@ def test_lse_of_key_groups(device, S, H):
 @pytest.mark.parametrize("B,H,H_kv,Sq,Sk,causal,W", [
     (1, 8, 8, 1, 300, False, None), (1, 8, 8, 33, 97, True, None), (1, 8, 2, 300, 300, True, None),
     (1, 8, 8, 700, 700, True, 100), (2, 16, 16, 300, 300, True, None),  # 10 tiles per XCD
-    (1, 16, 16, 1300, 1300, True, None),   # 42 q-tiles on each XCD (D = 32: second half reversed)
+    (1, 16, 16, 1300, 1300, True, None),
     (2, 12, 12, 1024, 1024, True, None),   # 48, the training case
     (1, 3, 1, 500, 500, False, None)])
 def test_float32_key_groups(device, B, H, H_kv, Sq, Sk, causal, W, D):
