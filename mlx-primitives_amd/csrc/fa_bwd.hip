@@ -1311,17 +1311,21 @@ bool bwd_joint(int B, int H, int Sq, int Sk, int D, int win_left) {
 }
 
 // Parts that a K/V head's query heads are cut into (1: none) for the grouped
-// backward at D <= 128: the fewest equal ones (a divisor of the group) that give
-// the dK/dV side a workgroup for each of the chip's slots (512; 256 in float32,
-// at one wave per SIMD). Causal bf16 (1, 2048, 32 heads over 8, 128): 409 -> 158
-// us with 4 parts in the joint launch; (8, 1024, 32 over 4, 128): 488 -> 325 us
-// with 4 parts of paired tiles. Where the next divisor is far (groups like 7:
-// from 1 to 7) its sums can be large; above kMaxPartBytes the group is cut into
-// as many parts as that holds, some a head longer, which is still a workgroup
-// per slot: `need` parts are below 1024 workgroups, 256 MiB of pairs at D = 128.
-// Causal bf16 forward and backward, the divisor's sums against these: (4, 4000,
-// 28 over 4, 128) 439 MiB 2.12 ms, 250 MiB 2.07; (15, 4096, 71 over 1, 64) 2.1
-// GiB 13.0 ms, 240 MiB 12.2.
+// backward at D <= 128, by estimated time: the longest chain of steps of one
+// workgroup or the chip's share of all of them, whichever takes longer, and for
+// parts their sums, written and read back at 2.5 TB/s, with a launch of 4 us. So
+// short queries, whose chains are short, and launches that are full anyway stay
+// whole. In 64 x 128 blocks of products (dQ 3 each, dK/dV 4): 0.55 us at D = 64,
+// 0.93 at D = 128, 4 and 8 in float32; the masks are not known here and taken as
+// three fifths of the pairs. bf16 forward and backward with 1 / 2 / 4 (or all)
+// parts, as (batch, queries, keys, heads over K/V heads, D): (1, 4688, 4688, 24
+// over 8, 128) causal 907 / 687 / 641 us, (4, 18, 847, 216 over 27, 128) 203 / 247
+// / 350, (2, 32, 783, 100 over 20, 64) 35 / 48 / 58, (4, 781, 781, 84 over 21,
+// 128) causal 404 / 472 / 514.
+// Parts are a divisor of the group, so that they are equal, or as many as
+// kMaxPartBytes of sums hold (groups like 7 have none between 1 and 7), some a
+// head longer: causal (4, 4000, 4000, 28 over 4, 128) 439 MiB in 7 parts 2.12
+// ms, 250 MiB in 4 parts 2.07.
 constexpr size_t kMaxPartBytes = 256u << 20;
 
 size_t part_bytes(int B, int H_kv, int Sk, int D, int parts) {
@@ -1332,16 +1336,27 @@ int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, in
   const int group = H / H_kv;
   if (group == 1 || D > 128) return 1;
   const bool f32 = dtype == MPX_F32;
-  const bool pairs = !f32 && D == 128 && !bwd_joint(B, H, Sq, Sk, D, win_left);
-  const int own = pairs ? 2 * kBwdOwn
-                        : (f32 && bwd32_joint(B, H, Sq, Sk, D) ? kBwdOwn / 2 : kBwdOwn);
-  const long wgs = (long)B * H_kv * ((Sk + own - 1) / own), slots = f32 ? 256 : 512;
-  const long need = (slots + wgs - 1) / wgs;
-  if (need >= group) return group;
-  int parts = (int)need;
-  while (group % parts != 0) ++parts;
-  if (parts == 1 || part_bytes(B, H_kv, Sk, D, parts) <= kMaxPartBytes) return parts;
-  return (int)(kMaxPartBytes / part_bytes(B, H_kv, Sk, D, 1));
+  const bool joint = f32 ? bwd32_joint(B, H, Sq, Sk, D) : bwd_joint(B, H, Sq, Sk, D, win_left);
+  const int own = f32 && joint ? kBwdOwn / 2 : kBwdOwn;
+  const double block = (f32 ? (D == 64 ? 4.0 : 8.0) : (D == 64 ? 0.55 : 0.93)) * own / kBwdOwn;
+  const double seen = 0.6, slots = f32 ? 256 : 512;
+  const double n_qt = (Sq + own - 1) / own, n_kt = (Sk + own - 1) / own;
+  const double q_blocks = (Sq + 63) / 64, k_blocks = (Sk + 63) / 64, heads = (double)B * H;
+  const double kv_share = seen * heads * n_kt * q_blocks * 4 * block / slots;
+  const double q_share = seen * heads * n_qt * k_blocks * 3 * block / slots;
+  // (paired tiles: two chains, which the mask shortens)
+  const double pair = !f32 && D == 128 && !joint && n_kt > 1 ? 2 * seen : 1.0;
+  auto time = [&](int parts) {
+    const double chain = 4 * q_blocks * ((group + parts - 1) / parts) * block * pair;
+    const double t = joint ? std::max({chain, 3 * k_blocks * block, kv_share + q_share})
+                           : std::max(chain, kv_share);
+    return parts == 1 ? t : t + 4.0 + 2 * part_bytes(B, H_kv, Sk, D, parts) / 2.5e6;
+  };
+  const long most = (long)(kMaxPartBytes / part_bytes(B, H_kv, Sk, D, 1));
+  int best = 1;
+  for (int parts = 2; parts <= std::min<long>(group, most); ++parts)
+    if ((group % parts == 0 || parts == most) && time(parts) < time(best)) best = parts;
+  return best;
 }
 
 template <int D, bool BF16>

@@ -92,9 +92,9 @@ CASES = [
     (2, 16, 16, 4096, 200, 128, False, None),    # 32 x 34 tiles: joint
     (1, 32, 4, 4096, 4096, 128, True, None),     # 2048 tiles: paired, 4 parts
     (1, 31, 31, 4100, 4100, 128, True, None),    # 2046 tiles: joint
-    (1, 20, 4, 64, 16384, 128, True, None),      # 5 heads in 4 parts: paired tiles
-    (1, 33, 3, 64, 16384, 64, False, None),      # 11 in 10, two launches at D = 64
-    (1, 4, 2, 64, 16384, 64, True, None),        # 2 parts of one head, two launches
+    (1, 20, 4, 2048, 16384, 128, True, None),    # 5 heads in 4 parts: paired tiles
+    (1, 33, 3, 1300, 16384, 64, False, None),    # 11 in 10, two launches at D = 64
+    (1, 4, 2, 1300, 16384, 64, True, None),      # 2 parts of one head, two launches
 ]
 
 
@@ -130,7 +130,7 @@ CASES32 = [  # float32: tiles of 64 rows, two key groups of 32
     (1, 1, 1, 128, 4032, 128, False, None),      # 2 + 2 x 63 tiles
     (1, 4, 1, 64, 6000, 128, False, None),       # too many for an order: parts alone
     (1, 31, 31, 2112, 2112, 64, True, None),     # 2046 tiles: joint
-    (1, 32, 8, 2048, 2048, 64, True, None),      # 2048: launches of their own, 2 parts
+    (1, 32, 8, 2048, 2048, 64, True, None),      # 2048: launches of their own, 4 parts
     (1, 74, 2, 64, 8256, 64, False, None),       # 37 heads in 31 parts, own launches
     (1, 34, 2, 64, 8256, 128, True, None),       # 17 in 15
 ]
@@ -192,8 +192,8 @@ def test_joint_dropout_agrees_with_stored_schedule(device, monkeypatch, H, H_kv,
 def test_uneven_parts_with_dropout(device, monkeypatch):
     # The keep mask of every head where one part holds a head more than the
     # others, against the stored-dS schedule, which has no parts.
-    H, H_kv, Sk = 20, 4, 16384
-    q, d = rnd((1, 64, H, 128), 1, torch.bfloat16), rnd((1, 64, H, 128), 2, torch.bfloat16)
+    H, H_kv, Sq, Sk = 20, 4, 2048, 16384
+    q, d = rnd((1, Sq, H, 128), 1, torch.bfloat16), rnd((1, Sq, H, 128), 2, torch.bfloat16)
     k, v = rnd((1, Sk, H_kv, 128), 3, torch.bfloat16), rnd((1, Sk, H_kv, 128), 4, torch.bfloat16)
     got = {}
     for stored in (True, None):
@@ -301,12 +301,19 @@ def test_grouped_workspace_is_bounded(group):
     assert most <= 256 << 20
 
 
-@pytest.mark.parametrize("H,H_kv,Sk,D,dtype,parts", [
-    (20, 4, 16384, 128, 2, 4), (33, 3, 16384, 64, 2, 10), (4, 2, 16384, 64, 2, 2),
-    (74, 2, 8256, 64, 0, 31), (34, 2, 8256, 128, 0, 15), (56, 8, 4096, 128, 2, 7)])
-def test_parts_of_a_group(H, H_kv, Sk, D, dtype, parts):
+@pytest.mark.parametrize("B,H,H_kv,Sq,Sk,D,dtype,parts", [
     # the parts that the cases above mean
+    (1, 20, 4, 2048, 16384, 128, 2, 4), (1, 33, 3, 1300, 16384, 64, 2, 10),
+    (1, 4, 2, 1300, 16384, 64, 2, 2), (1, 74, 2, 64, 8256, 64, 0, 31),
+    (1, 34, 2, 64, 8256, 128, 0, 15), (1, 8, 1, 130, 70, 128, 2, 8), (1, 12, 4, 200, 333, 64, 2, 3),
+    (1, 32, 4, 4096, 4096, 128, 2, 8), (1, 32, 8, 2048, 2048, 64, 0, 4),
+    # short queries, where parts cost more than the chains they cut
+    # (forward and backward whole and in all parts: 203 / 539 us, 35 / 63, 36 / 45)
+    (4, 216, 27, 18, 847, 128, 2, 1), (2, 100, 20, 32, 783, 64, 2, 1), (8, 54, 18, 4, 56, 128, 2, 1),
+    # full launches (152 / 203 and 404 / 514)
+    (6, 108, 27, 378, 378, 64, 2, 1), (4, 84, 21, 781, 781, 128, 2, 1)])
+def test_parts_of_a_group(B, H, H_kv, Sq, Sk, D, dtype, parts):
     lib = _native.load()
-    plain = -(-lib.mpx_attn_bwd_workspace_bytes(1, H, 64) // 256) * 256
-    assert lib.mpx_attn_bwd_grouped_workspace_bytes(1, H, H_kv, 64, Sk, D, dtype, -1) \
-        == plain + 2 * H_kv * parts * Sk * D * 4
+    plain = -(-lib.mpx_attn_bwd_workspace_bytes(B, H, Sq) // 256) * 256
+    got = lib.mpx_attn_bwd_grouped_workspace_bytes(B, H, H_kv, Sq, Sk, D, dtype, -1)
+    assert max(0, got - plain) == (2 * B * H_kv * parts * Sk * D * 4 if parts > 1 else 0)
