@@ -80,14 +80,18 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 
 def host_command(out: str) -> list[str]:
-    """The host compiler's command for the Python extension (no device code)."""
+    """The host compiler's command for the Python extension (no device code).
+    NDEBUG: without it a pybind11 header brings a thread-local counter, and a
+    module with thread-local storage that is loaded but never touches its own
+    leaves glibc (2.35) on the slow path for everyone's: torch.empty took 2.4 us
+    of host time instead of 2.0, x.shape 0.09 instead of 0.06."""
     import sysconfig
 
     import torch
     from torch.utils import cpp_extension
 
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    return ([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+    return ([shutil.which("g++") or "g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-w",
              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
              "-I" + INCLUDE, "-I" + sysconfig.get_paths()["include"]]
             + ["-isystem" + d for d in cpp_extension.include_paths()]

@@ -2,6 +2,8 @@
 calls with the extension answering None give the same bits, over the layouts
 that it takes and those that it leaves."""
 
+import struct
+
 import numpy as np
 import pytest
 import torch
@@ -69,6 +71,14 @@ def test_entries_are_the_librarys():
     with pytest.raises(KeyError):
         _native.host().init({})
     assert _native._load_host(lib) is not None  # (binds the entries again)
+
+
+def test_extension_has_no_thread_local_storage():
+    # (a segment of type PT_TLS slows every thread-local access of the process)
+    data = open(_native._HOST_PATH, "rb").read()
+    assert data[:5] == b"\x7fELF\x02"
+    off, size, count = struct.unpack_from("<Q", data, 32)[0], *struct.unpack_from("<HH", data, 54)
+    assert 7 not in [struct.unpack_from("<I", data, off + i * size)[0] for i in range(count)]
 
 
 @pytest.mark.parametrize("content", [None, b"", b"\x7fELF of another torch"])
