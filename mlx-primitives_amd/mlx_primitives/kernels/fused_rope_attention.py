@@ -55,20 +55,22 @@ def _check_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
 def _k_in_kernel(q, k, cos_cache, sin_cache, q_offset: int, kv_offset: int, mask: dict) -> bool:
     """Whether K is rotated by the attention kernel: few q-tiles per K tile
     (_native.rope_qk_preferred), tables as the kernel reads them, and nothing
-    that the general path would refuse or copy."""
-    half = q.shape[-1] // 2
-    for c in (cos_cache, sin_cache):
-        if (c.ndim != 2 or c.shape[1] != half or c.dtype != cos_cache.dtype
-                or c.dtype not in (torch.float16, torch.bfloat16) or c.device != q.device
-                or not c.is_contiguous() or c.data_ptr() % 16):
-            return False
-    if (cos_cache.shape != sin_cache.shape or cos_cache.requires_grad or sin_cache.requires_grad
-            or not q.is_cuda or q.dtype != torch.bfloat16 or q.numel() == 0 or k.numel() == 0
-            or max(q.shape[1] + q_offset, k.shape[1] + kv_offset) > cos_cache.shape[0]):
+    that the general path would refuse or copy. What rules most calls out comes
+    first: a call that launches two small kernels waits for the host."""
+    if (q.dtype != torch.bfloat16 or q.shape[3] != 128 or not q.is_cuda
+            or cos_cache.dtype not in (torch.float16, torch.bfloat16)
+            or q.numel() == 0 or k.numel() == 0
+            or not _native.rope_qk_preferred(
+                q.shape[0], q.shape[2], q.shape[1], k.shape[1], 128, mask["causal"], -1,
+                int(mask.get("window_right", -1)), q.dtype, cos_cache.dtype)):
         return False
-    return _native.rope_qk_preferred(
-        q.shape[0], q.shape[2], q.shape[1], k.shape[1], q.shape[3], mask["causal"], -1,
-        int(mask.get("window_right", -1)), q.dtype, cos_cache.dtype)
+    for c in (cos_cache, sin_cache):
+        if (c.ndim != 2 or c.shape[1] != 64 or c.dtype != cos_cache.dtype
+                or c.device != q.device or not c.is_contiguous() or c.data_ptr() % 16):
+            return False
+    return (cos_cache.shape == sin_cache.shape
+            and not cos_cache.requires_grad and not sin_cache.requires_grad
+            and max(q.shape[1] + q_offset, k.shape[1] + kv_offset) <= cos_cache.shape[0])
 
 
 def _rope_attention(q, k, v, scale, cos_cache, sin_cache, rope_base, q_offset, kv_offset,
