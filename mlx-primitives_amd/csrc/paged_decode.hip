@@ -686,6 +686,11 @@ int halved_part(int B, int H, long heads, int D, int block_size, int max_blocks,
 //            30 x 6000, 16 heads of 64:         96.9 / 90.1 / 88.2 / 111 / 170
 // Head dims up to 64 in 16 bits take 128 tokens per batch of loads (64 at head
 // dim 128): they stop there, and gain up to a larger grid.
+// The tables' width decides, not the contexts, which only the device knows: in
+// tables as wide as a model's longest context, short contexts run in the few
+// long partitions that the width fills the chip with (4 sequences of about 1400
+// tokens, 8 K/V heads: 64-token partitions with tables 2100 tokens wide, 256 at
+// 8192, 512 from 16384 on).
 constexpr long kGroupedWaves = 1024, kHeadWaves = 2048, kSmallHeadWaves = 8192;
 
 int decode_part(int B, int H, int H_kv, int D, int block_size, int max_blocks, int dtype) {
