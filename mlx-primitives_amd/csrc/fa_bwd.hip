@@ -1313,11 +1313,12 @@ bool bwd_joint(int B, int H, int Sq, int Sk, int D, int win_left) {
 // Parts that a K/V head's query heads are cut into (1: none) for the grouped
 // backward at D <= 128, by estimated time: the longest chain of steps of one
 // workgroup or the chip's share of all of them, whichever takes longer, and for
-// parts their sums, written and read back at 2.5 TB/s, with a launch of 4 us. So
+// parts their sums, written and read back at 2.5 TB/s, with a launch of 3 us. So
 // short queries, whose chains are short, and launches that are full anyway stay
-// whole. In 64 x 128 blocks of products (dQ 3 each, dK/dV 4): 0.55 us at D = 64,
-// 0.93 at D = 128, 4 and 8 in float32; the masks are not known here and taken as
-// three fifths of the pairs. bf16 forward and backward with 1 / 2 / 4 (or all)
+// whole. In 64 x 128 blocks of products (dQ 3 each, dK/dV 4): 0.65 us at D = 64,
+// 1.0 at D = 128, 4 and 8 in float32; the masks are not known here and taken as
+// three fifths of the pairs (fitted to 600 calls, each timed in 1, 2, 4 and all
+// parts: 0.7% over the best of these in the mean). bf16 forward and backward with 1 / 2 / 4 (or all)
 // parts, as (batch, queries, keys, heads over K/V heads, D): (1, 4688, 4688, 24
 // over 8, 128) causal 907 / 687 / 641 us, (4, 18, 847, 216 over 27, 128) 203 / 247
 // / 350, (2, 32, 783, 100 over 20, 64) 35 / 48 / 58, (4, 781, 781, 84 over 21,
@@ -1338,7 +1339,7 @@ int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, in
   const bool f32 = dtype == MPX_F32;
   const bool joint = f32 ? bwd32_joint(B, H, Sq, Sk, D) : bwd_joint(B, H, Sq, Sk, D, win_left);
   const int own = f32 && joint ? kBwdOwn / 2 : kBwdOwn;
-  const double block = (f32 ? (D == 64 ? 4.0 : 8.0) : (D == 64 ? 0.55 : 0.93)) * own / kBwdOwn;
+  const double block = (f32 ? (D == 64 ? 4.0 : 8.0) : (D == 64 ? 0.65 : 1.0)) * own / kBwdOwn;
   const double seen = 0.6, slots = f32 ? 256 : 512;
   const double n_qt = (Sq + own - 1) / own, n_kt = (Sk + own - 1) / own;
   const double q_blocks = (Sq + 63) / 64, k_blocks = (Sk + 63) / 64, heads = (double)B * H;
@@ -1350,7 +1351,7 @@ int bwd_kv_parts(int B, int H, int H_kv, int Sq, int Sk, int D, int win_left, in
     const double chain = 4 * q_blocks * ((group + parts - 1) / parts) * block * pair;
     const double t = joint ? std::max({chain, 3 * k_blocks * block, kv_share + q_share})
                            : std::max(chain, kv_share);
-    return parts == 1 ? t : t + 4.0 + 2 * part_bytes(B, H_kv, Sk, D, parts) / 2.5e6;
+    return parts == 1 ? t : t + 3.0 + 2 * part_bytes(B, H_kv, Sk, D, parts) / 2.5e6;
   };
   const long most = (long)(kMaxPartBytes / part_bytes(B, H_kv, Sk, D, 1));
   int best = 1;

@@ -210,8 +210,8 @@ double plan_time32(const Plan& pl, long bh, int Sq, int Sk, int D) {
   // (more than one workgroup per CU in the order of the heads: long ones meet)
   if (pl.splits == 1 && !pl.snake && wgs > kNumCUs) longest *= 2;
   const double share = total * bh / kNumCUs * busy;
-  if (pl.splits > 1)  // (and the merge, by its partial sums' bytes)
-    return std::max(longest * chain, 1.05 * share) + 10.0 + 0.35e-6 * pl.ws_bytes;
+  if (pl.splits > 1)  // (and the shorter items and the merge, by its partial sums' bytes)
+    return std::max(longest * chain, 1.05 * share) + 6.0 + 10.0 * D / 64 + 0.35e-6 * pl.ws_bytes;
   // (snake: every CU has at most the longest item and a shortest one)
   if (pl.snake) return (longest + 1) * 2.65 * D / 64 + 8.0;
   return std::max(longest * chain, share) + 8.0 * std::ceil(wgs / (2 * kNumCUs));
